@@ -79,6 +79,16 @@ __device__ __forceinline__ void st_nt(float4 *p, float4 v) {
   const v4f w = {v.x, v.y, v.z, v.w};
   __builtin_nontemporal_store(w, reinterpret_cast<v4f *>(p));
 }
+// The same for four floats at any float address (gfx950 takes a 16-byte access at 4-byte alignment).
+typedef float v4f_u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 ld_nt4(const float *p) {
+  const v4f_u v = __builtin_nontemporal_load(reinterpret_cast<const v4f_u *>(p));
+  return make_float4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ void st_nt4(float *p, float4 v) {
+  const v4f_u w = {v.x, v.y, v.z, v.w};
+  __builtin_nontemporal_store(w, reinterpret_cast<v4f_u *>(p));
+}
 __device__ __forceinline__ float ld_nt(const float *p) { return __builtin_nontemporal_load(p); }
 __device__ __forceinline__ void st_nt(float *p, float v) { __builtin_nontemporal_store(v, p); }
 

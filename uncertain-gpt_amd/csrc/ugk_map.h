@@ -9,8 +9,19 @@
 // the last-level cache (unroll 1-8, 256-1024 threads, flat or grid-stride,
 // with and without nt) put nt loads and stores with unroll 1-2 and 256-512
 // threads on top; each operator picks its own (the spread is a few percent).
-// Arrays whose pointers are not all 16-byte aligned, and the n % 4 tail, take
-// a scalar grid-stride path with identical arithmetic.
+//
+// Any address and any n take this path, in one launch. gfx950 accepts a
+// 16-byte access at a 4-byte address, so the slots start at the first element
+// whose address in the first output is a cache line's (full lines are then
+// written there whatever the streams' offsets: 478 against 482 us for a whole
+// block of layer kernels whose arrays are 8 bytes off, with the slots started at
+// element 0 instead), and the up to 31 elements before them and 3 after them
+// are taken one by one by a workgroup of their own, told from the others by a
+// scalar compare. Both were separate paths before: misaligned arrays took
+// dwords (residual forward over 11.8M elements 32 against 22.9 us, its
+// backward 42.3 against 39.0), and a ragged end took a second launch, which cost
+// 4.4-4.8 us per call (six such calls over 11,061,531 parameters: 281 against
+// 268 us).
 //
 // An operator is a struct with
 //   kLoads, kStores          stream counts;
@@ -20,6 +31,10 @@
 //                            using them (0: none), which caps the workgroups
 //                            resident on a CU (160 KiB of LDS each);
 //   Params                   per-launch scalars passed by value;
+//   kIndexed                 whether apply reads i: the slots then start at
+//                            element 0 (their indexes need no 64-bit add per
+//                            element, which the ops that draw eps are short of
+//                            the cycles for);
 //   apply(ld, st, tab, i, p) the per-element body; i is the element index;
 //   kPre, Pre, pre(i, p)     optionally (kPre true), the part of the body that
 //                            reads no stream (a Philox draw): the kernel
@@ -40,6 +55,7 @@ struct MapOp {
   static constexpr int kUnroll = 2;
   static constexpr int kThreads = kBlock;
   static constexpr unsigned kLdsReserve = 0;
+  static constexpr bool kIndexed = false;
   static constexpr bool kPre = false;
   struct Pre {};
 };
@@ -51,14 +67,39 @@ struct Streams {
   typename Op::Params p;
 };
 
+constexpr unsigned kLine = 32;  // floats of a cache line
+
+// Element i alone.
 template <class Op>
-__global__ __launch_bounds__(Op::kThreads) void k_map_vec4(Streams<Op> s, size_t n4) {
+__device__ __forceinline__ void map_one(const Streams<Op> &s, size_t i, const uint64_t *tab) {
+  float in[Op::kLoads], out[Op::kStores];
+#pragma unroll
+  for (int l = 0; l < Op::kLoads; l++) in[l] = s.ld[l][i];
+  if constexpr (Op::kPre)
+    Op::apply_pre(in, out, tab, i, s.p, Op::pre(i, s.p));
+  else
+    Op::apply(in, out, tab, i, s.p);
+#pragma unroll
+  for (int o = 0; o < Op::kStores; o++) s.st[o][i] = out[o];
+}
+
+template <class Op>
+__global__ __launch_bounds__(Op::kThreads) void k_map_vec4(Streams<Op> s, size_t n4, unsigned full, unsigned lead, unsigned rest) {
   __shared__ uint64_t tab[Op::kTable ? 32 : 1];
   if (Op::kTable) {
     ugk_exp2_stage(tab);
     __syncthreads();
   }
   constexpr int kU = Op::kUnroll, kT = Op::kThreads;
+  if (blockIdx.x == full) {  // the workgroup past the float4 slots: the elements around them
+    for (unsigned k = threadIdx.x; k < rest; k += kT) map_one<Op>(s, k < lead ? k : 4 * n4 + k, tab);
+    return;
+  }
+  if (Op::kIndexed) lead = 0;  // as the launch has it: the element index is 4 times the slot's
+#pragma unroll
+  for (int l = 0; l < Op::kLoads; l++) s.ld[l] += lead;
+#pragma unroll
+  for (int o = 0; o < Op::kStores; o++) s.st[o] += lead;
   const size_t base = (size_t)blockIdx.x * (kT * kU) + threadIdx.x;
   float4 v[kU][Op::kLoads];
 #pragma unroll
@@ -66,7 +107,7 @@ __global__ __launch_bounds__(Op::kThreads) void k_map_vec4(Streams<Op> s, size_t
     const size_t i = base + (size_t)u * kT;
     if (i < n4) {
 #pragma unroll
-      for (int l = 0; l < Op::kLoads; l++) v[u][l] = ld_nt(reinterpret_cast<const float4 *>(s.ld[l]) + i);
+      for (int l = 0; l < Op::kLoads; l++) v[u][l] = ld_nt4(s.ld[l] + 4 * i);
     }
   }
   typename Op::Pre pre[kU][4];
@@ -76,7 +117,7 @@ __global__ __launch_bounds__(Op::kThreads) void k_map_vec4(Streams<Op> s, size_t
       const size_t i = base + (size_t)u * kT;
       if (i < n4) {
 #pragma unroll
-        for (int e = 0; e < 4; e++) pre[u][e] = Op::pre(4 * i + e, s.p);
+        for (int e = 0; e < 4; e++) pre[u][e] = Op::pre(lead + 4 * i + e, s.p);
       }
     }
   }
@@ -93,57 +134,26 @@ __global__ __launch_bounds__(Op::kThreads) void k_map_vec4(Streams<Op> s, size_t
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         if constexpr (Op::kPre)
-          Op::apply_pre(in[e], out[e], tab, 4 * i + e, s.p, pre[u][e]);
+          Op::apply_pre(in[e], out[e], tab, lead + 4 * i + e, s.p, pre[u][e]);
         else
-          Op::apply(in[e], out[e], tab, 4 * i + e, s.p);
+          Op::apply(in[e], out[e], tab, lead + 4 * i + e, s.p);
       }
 #pragma unroll
       for (int o = 0; o < Op::kStores; o++)
-        st_nt(reinterpret_cast<float4 *>(s.st[o]) + i, make_float4(out[0][o], out[1][o], out[2][o], out[3][o]));
+        st_nt4(s.st[o] + 4 * i, make_float4(out[0][o], out[1][o], out[2][o], out[3][o]));
     }
-  }
-}
-
-template <class Op>
-__global__ __launch_bounds__(kBlock) void k_map_scalar(Streams<Op> s, size_t begin, size_t n) {
-  __shared__ uint64_t tab[Op::kTable ? 32 : 1];
-  if (Op::kTable) {
-    ugk_exp2_stage(tab);
-    __syncthreads();
-  }
-  for (size_t i = begin + (size_t)blockIdx.x * kBlock + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * kBlock) {
-    float in[Op::kLoads], out[Op::kStores];
-#pragma unroll
-    for (int l = 0; l < Op::kLoads; l++) in[l] = s.ld[l][i];
-    if constexpr (Op::kPre)
-      Op::apply_pre(in, out, tab, i, s.p, Op::pre(i, s.p));
-    else
-      Op::apply(in, out, tab, i, s.p);
-#pragma unroll
-    for (int o = 0; o < Op::kStores; o++) s.st[o][i] = out[o];
   }
 }
 
 template <class Op>
 int run_map(const Streams<Op> &s, size_t n, const char *name) {
   if (n == 0) return 0;
-  bool vec = true;
-  for (int l = 0; l < Op::kLoads; l++) vec = vec && aligned16(s.ld[l]);
-  for (int o = 0; o < Op::kStores; o++) vec = vec && aligned16(s.st[o]);
-  size_t done = 0;
-  if (vec && n >= 4) {
-    const size_t n4 = n / 4;
-    launch(k_map_vec4<Op>, dim3(grid_for(n4, (size_t)Op::kThreads * Op::kUnroll)),
-                       dim3(Op::kThreads), Op::kLdsReserve, s, n4);
-    done = n4 * 4;
-  }
-  if (done < n) {
-    const size_t rest = n - done;
-    unsigned g = grid_for(rest, kBlock);
-    if (g > 65536u) g = 65536u;
-    launch(k_map_scalar<Op>, dim3(g), dim3(kBlock), 0, s, done, n);
-  }
+  size_t lead = Op::kIndexed ? 0 : (0 - ((uintptr_t)s.st[0] >> 2)) & (kLine - 1);
+  if (lead > n) lead = n;
+  const size_t n4 = (n - lead) / 4;
+  const unsigned full = grid_for(n4, (size_t)Op::kThreads * Op::kUnroll);
+  launch(k_map_vec4<Op>, dim3(full + (n != 4 * n4 ? 1 : 0)), dim3(Op::kThreads), Op::kLdsReserve, s, n4, full,
+         (unsigned)lead, (unsigned)(n - 4 * n4));
   return check_launch(name);
 }
 
