@@ -941,11 +941,12 @@ int layers_backward(const char *fn, bool zeroed, float *grads, float *grads_acts
     // in gpt2_backward nothing reads it after the residual_backward that
     // splits it into dx and dy (res1 of every block and each block's resa).
     if (int e = timed(dx ? UGK_OP_LAYERNORM_RESIDUAL_BACKWARD_MAIN : UGK_OP_LAYERNORM_BACKWARD_MAIN, [&] {
-          return launch_layernorm_backward_partials(dinp, part, dx, dy, dout, inp, w, mean, rstd, M, C, slot_rows,
-                                                    &nblk, dx ? dinp_mode : kDinpRw, zeroed && dx != nullptr);
+          return launch_layernorm_backward_partials(dinp, part, nullptr, nullptr, dx, dy, dout, inp, w, mean, rstd,
+                                                    M, C, slot_rows, &nblk, dx ? dinp_mode : kDinpRw,
+                                                    zeroed && dx != nullptr);
         }))
       return e;
-    jobs.push_back({part, dw, db, nblk});
+    jobs.push_back({part, dw, db, nblk, dout, inp, mean, rstd});
     return 0;
   };
   const size_t last = cfg.L > 0 ? A(cfg.L - 1, a.res1) : a.enc;
@@ -997,7 +998,7 @@ int layers_backward(const char *fn, bool zeroed, float *grads, float *grads_acts
   }
   if (!jobs.empty())
     UGK_TRY(timed(UGK_OP_LAYERNORM_COLUMN_SUMS,
-                  [&] { return launch_layernorm_reduce(jobs.data(), (int)jobs.size(), C); }));
+                  [&] { return launch_layernorm_reduce(jobs.data(), (int)jobs.size(), M, C); }));
   UGK_TRY(timed(UGK_OP_ENCODER_BACKWARD, [&] {
     return ugk_encoder_backward(grads + p.wte, grads + p.wpe, grads_acts + a.enc, inputs, B, T, C);
   }));

@@ -89,6 +89,14 @@ __device__ __forceinline__ void st_nt4(float *p, float4 v) {
   const v4f_u w = {v.x, v.y, v.z, v.w};
   __builtin_nontemporal_store(w, reinterpret_cast<v4f_u *>(p));
 }
+__device__ __forceinline__ float4 ld4(const float *p) {
+  const v4f_u v = *reinterpret_cast<const v4f_u *>(p);
+  return make_float4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ void st4(float *p, float4 v) {
+  const v4f_u w = {v.x, v.y, v.z, v.w};
+  *reinterpret_cast<v4f_u *>(p) = w;
+}
 __device__ __forceinline__ float ld_nt(const float *p) { return __builtin_nontemporal_load(p); }
 __device__ __forceinline__ void st_nt(float *p, float v) { __builtin_nontemporal_store(v, p); }
 
@@ -221,10 +229,14 @@ int launch_layernorm_residual_backward(float *dinp, float *dweight, float *dbias
 // non-null, applies residual_backward(dx, dy, dinp)) and *nblk partial rows
 // of the dweight/dbias column sums to `partial`; launch_layernorm_reduce then
 // adds each job's column totals into its dweight/dbias, many jobs per launch.
+// (Few rows have no partial rows: *nblk = 0, and the main pass adds the column
+// totals itself if dweight and dbias are given, else launch_layernorm_reduce
+// takes them from the job's dout, inp, mean and rstd.)
 struct LnReduceJob {
   const float *partial;
   float *dweight, *dbias;
   int nblk;
+  const float *dout, *inp, *mean, *rstd;
 };
 // What a fused LayerNorm -> residual backward does with its dinp (the
 // float4 path; the scalar path always reads and writes it):
@@ -237,11 +249,11 @@ enum LnDinp {
 // scalar path up to 512). With dx non-null, dinp_mode says what happens to
 // dinp, and assign_res takes dx and dy as +0.0 instead of reading them (float4
 // path; the scalar path reads and writes everything).
-int launch_layernorm_backward_partials(float *dinp, float *partial, float *dx, float *dy, const float *dout,
-                                       const float *inp, const float *weight, const float *mean,
+int launch_layernorm_backward_partials(float *dinp, float *partial, float *dweight, float *dbias, float *dx, float *dy,
+                                       const float *dout, const float *inp, const float *weight, const float *mean,
                                        const float *rstd, int rows, int C, int max_blocks, int *nblk,
                                        int dinp_mode = kDinpRw, bool assign_res = false);
-int launch_layernorm_reduce(const LnReduceJob *jobs, int njobs, int C);
+int launch_layernorm_reduce(const LnReduceJob *jobs, int njobs, int rows, int C);
 // The per-op LayerNorm backward (launch_layernorm_residual_backward_into) on
 // the float4 path finishes its column sums in its main launch (1) or in a
 // second launch (0, the default); both give the same bits. The step driver always

@@ -19,9 +19,11 @@
 // a second, small kernel adds the partial rows in index order into
 // dweight/dbias. No atomics, so the result is identical run to run.
 //
-// Every load of the float4 paths is unconditional: a lane's columns past the
-// row are clamped onto the row's last float4, and rows past a wavefront's
-// range repeat its last row; the values so loaded are masked out of the sums
+// The float4 paths take rows at any alignment (gfx950 accepts a 16-byte access
+// at a 4-byte address) and widths that are no multiple of 4, whose last slot
+// overlaps the one before it (Cols). Every load of theirs is unconditional: a
+// lane's columns past the row are clamped onto the row's last four floats, and
+// rows past a wavefront's range repeat its last row; the values so loaded are masked out of the sums
 // (added as -0.0f, the identity of IEEE addition) or skipped by a branch that
 // is uniform across the wavefront, and never stored. Per-lane
 // conditions around loads made the compiler wait for one row's loads before
@@ -38,67 +40,110 @@ namespace {
 
 constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr int kMaxV = 8;  // float4 per lane held in registers: C <= 2048
+constexpr int kMaxWide = 8192;  // channels of the workgroup-per-row kernels
 
 __device__ __forceinline__ float4 add4(float4 a, float4 b) {
   return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
 }
 
-// Clamped float4 column of each of a lane's V slots, and whether it is in the row.
-template <int V>
+// A lane's V slots of four columns in a row: the slot's first float and the
+// components that are the slot's own, [lo, 4). Slots past the row repeat its
+// last four floats (lo = 4). With C no multiple of 4 (kRag) the last slot
+// does so too, for the components that the slot before it does not hold; they
+// are loaded twice and summed and stored once. C >= 4.
+template <int V, bool kRag>
 struct Cols {
-  int col[V];
-  bool in[V];
-  __device__ __forceinline__ Cols(int lane, int C4) {
+  int at[V], lo[V];
+  // slot v of the lane is slot first + v * step of the row
+  __device__ __forceinline__ Cols(int first, int step, int C) {
 #pragma unroll
     for (int v = 0; v < V; v++) {
-      const int c4 = lane + v * kWave;
-      in[v] = c4 < C4;
-      col[v] = in[v] ? c4 : C4 - 1;
+      const int c = 4 * (first + v * step);
+      at[v] = min(c, C - 4);
+      lo[v] = kRag ? min(c - at[v], 4) : c < C ? 0 : 4;
+    }
+  }
+  // component j of slot v is the slot's own
+  __device__ __forceinline__ bool own(int v, int j) const { return kRag ? j >= lo[v] : lo[v] == 0; }
+  __device__ __forceinline__ bool any(int v) const { return lo[v] < 4; }
+  // x where own, else the identity of IEEE addition
+  __device__ __forceinline__ float sel(int v, int j, float x) const { return own(v, j) ? x : -0.0f; }
+  // non-temporal store of the slot's own components to row + at[v]
+  __device__ __forceinline__ void put(float *row, int v, float4 x) const {
+    float *p = row + at[v];
+    if (lo[v] == 0) {
+      st_nt4(p, x);
+    } else if (kRag) {
+      if (lo[v] <= 1) st_nt(p + 1, x.y);
+      if (lo[v] <= 2) st_nt(p + 2, x.z);
+      if (lo[v] <= 3) st_nt(p + 3, x.w);
     }
   }
 };
 
-// Normalise one row held in registers (V float4 per lane) and store out, mean
-// and rstd: two-pass mean and variance with wavefront sums, IEEE 1/sqrtf.
-// Shared by every forward kernel, so that they give the same bits.
-template <int V>
-__device__ __forceinline__ void ln_row_out(const float4 (&xv)[V], const Cols<V> &cl, int C, int row, int lane,
-                                           const float4 *__restrict__ w4, const float4 *__restrict__ b4,
-                                           float4 *__restrict__ o4, float *__restrict__ mean,
-                                           float *__restrict__ rstd) {
-  const size_t off = (size_t)row * (C >> 2);
+// Row statistics to outputs: v = (x - m) r w + b.
+__device__ __forceinline__ float4 ln_norm4(float4 x, float m, float r, float4 w, float4 b) {
+  return make_float4((x.x - m) * r * w.x + b.x, (x.y - m) * r * w.y + b.y, (x.z - m) * r * w.z + b.z,
+                     (x.w - m) * r * w.w + b.w);
+}
+
+// A lane's share of a row's sum, and of the sum of its squared distances from m.
+template <int V, bool kRag>
+__device__ __forceinline__ float ln_lane_sum(const float4 (&xv)[V], const Cols<V, kRag> &cl) {
   float s = 0.0f;
 #pragma unroll
   for (int v = 0; v < V; v++) {
-    const bool c = cl.in[v];
-    s += c ? xv[v].x : -0.0f; s += c ? xv[v].y : -0.0f; s += c ? xv[v].z : -0.0f; s += c ? xv[v].w : -0.0f;
+    s += cl.sel(v, 0, xv[v].x); s += cl.sel(v, 1, xv[v].y); s += cl.sel(v, 2, xv[v].z); s += cl.sel(v, 3, xv[v].w);
   }
-  s = wave_sum(s);
-  const float m = s / (float)C;
+  return s;
+}
+template <int V, bool kRag>
+__device__ __forceinline__ float ln_lane_sq(const float4 (&xv)[V], const Cols<V, kRag> &cl, float m) {
   float vs = 0.0f;
 #pragma unroll
   for (int v = 0; v < V; v++) {
-    const bool c = cl.in[v];
     float d;
-    d = xv[v].x - m; vs += c ? d * d : -0.0f;
-    d = xv[v].y - m; vs += c ? d * d : -0.0f;
-    d = xv[v].z - m; vs += c ? d * d : -0.0f;
-    d = xv[v].w - m; vs += c ? d * d : -0.0f;
+    d = xv[v].x - m; vs += cl.sel(v, 0, d * d);
+    d = xv[v].y - m; vs += cl.sel(v, 1, d * d);
+    d = xv[v].z - m; vs += cl.sel(v, 2, d * d);
+    d = xv[v].w - m; vs += cl.sel(v, 3, d * d);
   }
-  vs = wave_sum(vs);
-  const float r = 1.0f / sqrtf(vs / (float)C + 1e-5f);
+  return vs;
+}
+
+// Normalise one row held in registers (V float4 per lane) and store out, mean
+// and rstd: two-pass mean and variance with wavefront sums, IEEE 1/sqrtf.
+// Shared by every one-wavefront forward kernel, so that they give the same bits.
+// kEarly: weight and bias are loaded before the sums rather than where they are
+// used, one round trip to the cache off the row's chain. It pays while the
+// rows leave the SIMDs idle for that long (residual and forward at 1,024 x 768
+// 4.3 against 4.6 us, 512 x 1,600 5.1 against 5.8), not for its registers beyond
+// (8,192 x 768 18.6 against 18.2).
+template <int V, bool kRag, bool kEarly>
+__device__ __forceinline__ void ln_row_out(const float4 (&xv)[V], const Cols<V, kRag> &cl, int C, int row, int lane,
+                                           const float *__restrict__ weight, const float *__restrict__ bias,
+                                           float *__restrict__ out, float *__restrict__ mean,
+                                           float *__restrict__ rstd) {
+  float4 w[kEarly ? V : 1], b[kEarly ? V : 1];
+  if constexpr (kEarly) {
 #pragma unroll
-  for (int v = 0; v < V; v++) {
-    if (cl.in[v]) {
-      const float4 w = w4[cl.col[v]], b = b4[cl.col[v]];
-      float4 o;
-      o.x = (xv[v].x - m) * r * w.x + b.x;
-      o.y = (xv[v].y - m) * r * w.y + b.y;
-      o.z = (xv[v].z - m) * r * w.z + b.z;
-      o.w = (xv[v].w - m) * r * w.w + b.w;
-      st_nt(o4 + off + cl.col[v], o);
+    for (int v = 0; v < V; v++) {
+      w[v] = ld4(weight + cl.at[v]);
+      b[v] = ld4(bias + cl.at[v]);
     }
+    __builtin_amdgcn_sched_barrier(0);
   }
+  const float m = wave_sum(ln_lane_sum(xv, cl)) / (float)C;
+  const float r = 1.0f / sqrtf(wave_sum(ln_lane_sq(xv, cl, m)) / (float)C + 1e-5f);
+  float *o = out + (size_t)row * C;
+#pragma unroll
+  for (int v = 0; v < V; v++)
+    if (cl.any(v)) {
+      if constexpr (kEarly)
+        cl.put(o, v, ln_norm4(xv[v], m, r, w[v], b[v]));
+      else
+        cl.put(o, v, ln_norm4(xv[v], m, r, ld4(weight + cl.at[v]), ld4(bias + cl.at[v])));
+    }
   if (lane == 0) {
     mean[row] = m;
     rstd[row] = r;
@@ -111,7 +156,7 @@ __device__ __forceinline__ void ln_row_out(const float4 (&xv)[V], const Cols<V> 
 // kRes: the row is first formed as res = inp + inp2 (residual_forward,
 // train_bnn.c:182-186), stored to res, and normalised from the registers, the
 // pair gpt2_kernels.cuh:793-797 launches back to back.
-template <int V, bool kRes, int RPW>
+template <int V, bool kRes, int RPW, bool kRag, bool kEarly>
 __global__ __launch_bounds__(kBlock) void k_ln_fwd_vec(float *__restrict__ out, float *__restrict__ mean,
                                                        float *__restrict__ rstd, const float *__restrict__ inp,
                                                        const float *__restrict__ weight,
@@ -120,21 +165,14 @@ __global__ __launch_bounds__(kBlock) void k_ln_fwd_vec(float *__restrict__ out, 
   const int lane = threadIdx.x & (kWave - 1);
   const int row0 = (blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6)) * RPW;
   if (row0 >= rows) return;
-  const int C4 = C >> 2;
-  const Cols<V> cl(lane, C4);
-  const float4 *x4 = reinterpret_cast<const float4 *>(inp);
-  const float4 *y4 = reinterpret_cast<const float4 *>(inp2);
-  float4 *r4 = reinterpret_cast<float4 *>(res);
-  float4 *o4 = reinterpret_cast<float4 *>(out);
-  const float4 *w4 = reinterpret_cast<const float4 *>(weight);
-  const float4 *b4 = reinterpret_cast<const float4 *>(bias);
+  const Cols<V, kRag> cl(lane, kWave, C);
   float4 xa[V], ya[kRes ? V : 1];
   {
-    const size_t off = (size_t)row0 * C4;
+    const size_t off = (size_t)row0 * C;
 #pragma unroll
     for (int v = 0; v < V; v++) {
-      xa[v] = ld_nt(x4 + off + cl.col[v]);
-      if (kRes) ya[kRes ? v : 0] = ld_nt(y4 + off + cl.col[v]);
+      xa[v] = ld_nt4(inp + off + cl.at[v]);
+      if (kRes) ya[kRes ? v : 0] = ld_nt4(inp2 + off + cl.at[v]);
     }
   }
 #pragma unroll
@@ -143,24 +181,23 @@ __global__ __launch_bounds__(kBlock) void k_ln_fwd_vec(float *__restrict__ out, 
     if (row >= rows) break;
     float4 xb[V], yb[kRes ? V : 1];
     if (k + 1 < RPW) {
-      const size_t off = (size_t)min(row + 1, rows - 1) * C4;
+      const size_t off = (size_t)min(row + 1, rows - 1) * C;
 #pragma unroll
       for (int v = 0; v < V; v++) {
-        xb[v] = ld_nt(x4 + off + cl.col[v]);
-        if (kRes) yb[kRes ? v : 0] = ld_nt(y4 + off + cl.col[v]);
+        xb[v] = ld_nt4(inp + off + cl.at[v]);
+        if (kRes) yb[kRes ? v : 0] = ld_nt4(inp2 + off + cl.at[v]);
       }
     }
-    const size_t off = (size_t)row * C4;
     float4 xv[V];
 #pragma unroll
     for (int v = 0; v < V; v++) {
       xv[v] = xa[v];
       if (kRes) {
         xv[v] = add4(xv[v], ya[kRes ? v : 0]);
-        if (cl.in[v]) st_nt(r4 + off + cl.col[v], xv[v]);
+        cl.put(res + (size_t)row * C, v, xv[v]);
       }
     }
-    ln_row_out<V>(xv, cl, C, row, lane, w4, b4, o4, mean, rstd);
+    ln_row_out<V, kRag, kEarly>(xv, cl, C, row, lane, weight, bias, out, mean, rstd);
     if (k + 1 < RPW) {
 #pragma unroll
       for (int v = 0; v < V; v++) {
@@ -178,7 +215,7 @@ __global__ __launch_bounds__(kBlock) void k_ln_fwd_vec(float *__restrict__ out, 
 // gpt2_kernels.cuh:775 -> :784 (or :813 when L = 0) launches back to back.
 // The rows of wte and wpe are read through the cache: tokens repeat, and the
 // B rows of a position share its wpe row.
-template <int V, int RPW>
+template <int V, int RPW, bool kEarly>
 __global__ __launch_bounds__(kBlock) void k_enc_ln_fwd_vec(float *__restrict__ enc, float *__restrict__ out,
                                                            float *__restrict__ mean, float *__restrict__ rstd,
                                                            const int *__restrict__ inp,
@@ -189,21 +226,14 @@ __global__ __launch_bounds__(kBlock) void k_enc_ln_fwd_vec(float *__restrict__ e
   const int lane = threadIdx.x & (kWave - 1);
   const int row0 = (blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6)) * RPW;
   if (row0 >= rows) return;
-  const int C4 = C >> 2;
-  const Cols<V> cl(lane, C4);
-  const float4 *te4 = reinterpret_cast<const float4 *>(wte);
-  const float4 *pe4 = reinterpret_cast<const float4 *>(wpe);
-  float4 *e4 = reinterpret_cast<float4 *>(enc);
-  float4 *o4 = reinterpret_cast<float4 *>(out);
-  const float4 *w4 = reinterpret_cast<const float4 *>(weight);
-  const float4 *b4 = reinterpret_cast<const float4 *>(bias);
+  const Cols<V, false> cl(lane, kWave, C);
   float4 xa[V], ya[V];
   {
-    const size_t ot = (size_t)inp[row0] * C4, op = (size_t)(row0 % T) * C4;
+    const float *te = wte + (size_t)inp[row0] * C, *pe = wpe + (size_t)(row0 % T) * C;
 #pragma unroll
     for (int v = 0; v < V; v++) {
-      xa[v] = te4[ot + cl.col[v]];
-      ya[v] = pe4[op + cl.col[v]];
+      xa[v] = ld4(te + cl.at[v]);
+      ya[v] = ld4(pe + cl.at[v]);
     }
   }
 #pragma unroll
@@ -213,21 +243,20 @@ __global__ __launch_bounds__(kBlock) void k_enc_ln_fwd_vec(float *__restrict__ e
     float4 xb[V], yb[V];
     if (k + 1 < RPW) {
       const int nx = min(row + 1, rows - 1);
-      const size_t ot = (size_t)inp[nx] * C4, op = (size_t)(nx % T) * C4;
+      const float *te = wte + (size_t)inp[nx] * C, *pe = wpe + (size_t)(nx % T) * C;
 #pragma unroll
       for (int v = 0; v < V; v++) {
-        xb[v] = te4[ot + cl.col[v]];
-        yb[v] = pe4[op + cl.col[v]];
+        xb[v] = ld4(te + cl.at[v]);
+        yb[v] = ld4(pe + cl.at[v]);
       }
     }
-    const size_t off = (size_t)row * C4;
     float4 xv[V];
 #pragma unroll
     for (int v = 0; v < V; v++) {
       xv[v] = add4(xa[v], ya[v]);
-      if (cl.in[v]) st_nt(e4 + off + cl.col[v], xv[v]);
+      cl.put(enc + (size_t)row * C, v, xv[v]);
     }
-    ln_row_out<V>(xv, cl, C, row, lane, w4, b4, o4, mean, rstd);
+    ln_row_out<V, false, kEarly>(xv, cl, C, row, lane, weight, bias, out, mean, rstd);
     if (k + 1 < RPW) {
 #pragma unroll
       for (int v = 0; v < V; v++) {
@@ -238,7 +267,59 @@ __global__ __launch_bounds__(kBlock) void k_enc_ln_fwd_vec(float *__restrict__ e
   }
 }
 
-// Any C and alignment: one wavefront per row, three passes over the row.
+// Forward for rows of more than 2,048 channels: a workgroup of W wavefronts
+// per row, V float4 per lane in registers, so the row is still read once
+// (the one-wavefront kernel would need more than 32 registers for it, and the
+// lane loop below reads it three times). Each of the row's two sums is a lane
+// sum, a wavefront sum and the W wavefronts' sums added in order by every
+// thread, one barrier each. Memory-bound: 4,092 x 4,096 in 26.4 us (5.1 TB/s),
+// 83 us in the lane loop.
+template <int V, int W, bool kRes>
+__global__ __launch_bounds__(W * kWave) void k_ln_fwd_wide(float *__restrict__ out, float *__restrict__ mean,
+                                                           float *__restrict__ rstd, const float *__restrict__ inp,
+                                                           const float *__restrict__ weight,
+                                                           const float *__restrict__ bias, int C,
+                                                           float *__restrict__ res, const float *__restrict__ inp2) {
+  __shared__ float part[2][W];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & (kWave - 1);
+  const int row = blockIdx.x;
+  const size_t off = (size_t)row * C;
+  const Cols<V, true> cl(threadIdx.x, W * kWave, C);
+  float4 xv[V], yv[kRes ? V : 1];
+#pragma unroll
+  for (int v = 0; v < V; v++) {
+    xv[v] = ld_nt4(inp + off + cl.at[v]);
+    if (kRes) yv[kRes ? v : 0] = ld_nt4(inp2 + off + cl.at[v]);
+  }
+  if (kRes) {
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+      xv[v] = add4(xv[v], yv[kRes ? v : 0]);
+      cl.put(res + off, v, xv[v]);
+    }
+  }
+  const auto row_sum = [&](float mine, float *p) {
+    mine = wave_sum(mine);
+    if (lane == 0) p[wave] = mine;
+    __syncthreads();
+    float t = p[0];
+#pragma unroll
+    for (int k = 1; k < W; k++) t += p[k];
+    return t;
+  };
+  const float m = row_sum(ln_lane_sum(xv, cl), part[0]) / (float)C;
+  const float r = 1.0f / sqrtf(row_sum(ln_lane_sq(xv, cl, m), part[1]) / (float)C + 1e-5f);
+#pragma unroll
+  for (int v = 0; v < V; v++)
+    if (cl.any(v)) cl.put(out + off, v, ln_norm4(xv[v], m, r, ld4(weight + cl.at[v]), ld4(bias + cl.at[v])));
+  if (threadIdx.x == 0) {
+    mean[row] = m;
+    rstd[row] = r;
+  }
+}
+
+// Any C (the rows that no kernel above takes: C < 4 or beyond 8,192): one
+// wavefront per row, three passes over the row.
 __global__ __launch_bounds__(kBlock) void k_ln_fwd_scalar(float *out, float *mean, float *rstd,
                                                           const float *inp, const float *weight,
                                                           const float *bias, int rows, int C) {
@@ -400,24 +481,18 @@ __device__ __forceinline__ void ln_bwd_tail(float *partial, int nblk, int C, flo
 // an ordinary dinp store made it faster alone (35.7 against 37.2 us cold at
 // 8,192 x 768) but the step slower (3.02 against 2.93 ms), the dirty lines
 // of its 24 launches being written back during the kernels that follow.
-template <int V, int W, int R, bool kRes, int MINW, bool kNt, int kDinp, bool kAssign, bool kTail>
+template <int V, int W, int R, bool kRes, int MINW, bool kNt, int kDinp, bool kAssign, bool kTail, bool kRag>
 __global__ __launch_bounds__(W * kWave, MINW) void k_ln_bwd_vec(
     float *__restrict__ dinp, float *__restrict__ partial, const float *__restrict__ dout,
     const float *__restrict__ inp, const float *__restrict__ weight, const float *__restrict__ mean,
     const float *__restrict__ rstd, int rows, int C, int rpw, float *__restrict__ rdx,
     float *__restrict__ rdy, int same, float *dweight, float *dbias) {
+  static_assert(!kRag || (kNt && !kTail), "ragged rows take the non-temporal stores and the second launch");
   __shared__ float4 red[W][2][V * kWave];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x >> 6;
-  const int C4 = C >> 2;
   const float Cf = (float)C;
-  const Cols<V> cl(lane, C4);
-  const float4 *x4 = reinterpret_cast<const float4 *>(inp);
-  const float4 *dy4 = reinterpret_cast<const float4 *>(dout);
-  float4 *dx4 = reinterpret_cast<float4 *>(dinp);
-  float4 *a4 = reinterpret_cast<float4 *>(rdx);
-  float4 *b4 = reinterpret_cast<float4 *>(rdy);
-  const float4 *w4 = reinterpret_cast<const float4 *>(weight);
+  const Cols<V, kRag> cl(lane, kWave, C);
   float4 ag[V], ab[V];
 #pragma unroll
   for (int v = 0; v < V; v++) ag[v] = ab[v] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -430,7 +505,7 @@ __global__ __launch_bounds__(W * kWave, MINW) void k_ln_bwd_vec(
 #pragma unroll
     for (int q = 0; q < R; q++) {
       rq[q] = row + min(q, nr - 1);
-      off[q] = (size_t)rq[q] * C4;
+      off[q] = (size_t)rq[q] * C;
     }
     float4 x[R][V], dy[R][V], dx[R][V], wv[V];
     float4 ra[kRes ? R : 1][kRes ? V : 1], rb[kRes ? R : 1][kRes ? V : 1];
@@ -438,13 +513,13 @@ __global__ __launch_bounds__(W * kWave, MINW) void k_ln_bwd_vec(
 #pragma unroll
     for (int q = 0; q < R; q++)
 #pragma unroll
-      for (int v = 0; v < V; v++) x[q][v] = ld_nt(x4 + off[q] + cl.col[v]);
+      for (int v = 0; v < V; v++) x[q][v] = ld_nt4(inp + off[q] + cl.at[v]);
 #pragma unroll
     for (int q = 0; q < R; q++)
 #pragma unroll
-      for (int v = 0; v < V; v++) dy[q][v] = ld_nt(dy4 + off[q] + cl.col[v]);
+      for (int v = 0; v < V; v++) dy[q][v] = ld_nt4(dout + off[q] + cl.at[v]);
 #pragma unroll
-    for (int v = 0; v < V; v++) wv[v] = w4[cl.col[v]];
+    for (int v = 0; v < V; v++) wv[v] = ld4(weight + cl.at[v]);
 #pragma unroll
     for (int q = 0; q < R; q++) {
       m[q] = mean[rq[q]];
@@ -453,15 +528,15 @@ __global__ __launch_bounds__(W * kWave, MINW) void k_ln_bwd_vec(
 #pragma unroll
     for (int q = 0; q < R; q++)
 #pragma unroll
-      for (int v = 0; v < V; v++) dx[q][v] = kDinp == kDinpNone ? zero4() : ld_nt(dx4 + off[q] + cl.col[v]);
+      for (int v = 0; v < V; v++) dx[q][v] = kDinp == kDinpNone ? zero4() : ld_nt4(dinp + off[q] + cl.at[v]);
     if (kRes) {
       // rdy is loaded even when it is rdx (same): a valid address, never used
 #pragma unroll
       for (int q = 0; q < R; q++)
 #pragma unroll
         for (int v = 0; v < V; v++) {
-          ra[kRes ? q : 0][kRes ? v : 0] = kAssign ? zero4() : ld_nt(a4 + off[q] + cl.col[v]);
-          rb[kRes ? q : 0][kRes ? v : 0] = kAssign ? zero4() : ld_nt(b4 + off[q] + cl.col[v]);
+          ra[kRes ? q : 0][kRes ? v : 0] = kAssign ? zero4() : ld_nt4(rdx + off[q] + cl.at[v]);
+          rb[kRes ? q : 0][kRes ? v : 0] = kAssign ? zero4() : ld_nt4(rdy + off[q] + cl.at[v]);
         }
     }
     // keep every load above the arithmetic (the scheduler would otherwise
@@ -480,11 +555,10 @@ __global__ __launch_bounds__(W * kWave, MINW) void k_ln_bwd_vec(
         xh.y = (x[q][v].y - m[q]) * r[q]; dn.y = dy[q][v].y * w.y;
         xh.z = (x[q][v].z - m[q]) * r[q]; dn.z = dy[q][v].z * w.z;
         xh.w = (x[q][v].w - m[q]) * r[q]; dn.w = dy[q][v].w * w.w;
-        const bool c = cl.in[v];
-        s1[q] += c ? dn.x : -0.0f; s2[q] += c ? dn.x * xh.x : -0.0f;
-        s1[q] += c ? dn.y : -0.0f; s2[q] += c ? dn.y * xh.y : -0.0f;
-        s1[q] += c ? dn.z : -0.0f; s2[q] += c ? dn.z * xh.z : -0.0f;
-        s1[q] += c ? dn.w : -0.0f; s2[q] += c ? dn.w * xh.w : -0.0f;
+        s1[q] += cl.sel(v, 0, dn.x); s2[q] += cl.sel(v, 0, dn.x * xh.x);
+        s1[q] += cl.sel(v, 1, dn.y); s2[q] += cl.sel(v, 1, dn.y * xh.y);
+        s1[q] += cl.sel(v, 2, dn.z); s2[q] += cl.sel(v, 2, dn.z * xh.z);
+        s1[q] += cl.sel(v, 3, dn.w); s2[q] += cl.sel(v, 3, dn.w * xh.w);
       }
     }
 #pragma unroll
@@ -509,30 +583,28 @@ __global__ __launch_bounds__(W * kWave, MINW) void k_ln_bwd_vec(
         o.y = dx[q][v].y + r[q] * (dn.y - dnm - xh.y * dnxm);
         o.z = dx[q][v].z + r[q] * (dn.z - dnm - xh.z * dnxm);
         o.w = dx[q][v].w + r[q] * (dn.w - dnm - xh.w * dnxm);
-        if (cl.in[v] && live) {
-          const size_t e = off[q] + cl.col[v];
+        if (cl.any(v) && live) {
           if (kDinp == kDinpRw) {
             if (kNt)
-              st_nt(dx4 + e, o);
+              cl.put(dinp + off[q], v, o);
             else
-              dx4[e] = o;
+              st4(dinp + off[q] + cl.at[v], o);
           }
           if (kRes) {
             float4 a = add4(ra[kRes ? q : 0][kRes ? v : 0], o);
             if (same) {
               a = add4(a, o);
             } else {
-              st_nt(b4 + e, add4(rb[kRes ? q : 0][kRes ? v : 0], o));
+              cl.put(rdy + off[q], v, add4(rb[kRes ? q : 0][kRes ? v : 0], o));
             }
-            st_nt(a4 + e, a);
+            cl.put(rdx + off[q], v, a);
           }
         }
         if (q > 0 && !live) continue;  // uniform across the wavefront: a branch, not a mask per lane
-        const bool c = cl.in[v];
-        ab[v].x += c ? dy[q][v].x : -0.0f; ag[v].x += c ? dy[q][v].x * xh.x : -0.0f;
-        ab[v].y += c ? dy[q][v].y : -0.0f; ag[v].y += c ? dy[q][v].y * xh.y : -0.0f;
-        ab[v].z += c ? dy[q][v].z : -0.0f; ag[v].z += c ? dy[q][v].z * xh.z : -0.0f;
-        ab[v].w += c ? dy[q][v].w : -0.0f; ag[v].w += c ? dy[q][v].w * xh.w : -0.0f;
+        ab[v].x += cl.sel(v, 0, dy[q][v].x); ag[v].x += cl.sel(v, 0, dy[q][v].x * xh.x);
+        ab[v].y += cl.sel(v, 1, dy[q][v].y); ag[v].y += cl.sel(v, 1, dy[q][v].y * xh.y);
+        ab[v].z += cl.sel(v, 2, dy[q][v].z); ag[v].z += cl.sel(v, 2, dy[q][v].z * xh.z);
+        ab[v].w += cl.sel(v, 3, dy[q][v].w); ag[v].w += cl.sel(v, 3, dy[q][v].w * xh.w);
       }
     }
   }
@@ -542,19 +614,24 @@ __global__ __launch_bounds__(W * kWave, MINW) void k_ln_bwd_vec(
     red[wave][1][v * kWave + lane] = ab[v];
   }
   __syncthreads();
-  float4 *prow = reinterpret_cast<float4 *>(partial + (size_t)blockIdx.x * 2 * C);
+  float *prow = partial + (size_t)blockIdx.x * 2 * C;
   for (int e = threadIdx.x; e < 2 * V * kWave; e += W * kWave) {
     const int which = e >= V * kWave ? 1 : 0;
     const int c4 = e - which * V * kWave;
-    if (c4 < C4) {
+    const Cols<1, kRag> cs(c4, 0, C);
+    if (cs.any(0)) {
       float4 t = red[0][which][c4];
 #pragma unroll
       for (int k = 1; k < W; k++) t = add4(t, red[k][which][c4]);
+      float *q = prow + which * C + cs.at[0];
       if (kTail) {
-        float *q = reinterpret_cast<float *>(prow + which * C4 + c4);
         st_dev(q, t.x); st_dev(q + 1, t.y); st_dev(q + 2, t.z); st_dev(q + 3, t.w);
+      } else if (!kRag || cs.lo[0] == 0) {
+        st4(q, t);
       } else {
-        prow[which * C4 + c4] = t;
+        if (cs.lo[0] <= 1) q[1] = t.y;
+        if (cs.lo[0] <= 2) q[2] = t.z;
+        if (cs.lo[0] <= 3) q[3] = t.w;
       }
     }
   }
@@ -592,12 +669,7 @@ __global__ __launch_bounds__(P * T * kWave, MINW) void k_ln_bwd_team(
   const int c4 = part * kWave + lane;
   const bool in = c4 < C4;
   const int col = in ? c4 : C4 - 1;  // past the row: a valid column, masked out of the sums, never stored
-  const float4 *x4 = reinterpret_cast<const float4 *>(inp);
-  const float4 *dy4 = reinterpret_cast<const float4 *>(dout);
-  float4 *dx4 = reinterpret_cast<float4 *>(dinp);
-  float4 *a4 = reinterpret_cast<float4 *>(rdx);
-  float4 *b4 = reinterpret_cast<float4 *>(rdy);
-  const float4 w = reinterpret_cast<const float4 *>(weight)[col];
+  const float4 w = ld4(weight + 4 * col);
   float4 ag = make_float4(0.f, 0.f, 0.f, 0.f), ab = ag;
   const int t0 = (blockIdx.x * T + team) * rpt;
   const int t1 = min(t0 + rpt, rows);
@@ -612,14 +684,14 @@ __global__ __launch_bounds__(P * T * kWave, MINW) void k_ln_bwd_team(
     for (int q = 0; q < R; q++) {
       live[q] = row + q < t1;
       rq[q] = live[q] ? row + q : last;
-      off[q] = (size_t)rq[q] * C4 + col;
+      off[q] = 4 * ((size_t)rq[q] * C4 + col);
     }
     float4 x[R], dy[R], dx[R], ra[kRes ? R : 1], rb[kRes ? R : 1];
     float m[R], r[R];
 #pragma unroll
     for (int q = 0; q < R; q++) {
-      x[q] = ld_nt(x4 + off[q]);
-      dy[q] = ld_nt(dy4 + off[q]);
+      x[q] = ld_nt4(inp + off[q]);
+      dy[q] = ld_nt4(dout + off[q]);
     }
 #pragma unroll
     for (int q = 0; q < R; q++) {
@@ -627,13 +699,13 @@ __global__ __launch_bounds__(P * T * kWave, MINW) void k_ln_bwd_team(
       r[q] = rstd[rq[q]];
     }
 #pragma unroll
-    for (int q = 0; q < R; q++) dx[q] = kDinp == kDinpNone ? zero4() : ld_nt(dx4 + off[q]);
+    for (int q = 0; q < R; q++) dx[q] = kDinp == kDinpNone ? zero4() : ld_nt4(dinp + off[q]);
     if (kRes) {
       // rdy is loaded even when it is rdx (same): a valid address, never used
 #pragma unroll
       for (int q = 0; q < R; q++) {
-        ra[kRes ? q : 0] = kAssign ? zero4() : ld_nt(a4 + off[q]);
-        rb[kRes ? q : 0] = kAssign ? zero4() : ld_nt(b4 + off[q]);
+        ra[kRes ? q : 0] = kAssign ? zero4() : ld_nt4(rdx + off[q]);
+        rb[kRes ? q : 0] = kAssign ? zero4() : ld_nt4(rdy + off[q]);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -672,18 +744,18 @@ __global__ __launch_bounds__(P * T * kWave, MINW) void k_ln_bwd_team(
       if (in) {
         if (kDinp == kDinpRw) {
           if (kNt)
-            st_nt(dx4 + off[q], o);
+            st_nt4(dinp + off[q], o);
           else
-            dx4[off[q]] = o;
+            st4(dinp + off[q], o);
         }
         if (kRes) {
           float4 a = add4(ra[kRes ? q : 0], o);
           if (same) {
             a = add4(a, o);
           } else {
-            st_nt(b4 + off[q], add4(rb[kRes ? q : 0], o));
+            st_nt4(rdy + off[q], add4(rb[kRes ? q : 0], o));
           }
-          st_nt(a4 + off[q], a);
+          st_nt4(rdx + off[q], a);
         }
       }
       ab.x += dy[q].x; ag.x += dy[q].x * xh[q].x;
@@ -695,24 +767,300 @@ __global__ __launch_bounds__(P * T * kWave, MINW) void k_ln_bwd_team(
   red[team][0][c4] = ag;
   red[team][1][c4] = ab;
   __syncthreads();
-  float4 *prow = reinterpret_cast<float4 *>(partial + (size_t)blockIdx.x * 2 * C);
+  float *prow = partial + (size_t)blockIdx.x * 2 * C;
   for (int e = threadIdx.x; e < 2 * C4; e += P * T * kWave) {
     const int which = e >= C4 ? 1 : 0;
     const int cc = e - which * C4;
     float4 t = red[0][which][cc];
 #pragma unroll
     for (int k = 1; k < T; k++) t = add4(t, red[k][which][cc]);
+    float *q = prow + 4 * (which * C4 + cc);
     if (kTail) {
-      float *q = reinterpret_cast<float *>(prow + which * C4 + cc);
       st_dev(q, t.x); st_dev(q + 1, t.y); st_dev(q + 2, t.z); st_dev(q + 3, t.w);
     } else {
-      prow[which * C4 + cc] = t;
+      st4(q, t);
     }
   }
   if (kTail) ln_bwd_tail<P * T * kWave>(partial, (int)gridDim.x, C, dweight, dbias);
 }
 
-// Backward for any C and alignment. Phase 1: one wavefront per row writes
+// What a backward kernel whose register budget does not depend on it does with
+// dinp and the residual targets: the kDinp and kAssign of k_ln_bwd_vec, the
+// same in every thread.
+struct LnBwdMode {
+  bool read_dinp, write_dinp, assign, same;
+};
+
+// The terms of a row slot: xhat and dout * w.
+__device__ __forceinline__ float4 ln_xhat4(float4 x, float m, float r) {
+  return make_float4((x.x - m) * r, (x.y - m) * r, (x.z - m) * r, (x.w - m) * r);
+}
+__device__ __forceinline__ float4 mul4(float4 a, float4 b) {
+  return make_float4(a.x * b.x, a.y * b.y, a.z * b.z, a.w * b.w);
+}
+// dinp + r (dn - mean(dn) - xhat mean(dn xhat))
+__device__ __forceinline__ float4 ln_dinp4(float4 dx, float r, float4 dn, float4 xh, float dnm, float dnxm) {
+  return make_float4(dx.x + r * (dn.x - dnm - xh.x * dnxm), dx.y + r * (dn.y - dnm - xh.y * dnxm),
+                     dx.z + r * (dn.z - dnm - xh.z * dnxm), dx.w + r * (dn.w - dnm - xh.w * dnxm));
+}
+
+// A lane's share of a row's two sums.
+template <int V>
+__device__ __forceinline__ void ln_bwd_lane_sums(const float4 (&x)[V], const float4 (&dy)[V], const float4 (&w)[V],
+                                                 float m, float r, const Cols<V, true> &cl, float &s1, float &s2) {
+  s1 = s2 = 0.0f;
+#pragma unroll
+  for (int v = 0; v < V; v++) {
+    const float4 xh = ln_xhat4(x[v], m, r), dn = mul4(dy[v], w[v]);
+    s1 += cl.sel(v, 0, dn.x); s2 += cl.sel(v, 0, dn.x * xh.x);
+    s1 += cl.sel(v, 1, dn.y); s2 += cl.sel(v, 1, dn.y * xh.y);
+    s1 += cl.sel(v, 2, dn.z); s2 += cl.sel(v, 2, dn.z * xh.z);
+    s1 += cl.sel(v, 3, dn.w); s2 += cl.sel(v, 3, dn.w * xh.w);
+  }
+}
+
+// One row's outputs in a lane's slots, from its two sums over C.
+template <int V, bool kRes>
+__device__ __forceinline__ void ln_bwd_row_out(const float4 (&x)[V], const float4 (&dy)[V], const float4 (&w)[V],
+                                               const float4 (&dx)[V], const float4 (&ra)[kRes ? V : 1],
+                                               const float4 (&rb)[kRes ? V : 1], float m, float r, float dnm,
+                                               float dnxm, const Cols<V, true> &cl, LnBwdMode md, float *dinp,
+                                               float *rdx, float *rdy) {
+#pragma unroll
+  for (int v = 0; v < V; v++) {
+    const float4 o = ln_dinp4(dx[v], r, mul4(dy[v], w[v]), ln_xhat4(x[v], m, r), dnm, dnxm);
+    if (cl.any(v)) {
+      if (md.write_dinp) cl.put(dinp, v, o);
+      if (kRes) {
+        float4 a = add4(ra[kRes ? v : 0], o);
+        if (md.same)
+          a = add4(a, o);
+        else
+          cl.put(rdy, v, add4(rb[kRes ? v : 0], o));
+        cl.put(rdx, v, a);
+      }
+    }
+  }
+}
+
+// Backward for rows of more than 2,048 channels: a workgroup of W wavefronts
+// takes rpw consecutive rows, R at a time, V float4 of each per lane. A row's
+// two sums are a lane sum, a wavefront sum and the W wavefronts' sums in order
+// (one barrier per pass, LDS double-buffered by pass); dweight/dbias terms are
+// added in registers in row order, and since a lane keeps its columns for all
+// of the workgroup's rows, they go straight to the workgroup's partial row.
+// Memory-bound: 4,092 x 4,096 in 50.9 us (5.3 TB/s), 167 us in the lane loops,
+// which read x and dout three times and add a column's rows one load at a time.
+template <int V, int W, int R, bool kRes>
+__global__ __launch_bounds__(W * kWave) void k_ln_bwd_wide(float *__restrict__ dinp, float *__restrict__ partial,
+                                                           const float *__restrict__ dout,
+                                                           const float *__restrict__ inp,
+                                                           const float *__restrict__ weight,
+                                                           const float *__restrict__ mean,
+                                                           const float *__restrict__ rstd, int rows, int C, int rpw,
+                                                           float *__restrict__ rdx, float *__restrict__ rdy,
+                                                           LnBwdMode md) {
+  __shared__ float part[2][R][W][2];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & (kWave - 1);
+  const float Cf = (float)C;
+  const Cols<V, true> cl(threadIdx.x, W * kWave, C);
+  float4 w[V], ag[V], ab[V];
+#pragma unroll
+  for (int v = 0; v < V; v++) {
+    w[v] = ld4(weight + cl.at[v]);
+    ag[v] = ab[v] = zero4();
+  }
+  const int row0 = blockIdx.x * rpw, row1 = min(row0 + rpw, rows);
+  for (int row = row0, ps = 0; row < row1; row += R, ps ^= 1) {
+    float4 x[R][V], dy[R][V], dx[R][V], ra[R][kRes ? V : 1], rb[R][kRes ? V : 1];
+    float m[R], r[R];
+    size_t off[R];
+#pragma unroll
+    for (int q = 0; q < R; q++) {  // rows past the end repeat the last one: computed, neither stored nor summed
+      const int rq = min(row + q, row1 - 1);
+      off[q] = (size_t)rq * C;
+      m[q] = mean[rq];
+      r[q] = rstd[rq];
+#pragma unroll
+      for (int v = 0; v < V; v++) {
+        x[q][v] = ld_nt4(inp + off[q] + cl.at[v]);
+        dy[q][v] = ld_nt4(dout + off[q] + cl.at[v]);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < R; q++)
+#pragma unroll
+      for (int v = 0; v < V; v++) {
+        dx[q][v] = md.read_dinp ? ld_nt4(dinp + off[q] + cl.at[v]) : zero4();
+        if (kRes) {
+          ra[q][kRes ? v : 0] = md.assign ? zero4() : ld_nt4(rdx + off[q] + cl.at[v]);
+          rb[q][kRes ? v : 0] = md.assign ? zero4() : ld_nt4(rdy + off[q] + cl.at[v]);
+        }
+      }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+      float s1, s2;
+      ln_bwd_lane_sums<V>(x[q], dy[q], w, m[q], r[q], cl, s1, s2);
+      s1 = wave_sum(s1);
+      s2 = wave_sum(s2);
+      if (lane == 0) {
+        part[ps][q][wave][0] = s1;
+        part[ps][q][wave][1] = s2;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+      if (row + q >= row1) break;  // the same in every thread
+      float s1 = part[ps][q][0][0], s2 = part[ps][q][0][1];
+#pragma unroll
+      for (int k = 1; k < W; k++) {
+        s1 += part[ps][q][k][0];
+        s2 += part[ps][q][k][1];
+      }
+      ln_bwd_row_out<V, kRes>(x[q], dy[q], w, dx[q], ra[q], rb[q], m[q], r[q], s1 / Cf, s2 / Cf, cl, md,
+                              dinp + off[q], rdx + off[q], rdy + off[q]);
+#pragma unroll
+      for (int v = 0; v < V; v++) {
+        ab[v] = add4(ab[v], dy[q][v]);
+        ag[v] = add4(ag[v], mul4(dy[q][v], ln_xhat4(x[q][v], m[q], r[q])));
+      }
+    }
+  }
+  float *prow = partial + (size_t)blockIdx.x * 2 * C;
+#pragma unroll
+  for (int v = 0; v < V; v++)
+    if (cl.any(v)) {
+      cl.put(prow, v, ag[v]);
+      cl.put(prow + C, v, ab[v]);
+    }
+}
+
+// Backward of few rows without partial rows. What bounds it is latency: a
+// launch, one round trip to memory, the reductions. A call's first workgroups
+// finish dweight and dbias by themselves, 16 columns each, reading x and dout
+// once more (they are in the caches): 64 groups of consecutive rows, each
+// added in row order, every eighth group together, then those eight sums as a
+// tree, then onto the arrays' values.
+// The others write dinp (and the residual targets), P wavefronts per row, every
+// row's loads in flight at once. The step driver's calls have the row
+// workgroups alone (ncol = 0), and one launch at its end takes the columns of
+// all its LayerNorms (k_ln_small_cols_batch). Per call, against the two launches
+// of the larger shapes' kernels: 256 x 384 3.6 against 8.6 us, 512 x 768 4.1
+// against 9.7, 1,024 x 384 6.4 against 9.0. Too few column workgroups then
+// stream too much each: 768 x 768 10.1 against 10.4, 1,024 x 768 13.4 against
+// 9.9 (8 or 32 columns a workgroup, and longer batches, moved that by 2 us at
+// most), hence small_path.
+constexpr int kSmallCols = 16, kSmallSlots = kSmallCols / 4, kSmallGroups = kBlock / kSmallSlots, kSmallBatch = 4;
+
+__device__ __forceinline__ void ln_small_cols(float (*red)[2][kSmallCols], int blk, float *__restrict__ dweight,
+                                              float *__restrict__ dbias, const float *__restrict__ dout,
+                                              const float *__restrict__ inp, const float *__restrict__ mean,
+                                              const float *__restrict__ rstd, int rows, int C) {
+  const int l = threadIdx.x % kSmallSlots, g = threadIdx.x / kSmallSlots;
+  const Cols<1, true> cl(blk * kSmallSlots + l, 0, C);
+  // the adder thread's column: component col % 4 of slot col / 4, if that is the slot's own
+  const int which = (int)threadIdx.x / kSmallCols, col = (int)threadIdx.x % kSmallCols;
+  const Cols<1, true> cc(blk * kSmallSlots + col / 4, 0, C);
+  const bool adder = (int)threadIdx.x < 2 * kSmallCols && cc.own(0, col & 3);
+  float *const dst = (which ? dbias : dweight) + cc.at[0] + (col & 3);
+  const float prev = adder ? *dst : 0.0f;
+  float4 ag = zero4(), ab = zero4();
+  const int J = (rows + kSmallGroups - 1) / kSmallGroups;
+  const int j0 = min(g * J, rows), j1 = min(j0 + J, rows);
+  for (int b = j0; b < j1; b += kSmallBatch) {
+    float4 x[kSmallBatch], dy[kSmallBatch];
+    float m[kSmallBatch], r[kSmallBatch];
+#pragma unroll
+    for (int q = 0; q < kSmallBatch; q++) {
+      const int row = min(b + q, j1 - 1);
+      x[q] = ld4(inp + (size_t)row * C + cl.at[0]);
+      dy[q] = ld4(dout + (size_t)row * C + cl.at[0]);
+      m[q] = mean[row];
+      r[q] = rstd[row];
+    }
+#pragma unroll
+    for (int q = 0; q < kSmallBatch; q++) {
+      if (b + q >= j1) break;
+      ab = add4(ab, dy[q]);
+      ag = add4(ag, mul4(dy[q], ln_xhat4(x[q], m[q], r[q])));
+    }
+  }
+  *reinterpret_cast<float4 *>(&red[g][0][4 * l]) = ag;
+  *reinterpret_cast<float4 *>(&red[g][1][4 * l]) = ab;
+  __syncthreads();
+  if (adder) {
+    float t[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      t[k] = red[k][which][col];
+#pragma unroll
+      for (int j = k + 8; j < kSmallGroups; j += 8) t[k] += red[j][which][col];
+    }
+    *dst = prev + (((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7])));
+  }
+}
+
+template <int V, int P, bool kRes>
+__global__ __launch_bounds__(kBlock) void k_ln_bwd_small(float *__restrict__ dinp, float *__restrict__ dweight,
+                                                         float *__restrict__ dbias, const float *__restrict__ dout,
+                                                         const float *__restrict__ inp,
+                                                         const float *__restrict__ weight,
+                                                         const float *__restrict__ mean,
+                                                         const float *__restrict__ rstd, int rows, int C, int ncol,
+                                                         float *__restrict__ rdx, float *__restrict__ rdy,
+                                                         LnBwdMode md) {
+  __shared__ __align__(16) float red[kSmallGroups][2][kSmallCols];
+  if ((int)blockIdx.x < ncol) {
+    ln_small_cols(red, blockIdx.x, dweight, dbias, dout, inp, mean, rstd, rows, C);
+    return;
+  }
+  constexpr int T = kWavesPerBlock / P;  // rows per workgroup
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & (kWave - 1);
+  const int row = ((int)blockIdx.x - ncol) * T + wave / P;
+  if (P == 1 && row >= rows) return;  // P > 1: one row per workgroup, all of them rows
+  const Cols<V, true> cl(wave % P * kWave + lane, P * kWave, C);
+  const size_t off = (size_t)row * C;
+  const float m = mean[row], r = rstd[row];
+  float4 x[V], dy[V], w[V], dx[V], ra[kRes ? V : 1], rb[kRes ? V : 1];
+#pragma unroll
+  for (int v = 0; v < V; v++) {
+    x[v] = ld_nt4(inp + off + cl.at[v]);
+    dy[v] = ld_nt4(dout + off + cl.at[v]);
+    w[v] = ld4(weight + cl.at[v]);
+    dx[v] = md.read_dinp ? ld_nt4(dinp + off + cl.at[v]) : zero4();
+    if (kRes) {
+      ra[kRes ? v : 0] = md.assign ? zero4() : ld_nt4(rdx + off + cl.at[v]);
+      rb[kRes ? v : 0] = md.assign ? zero4() : ld_nt4(rdy + off + cl.at[v]);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  float s1, s2;
+  ln_bwd_lane_sums<V>(x, dy, w, m, r, cl, s1, s2);
+  s1 = wave_sum(s1);
+  s2 = wave_sum(s2);
+  if (P > 1) {
+    float(*part)[2] = reinterpret_cast<float(*)[2]>(&red[0][0][0]);
+    if (lane == 0) {
+      part[wave][0] = s1;
+      part[wave][1] = s2;
+    }
+    __syncthreads();
+    s1 = part[0][0];
+    s2 = part[0][1];
+#pragma unroll
+    for (int k = 1; k < P; k++) {
+      s1 += part[k][0];
+      s2 += part[k][1];
+    }
+  }
+  ln_bwd_row_out<V, kRes>(x, dy, w, dx, ra, rb, m, r, s1 / (float)C, s2 / (float)C, cl, md, dinp + off, rdx + off,
+                          rdy + off);
+}
+
+// Backward for the rows that no kernel above takes (C < 4 or beyond 8,192).
+// Phase 1: one wavefront per row writes
 // dinp. Phase 2: thread-per-channel column sums over the workgroup's rows.
 __global__ __launch_bounds__(kBlock) void k_ln_bwd_scalar(float *dinp, float *partial, const float *dout,
                                                           const float *inp, const float *weight,
@@ -814,12 +1162,18 @@ __global__ __launch_bounds__(kRedCols * kRedGroups) void k_ln_bwd_reduce_batch(L
   ln_bwd_reduce_tile(j.dweight, j.dbias, j.partial, j.nblk, C, red);
 }
 
-bool vec_ok(int C, std::initializer_list<const void *> ptrs) {
-  if ((C & 3) != 0 || C > kMaxV * kWave * 4) return false;
-  for (const void *p : ptrs)
-    if (!aligned16(p)) return false;
-  return true;
+// The columns of several few-row LayerNorms in one launch (blockIdx.y picks the job).
+__global__ __launch_bounds__(kBlock) void k_ln_small_cols_batch(LnReduceBatch b, int rows, int C) {
+  __shared__ __align__(16) float red[kSmallGroups][2][kSmallCols];
+  const LnReduceJob &j = b.job[blockIdx.y];
+  ln_small_cols(red, blockIdx.x, j.dweight, j.dbias, j.dout, j.inp, j.mean, j.rstd, rows, C);
 }
+
+// Which kernels take rows of C channels, at any alignment: one wavefront per
+// row up to 2,048, a workgroup per row up to 8,192, else the lane loops.
+bool row_in_wave(int C) { return C >= 4 && C <= kMaxV * kWave * 4; }
+bool row_in_block(int C) { return C > kMaxV * kWave * 4 && C <= kMaxWide; }
+int slots_of(int C, int lanes) { return ((C + 3) / 4 + lanes - 1) / lanes; }  // float4 per lane
 
 // Scalar path: workgroups of 4 wavefronts, at most max_blocks of them.
 void bwd_shape(int rows, int max_blocks, int *nblk, int *rpb) {
@@ -886,7 +1240,7 @@ int cu_count() {
 // for the plain backward (41.7 against 45.0 us with the column sums).
 constexpr int kTeamParts = 3, kTeams = 4, kTeamRows = 4;
 bool team_path(int rows, int C) {
-  return ((C >> 2) + kWave - 1) / kWave == kTeamParts && rows <= cu_count() * 32;
+  return (C & 3) == 0 && slots_of(C, kWave) == kTeamParts && rows <= cu_count() * 32;
 }
 void team_shape(int rows, int max_blocks, int *nblk, int *rpt) {
   const int per_team = (rows + max_blocks * kTeams - 1) / (max_blocks * kTeams);
@@ -899,7 +1253,7 @@ void team_shape(int rows, int max_blocks, int *nblk, int *rpt) {
 // depend on the device the call later runs on.
 int vec_blocks(int rows, int C, bool res, int max_blocks) {
   int nblk, rpw;
-  const int V = ((C >> 2) + kWave - 1) / kWave;
+  const int V = slots_of(C, kWave);
   bwd_shape_vec(rows, bwd_cfg(V, res), max_blocks, &nblk, &rpw);
   if (V == kTeamParts) {
     int nt, rpt;
@@ -909,22 +1263,51 @@ int vec_blocks(int rows, int C, bool res, int max_blocks) {
   return nblk;
 }
 
+// Workgroup-per-row path: W wavefronts per workgroup, at least 4 rows each (as
+// many partial rows as the scalar path may take, which sizes the workspace),
+// at most 512 workgroups.
+constexpr int kWideWaves = 8, kWideRows = 4;
+void wide_shape(int rows, int max_blocks, int *nblk, int *rpw) {
+  const int cap = std::min(max_blocks, kMaxScalarBlocks);
+  const int per = (rows + cap - 1) / cap;
+  *rpw = per < kWideRows ? kWideRows : per;
+  *nblk = (rows + *rpw - 1) / *rpw;
+}
+
+// The backward without partial rows (k_ln_bwd_small, which has the timings on
+// both sides of the line).
+bool small_path(int rows, int C) {
+  if (!row_in_wave(C) && !row_in_block(C)) return false;
+  return rows <= 512 ? (size_t)rows * C <= ((size_t)1 << 20) : rows <= 1024 && C <= 384;
+}
+
 // Rows per wavefront of the fused forward: two while one wavefront per row
 // would fill the GPU only once (the reads and writes of a single round of
 // wavefronts cannot overlap; measured 17.7 against 18.8 us at 8,192 x 768),
-// else one (35.0 against 37.1 us at 16,384 x 768). The plain forward keeps
-// one (9.3 against 9.6 us with two at 8,192 x 768).
-int fwd_rpw(int rows, bool res) {
+// else one (35.0 against 37.1 us at 16,384 x 768), and one again while a SIMD
+// waits for its rows anyway (fwd_early), where a wavefront's second row only
+// adds to the latency (1,024 x 768 4.6 against 5.4 us, 256 x 384 3.3 against
+// 3.9, 512 x 1,600 5.7 against 7.9). The plain forward keeps one (9.3 against
+// 9.6 us with two at 8,192 x 768).
+// Weight and bias loaded early (ln_row_out): up to two rows per SIMD, of rows
+// that keep it waiting (2,048 x 768 6.4 against 6.9 us, but 2,048 x 1,600 12.1
+// against 11.0 and 2,000 x 1,024 8.1 against 7.8).
+bool fwd_early(int rows, int C) { return rows <= cu_count() * 8 && (size_t)rows * C <= ((size_t)3 << 19); }
+int fwd_rpw(int rows, int C, bool res) {
   if (!res) return 1;
-  return rows <= cu_count() * 32 ? 2 : 1;
+  return !fwd_early(rows, C) && rows <= cu_count() * 32 ? 2 : 1;
 }
 
 }  // namespace
 
 int layernorm_backward_blocks(int rows, int C, bool res, int max_blocks) {
   if (rows <= 0) return 0;
-  if ((C & 3) == 0 && C <= kMaxV * kWave * 4) return vec_blocks(rows, C, res, max_blocks);
+  if (row_in_wave(C)) return vec_blocks(rows, C, res, max_blocks);
   int nblk, rpb;
+  if (row_in_block(C)) {
+    wide_shape(rows, max_blocks, &nblk, &rpb);
+    return nblk;
+  }
   bwd_shape(rows, max_blocks < kMaxScalarBlocks ? max_blocks : kMaxScalarBlocks, &nblk, &rpb);
   return nblk;
 }
@@ -956,21 +1339,35 @@ size_t layernorm_backward_scratch(int rows, int C) {
 }
 
 namespace {
+// Rows of 4 to 8,192 channels, at any alignment.
 template <bool kRes>
-void launch_ln_fwd_vec(float *out, float *mean, float *rstd, const float *inp, const float *weight,
-                       const float *bias, int rows, int C, float *res, const float *inp2) {
-  const int V = ((C >> 2) + kWave - 1) / kWave;
-  const int rpw = fwd_rpw(rows, kRes);
+void launch_ln_fwd_rows(float *out, float *mean, float *rstd, const float *inp, const float *weight,
+                        const float *bias, int rows, int C, float *res, const float *inp2) {
+  if (row_in_block(C)) {
+    // 4 wavefronts with 3 or 4 float4 per lane up to 4,096 channels, 8 up to 8,192
+    const bool w8 = C > 4 * kWave * 4 * 4;
+    const int V = slots_of(C, (w8 ? 8 : 4) * kWave);
+    const auto go = [&](auto k, int W) {
+      launch(k, dim3(rows), dim3(W * kWave), 0, out, mean, rstd, inp, weight, bias, C, res, inp2);
+    };
+    if (!w8 && V <= 3) go(k_ln_fwd_wide<3, 4, kRes>, 4);
+    else if (!w8) go(k_ln_fwd_wide<4, 4, kRes>, 4);
+    else if (V <= 3) go(k_ln_fwd_wide<3, 8, kRes>, 8);
+    else go(k_ln_fwd_wide<4, 8, kRes>, 8);
+    return;
+  }
+  const bool rag = (C & 3) != 0, early = fwd_early(rows, C);
+  const int rpw = rag ? 1 : fwd_rpw(rows, C, kRes);
   const dim3 grid(grid_for((size_t)rows, (size_t)kWavesPerBlock * rpw)), block(kBlock);
-  switch (V * 2 + (rpw - 1)) {
-#define UGK_LN_FWD(v)                                                                                           \
-  case 2 * v:                                                                                                   \
-    launch((k_ln_fwd_vec<v, kRes, 1>), grid, block, 0, out, mean, rstd, inp, weight, bias, \
-                       rows, C, res, inp2);                                                                     \
-    break;                                                                                                      \
-  case 2 * v + 1:                                                                                               \
-    launch((k_ln_fwd_vec<v, kRes, 2>), grid, block, 0, out, mean, rstd, inp, weight, bias, \
-                       rows, C, res, inp2);                                                                     \
+  const auto go = [&](auto k) { launch(k, grid, block, 0, out, mean, rstd, inp, weight, bias, rows, C, res, inp2); };
+  switch (slots_of(C, kWave)) {
+#define UGK_LN_FWD(v)                                                  \
+  case v:                                                              \
+    if (rag && early) go(k_ln_fwd_vec<v, kRes, 1, true, true>);        \
+    else if (rag) go(k_ln_fwd_vec<v, kRes, 1, true, false>);           \
+    else if (early) go(k_ln_fwd_vec<v, kRes, 1, false, true>);         \
+    else if (rpw == 1) go(k_ln_fwd_vec<v, kRes, 1, false, false>);     \
+    else go(k_ln_fwd_vec<v, kRes, 2, false, false>);                   \
     break;
     UGK_LN_FWD(1) UGK_LN_FWD(2) UGK_LN_FWD(3) UGK_LN_FWD(4)
     UGK_LN_FWD(5) UGK_LN_FWD(6) UGK_LN_FWD(7) UGK_LN_FWD(8)
@@ -983,11 +1380,11 @@ int launch_residual_layernorm_forward(float *res, float *out, float *mean, float
                                       const float *y, const float *weight, const float *bias, int rows,
                                       int C) {
   if (rows == 0) return 0;
-  if (layernorm_exact() || !vec_ok(C, {res, out, x, y, weight, bias})) {
+  if (layernorm_exact() || !(row_in_wave(C) || row_in_block(C))) {
     if (int e = launch_residual_forward(res, x, y, (size_t)rows * C)) return e;
     return launch_layernorm_forward(out, mean, rstd, res, weight, bias, rows, C);
   }
-  launch_ln_fwd_vec<true>(out, mean, rstd, x, weight, bias, rows, C, res, y);
+  launch_ln_fwd_rows<true>(out, mean, rstd, x, weight, bias, rows, C, res, y);
   return check_launch("residual_layernorm_forward");
 }
 
@@ -996,22 +1393,22 @@ int launch_encoder_layernorm_forward(float *enc, float *out, float *mean, float 
                                      int B, int T, int C) {
   const int rows = B * T;
   if (rows == 0) return 0;
-  if (layernorm_exact() || !vec_ok(C, {enc, out, wte, wpe, weight, bias})) {
+  if (layernorm_exact() || !row_in_wave(C) || (C & 3) != 0) {
     if (int e = launch_encoder_forward(enc, inp, wte, wpe, B, T, C)) return e;
     return launch_layernorm_forward(out, mean, rstd, enc, weight, bias, rows, C);
   }
-  const int V = ((C >> 2) + kWave - 1) / kWave;
-  const int rpw = fwd_rpw(rows, true);
+  const int V = slots_of(C, kWave);
+  const int rpw = fwd_rpw(rows, C, true);
   const dim3 grid(grid_for((size_t)rows, (size_t)kWavesPerBlock * rpw)), block(kBlock);
-  switch (V * 2 + (rpw - 1)) {
-#define UGK_ENC_LN(v)                                                                                          \
-  case 2 * v:                                                                                                  \
-    launch((k_enc_ln_fwd_vec<v, 1>), grid, block, 0, enc, out, mean, rstd, inp, wte, wpe, weight, bias, rows, \
-           T, C);                                                                                              \
-    break;                                                                                                     \
-  case 2 * v + 1:                                                                                              \
-    launch((k_enc_ln_fwd_vec<v, 2>), grid, block, 0, enc, out, mean, rstd, inp, wte, wpe, weight, bias, rows, \
-           T, C);                                                                                              \
+  const auto go = [&](auto k) {
+    launch(k, grid, block, 0, enc, out, mean, rstd, inp, wte, wpe, weight, bias, rows, T, C);
+  };
+  switch (V) {
+#define UGK_ENC_LN(v)                                             \
+  case v:                                                         \
+    if (fwd_early(rows, C)) go(k_enc_ln_fwd_vec<v, 1, true>);        \
+    else if (rpw == 1) go(k_enc_ln_fwd_vec<v, 1, false>);         \
+    else go(k_enc_ln_fwd_vec<v, 2, false>);                       \
     break;
     UGK_ENC_LN(1) UGK_ENC_LN(2) UGK_ENC_LN(3) UGK_ENC_LN(4)
     UGK_ENC_LN(5) UGK_ENC_LN(6) UGK_ENC_LN(7) UGK_ENC_LN(8)
@@ -1469,8 +1866,8 @@ int launch_layernorm_forward(float *out, float *mean, float *rstd, const float *
                              const float *weight, const float *bias, int rows, int C) {
   if (rows == 0) return 0;
   if (layernorm_exact()) return launch_layernorm_forward_exact(out, mean, rstd, inp, weight, bias, rows, C);
-  if (vec_ok(C, {out, inp, weight, bias})) {
-    launch_ln_fwd_vec<false>(out, mean, rstd, inp, weight, bias, rows, C, nullptr, nullptr);
+  if (row_in_wave(C) || row_in_block(C)) {
+    launch_ln_fwd_rows<false>(out, mean, rstd, inp, weight, bias, rows, C, nullptr, nullptr);
   } else {
     const dim3 grid(grid_for((size_t)rows, kWavesPerBlock)), block(kBlock);
     launch(k_ln_fwd_scalar, grid, block, 0, out, mean, rstd, inp, weight, bias,
@@ -1491,7 +1888,7 @@ int launch_ln_bwd_vec(float *dinp, float *partial, const float *dout, const floa
   static_assert(kRes || (kDinp == kDinpRw && !kAssign), "the plain backward reads and writes dinp");
   constexpr bool kTailOk = kDinp == kDinpRw && !kAssign;
   int nblk, rpw;
-  const int V = ((C >> 2) + kWave - 1) / kWave;
+  const int V = slots_of(C, kWave);
   const int same = rdx == rdy ? 1 : 0;
   const bool nt = (size_t)rows * (size_t)C < ((size_t)1 << 21);
   // the kernel with and without the in-launch column sums
@@ -1521,12 +1918,19 @@ int launch_ln_bwd_vec(float *dinp, float *partial, const float *dout, const floa
   const BwdCfg k = bwd_cfg(V, kRes);
   bwd_shape_vec(rows, k, max_blocks, &nblk, &rpw);
   const dim3 grid(nblk), block(k.W * kWave);
+  const bool rag = (C & 3) != 0;  // takes only the modes of the per-op calls (kTailOk)
   switch (V) {
 #define UGK_LN_BWD_K(v, ntv, tl)                                                                                    \
-  k_ln_bwd_vec<v, bwd_cfg(v, kRes).W, bwd_cfg(v, kRes).R, kRes, bwd_cfg(v, kRes).MINW, ntv, kDinp, kAssign, tl>
+  k_ln_bwd_vec<v, bwd_cfg(v, kRes).W, bwd_cfg(v, kRes).R, kRes, bwd_cfg(v, kRes).MINW, ntv, kDinp, kAssign, tl, false>
 #define UGK_LN_BWD(v)                                                                                               \
   case v:                                                                                                           \
-    if (kRes || nt)                                                                                                 \
+    if (rag) {                                                                                                      \
+      if constexpr (kTailOk)                                                                                        \
+        launch(k_ln_bwd_vec<v, bwd_cfg(v, kRes).W, bwd_cfg(v, kRes).R, kRes, bwd_cfg(v, kRes).MINW, true, kDinpRw,   \
+                            false, false, true>,                                                                    \
+               grid, block, 0, dinp, partial, dout, inp, weight, mean, rstd, rows, C, rpw, rdx, rdy, same, nullptr, \
+               nullptr);                                                                                            \
+    } else if (kRes || nt)                                                                                          \
       both(UGK_LN_BWD_K(v, true, false), UGK_LN_BWD_K(v, true, kTailOk), grid, block, rpw);                         \
     else                                                                                                            \
       both(UGK_LN_BWD_K(v, kRes, false), UGK_LN_BWD_K(v, kRes, kTailOk), grid, block, rpw);                         \
@@ -1548,31 +1952,91 @@ std::atomic<int> g_ln_tail{0};
 void set_layernorm_tail(int on) { g_ln_tail.store(on ? 1 : 0); }
 int layernorm_tail() { return g_ln_tail.load(); }
 
-int launch_layernorm_backward_partials(float *dinp, float *partial, float *dx, float *dy, const float *dout,
-                                       const float *inp, const float *weight, const float *mean,
-                                       const float *rstd, int rows, int C, int max_blocks, int *nblk,
-                                       int dinp_mode, bool assign_res) {
+namespace {
+// The backward of small_path(rows, C); without the columns if dweight is null.
+template <bool kRes>
+void launch_ln_bwd_small(float *dinp, float *dweight, float *dbias, float *dx, float *dy, const float *dout,
+                         const float *inp, const float *weight, const float *mean, const float *rstd, int rows, int C,
+                         LnBwdMode md) {
+  const bool wide = row_in_block(C);
+  const int ncol = dweight ? (int)grid_for((size_t)C, kSmallCols) : 0;
+  const int nrow = wide ? rows : (int)grid_for((size_t)rows, kWavesPerBlock);
+  const auto go = [&](auto k) {
+    launch(k, dim3(ncol + nrow), dim3(kBlock), 0, dinp, dweight, dbias, dout, inp, weight, mean, rstd, rows, C, ncol, dx,
+           dy, md);
+  };
+  switch (slots_of(C, wide ? kBlock : kWave)) {
+#define UGK_LN_SMALL(v)                              \
+  case v:                                            \
+    if (wide) go(k_ln_bwd_small<v, kWavesPerBlock, kRes>); \
+    else go(k_ln_bwd_small<v, 1, kRes>);             \
+    break;
+    UGK_LN_SMALL(1) UGK_LN_SMALL(2) UGK_LN_SMALL(3) UGK_LN_SMALL(4)
+    UGK_LN_SMALL(5) UGK_LN_SMALL(6) UGK_LN_SMALL(7) UGK_LN_SMALL(8)
+#undef UGK_LN_SMALL
+  }
+}
+
+template <bool kRes>
+void launch_ln_bwd_wide(float *dinp, float *partial, float *dx, float *dy, const float *dout, const float *inp,
+                        const float *weight, const float *mean, const float *rstd, int rows, int C, int max_blocks,
+                        LnBwdMode md, int *nblk) {
+  int rpw;
+  wide_shape(rows, max_blocks, nblk, &rpw);
+  const auto go = [&](auto k) {
+    launch(k, dim3(*nblk), dim3(kWideWaves * kWave), 0, dinp, partial, dout, inp, weight, mean, rstd, rows, C, rpw, dx,
+           dy, md);
+  };
+  const int V = slots_of(C, kWideWaves * kWave);
+  if (V <= 2) go(k_ln_bwd_wide<2, kWideWaves, 2, kRes>);
+  else if (V == 3) go(k_ln_bwd_wide<3, kWideWaves, 1, kRes>);
+  else go(k_ln_bwd_wide<4, kWideWaves, 1, kRes>);
+}
+}  // namespace
+
+int launch_layernorm_backward_partials(float *dinp, float *partial, float *dweight, float *dbias, float *dx, float *dy,
+                                       const float *dout, const float *inp, const float *weight, const float *mean,
+                                       const float *rstd, int rows, int C, int max_blocks, int *nblk, int dinp_mode,
+                                       bool assign_res) {
   *nblk = 0;
   if (rows == 0) return 0;
   const bool res = dx != nullptr;
-  if (vec_ok(C, {dinp, dout, inp, weight}) && (!res || vec_ok(C, {dx, dy}))) {
+  if (!(res && dinp_mode == kDinpNone ? assign_res : !assign_res || (res && dinp_mode == kDinpRead)))
+    return set_error(UGK_EINVAL, "layernorm_backward: unsupported dinp mode %d with assign %d", dinp_mode,
+                     (int)assign_res);
+  const LnBwdMode md{dinp_mode != kDinpNone, dinp_mode == kDinpRw, assign_res, dx == dy};
+  if (small_path(rows, C)) {
+    if (res)
+      launch_ln_bwd_small<true>(dinp, dweight, dbias, dx, dy, dout, inp, weight, mean, rstd, rows, C, md);
+    else
+      launch_ln_bwd_small<false>(dinp, dweight, dbias, dx, dy, dout, inp, weight, mean, rstd, rows, C, md);
+    return check_launch("layernorm_backward");
+  }
+  if (row_in_wave(C)) {
+    // ragged rows have the kernels of the per-op modes only, which read and write everything
+    const int mode = (C & 3) != 0 ? kDinpRw : dinp_mode;
+    const bool assign = (C & 3) == 0 && assign_res;
 #define UGK_LN_BWD_MODE(d, a) \
   launch_ln_bwd_vec<true, d, a>(dinp, partial, dout, inp, weight, mean, rstd, rows, C, dx, dy, max_blocks)
     if (!res)
       *nblk = launch_ln_bwd_vec<false, kDinpRw, false>(dinp, partial, dout, inp, weight, mean, rstd, rows, C,
                                                        nullptr, nullptr, max_blocks);
-    else if (dinp_mode == kDinpRw && !assign_res)
+    else if (mode == kDinpRw)
       *nblk = UGK_LN_BWD_MODE(kDinpRw, false);
-    else if (dinp_mode == kDinpRead && !assign_res)
-      *nblk = UGK_LN_BWD_MODE(kDinpRead, false);
-    else if (dinp_mode == kDinpRead)
-      *nblk = UGK_LN_BWD_MODE(kDinpRead, true);
-    else if (dinp_mode == kDinpNone && assign_res)
+    else if (mode == kDinpNone)
       *nblk = UGK_LN_BWD_MODE(kDinpNone, true);
+    else if (assign)
+      *nblk = UGK_LN_BWD_MODE(kDinpRead, true);
     else
-      return set_error(UGK_EINVAL, "layernorm_backward: unsupported dinp mode %d with assign %d", dinp_mode,
-                       (int)assign_res);
+      *nblk = UGK_LN_BWD_MODE(kDinpRead, false);
 #undef UGK_LN_BWD_MODE
+    return check_launch("layernorm_backward");
+  }
+  if (row_in_block(C)) {
+    if (res)
+      launch_ln_bwd_wide<true>(dinp, partial, dx, dy, dout, inp, weight, mean, rstd, rows, C, max_blocks, md, nblk);
+    else
+      launch_ln_bwd_wide<false>(dinp, partial, dx, dy, dout, inp, weight, mean, rstd, rows, C, max_blocks, md, nblk);
     return check_launch("layernorm_backward");
   }
   int rpb;
@@ -1583,11 +2047,15 @@ int launch_layernorm_backward_partials(float *dinp, float *partial, float *dx, f
   return res ? launch_residual_backward(dx, dy, dinp, (size_t)rows * C) : 0;
 }
 
-int launch_layernorm_reduce(const LnReduceJob *jobs, int njobs, int C) {
+int launch_layernorm_reduce(const LnReduceJob *jobs, int njobs, int rows, int C) {
   for (int j0 = 0; j0 < njobs; j0 += kMaxReduceJobs) {
     LnReduceBatch b{};
     const int n = njobs - j0 < kMaxReduceJobs ? njobs - j0 : kMaxReduceJobs;
     for (int k = 0; k < n; k++) b.job[k] = jobs[j0 + k];
+    if (small_path(rows, C)) {
+      launch(k_ln_small_cols_batch, dim3(grid_for((size_t)C, kSmallCols), n), dim3(kBlock), 0, b, rows, C);
+      continue;
+    }
     launch(k_ln_bwd_reduce_batch, dim3(grid_for((size_t)2 * C, kRedCols), n), dim3(kRedCols * kRedGroups), 0, b,
            C);
   }
@@ -1605,7 +2073,7 @@ int launch_layernorm_residual_backward_into(float *partial, int max_blocks, floa
       return e;
     return res ? launch_residual_backward(dx, dy, dinp, (size_t)rows * C) : 0;
   }
-  if (layernorm_tail() && vec_ok(C, {dinp, dout, inp, weight}) && (!res || vec_ok(C, {dx, dy}))) {
+  if (layernorm_tail() && row_in_wave(C) && (C & 3) == 0 && !small_path(rows, C)) {
     if (res)
       launch_ln_bwd_vec<true, kDinpRw, false>(dinp, partial, dout, inp, weight, mean, rstd, rows, C, dx, dy,
                                               max_blocks, true, dweight, dbias);
@@ -1615,11 +2083,12 @@ int launch_layernorm_residual_backward_into(float *partial, int max_blocks, floa
     return check_launch("layernorm_backward");
   }
   int nblk;
-  if (int e = launch_layernorm_backward_partials(dinp, partial, dx, dy, dout, inp, weight, mean, rstd, rows, C,
-                                                 max_blocks, &nblk))
+  if (int e = launch_layernorm_backward_partials(dinp, partial, dweight, dbias, dx, dy, dout, inp, weight, mean, rstd,
+                                                 rows, C, max_blocks, &nblk))
     return e;
-  const LnReduceJob job{partial, dweight, dbias, nblk};
-  return launch_layernorm_reduce(&job, 1, C);
+  if (nblk == 0) return 0;  // the launch has added the column sums
+  const LnReduceJob job{partial, dweight, dbias, nblk, dout, inp, mean, rstd};
+  return launch_layernorm_reduce(&job, 1, rows, C);
 }
 
 int launch_layernorm_residual_backward(float *dinp, float *dweight, float *dbias, float *dx, float *dy,

@@ -69,9 +69,9 @@ struct Streams {
 
 constexpr unsigned kLine = 32;  // floats of a cache line
 
-// Element i alone.
+// Element i of the pointers alone (before them, where i is negative).
 template <class Op>
-__device__ __forceinline__ void map_one(const Streams<Op> &s, size_t i, const uint64_t *tab) {
+__device__ __forceinline__ void map_one(const Streams<Op> &s, ptrdiff_t i, const uint64_t *tab) {
   float in[Op::kLoads], out[Op::kStores];
 #pragma unroll
   for (int l = 0; l < Op::kLoads; l++) in[l] = s.ld[l][i];
@@ -83,6 +83,8 @@ __device__ __forceinline__ void map_one(const Streams<Op> &s, size_t i, const ui
   for (int o = 0; o < Op::kStores; o++) s.st[o][i] = out[o];
 }
 
+// Float4 slots [0, n4) from the pointers on; the `rest` elements around them,
+// the first `lead` of those before the pointers, by workgroup `full`.
 template <class Op>
 __global__ __launch_bounds__(Op::kThreads) void k_map_vec4(Streams<Op> s, size_t n4, unsigned full, unsigned lead, unsigned rest) {
   __shared__ uint64_t tab[Op::kTable ? 32 : 1];
@@ -92,14 +94,10 @@ __global__ __launch_bounds__(Op::kThreads) void k_map_vec4(Streams<Op> s, size_t
   }
   constexpr int kU = Op::kUnroll, kT = Op::kThreads;
   if (blockIdx.x == full) {  // the workgroup past the float4 slots: the elements around them
-    for (unsigned k = threadIdx.x; k < rest; k += kT) map_one<Op>(s, k < lead ? k : 4 * n4 + k, tab);
+    for (unsigned k = threadIdx.x; k < rest; k += kT)
+      map_one<Op>(s, (ptrdiff_t)k - (ptrdiff_t)lead + (ptrdiff_t)(k < lead ? 0 : 4 * n4), tab);
     return;
   }
-  if (Op::kIndexed) lead = 0;  // as the launch has it: the element index is 4 times the slot's
-#pragma unroll
-  for (int l = 0; l < Op::kLoads; l++) s.ld[l] += lead;
-#pragma unroll
-  for (int o = 0; o < Op::kStores; o++) s.st[o] += lead;
   const size_t base = (size_t)blockIdx.x * (kT * kU) + threadIdx.x;
   float4 v[kU][Op::kLoads];
 #pragma unroll
@@ -117,7 +115,7 @@ __global__ __launch_bounds__(Op::kThreads) void k_map_vec4(Streams<Op> s, size_t
       const size_t i = base + (size_t)u * kT;
       if (i < n4) {
 #pragma unroll
-        for (int e = 0; e < 4; e++) pre[u][e] = Op::pre(lead + 4 * i + e, s.p);
+        for (int e = 0; e < 4; e++) pre[u][e] = Op::pre(4 * i + e, s.p);
       }
     }
   }
@@ -134,9 +132,9 @@ __global__ __launch_bounds__(Op::kThreads) void k_map_vec4(Streams<Op> s, size_t
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         if constexpr (Op::kPre)
-          Op::apply_pre(in[e], out[e], tab, lead + 4 * i + e, s.p, pre[u][e]);
+          Op::apply_pre(in[e], out[e], tab, 4 * i + e, s.p, pre[u][e]);
         else
-          Op::apply(in[e], out[e], tab, lead + 4 * i + e, s.p);
+          Op::apply(in[e], out[e], tab, 4 * i + e, s.p);
       }
 #pragma unroll
       for (int o = 0; o < Op::kStores; o++)
@@ -146,10 +144,12 @@ __global__ __launch_bounds__(Op::kThreads) void k_map_vec4(Streams<Op> s, size_t
 }
 
 template <class Op>
-int run_map(const Streams<Op> &s, size_t n, const char *name) {
+int run_map(Streams<Op> s, size_t n, const char *name) {
   if (n == 0) return 0;
   size_t lead = Op::kIndexed ? 0 : (0 - ((uintptr_t)s.st[0] >> 2)) & (kLine - 1);
   if (lead > n) lead = n;
+  for (int l = 0; l < Op::kLoads; l++) s.ld[l] += lead;
+  for (int o = 0; o < Op::kStores; o++) s.st[o] += lead;
   const size_t n4 = (n - lead) / 4;
   const unsigned full = grid_for(n4, (size_t)Op::kThreads * Op::kUnroll);
   launch(k_map_vec4<Op>, dim3(full + (n != 4 * n4 ? 1 : 0)), dim3(Op::kThreads), Op::kLdsReserve, s, n4, full,
