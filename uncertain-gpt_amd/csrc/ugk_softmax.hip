@@ -24,10 +24,10 @@
 // registers of one workgroup; rows of up to 51,393 (GPT-2's 50257) keep 42
 // slots per thread in registers and 25 in LDS (768 threads), two rows resident
 // per CU so that one row's loads overlap the other's arithmetic and stores
-// (k_softmax_xent_split). Longer rows take two passes
-// instead: one wavefront per row streams the logits once for the exact max
-// and the sum (kept per lane in double and rescaled as the max grows), then a
-// flat map over all rows forms expf(x - max) / sum, 12 bytes per logit.
+// (k_softmax_xent_split). Longer rows take two passes instead: a workgroup per
+// row streams the logits once for the exact max and the sum (kept per lane in
+// double and rescaled as the max grows), then a pass over chunks of all rows
+// forms expf(x - max) / sum, 12 bytes per logit.
 //
 // Exact mode (ugk_set_softmax_exact): the row sum in train_bnn.c's order, one
 // element after another, so that every probability and loss is the CPU's bit
@@ -252,79 +252,87 @@ __device__ __forceinline__ size_t row_of(size_t i, size_t V, double inv_v) {
   return r;
 }
 
-// Long rows, pass 1: one wavefront per row streams its logits once and keeps,
-// per lane, the running max (the CPU's rule, from -1e30) and the sum of
+// Long rows, pass 1: a workgroup per row streams its logits once and keeps, per
+// lane, the running max (the CPU's rule, from -1e30) and the sum of
 // exp(x - running max) in double, rescaled when the max grows; the lanes are
 // then combined onto the row max. stats[row] = {max, sum}. The max is exact;
 // the sum is within float rounding of the exact sum of expf(x - max).
-constexpr int kStatsWaves = 4, kStatsUnroll = 8;
-__global__ __launch_bounds__(kStatsWaves * kWave) void k_softmax_stats(float2 *__restrict__ stats,
-                                                                       const float *__restrict__ logits, int rows,
-                                                                       int V) {
+// A thread holds kStatsUnroll float4 of the row at any alignment, with the next
+// ones loading meanwhile; slots past the row hold -inf, which the max rule
+// skips and whose exponential adds +0.
+// Bound by memory and the exponentials about evenly: 2,048 rows of 100,003 in
+// 179 us (4.6 TB/s). One wavefront per row with 8 dword loads in flight and the
+// branching exponential took 361, and the flat pass that then divided each
+// element (IEEE division, a 64-bit row index per element) 560 against the
+// 247 us of k_softmax_norm_rows; with few rows the workgroup is larger, since
+// it alone fills its CU.
+constexpr int kStatsUnroll = 4;
+template <int kThreads>
+__global__ __launch_bounds__(kThreads) void k_softmax_stats(float2 *__restrict__ stats,
+                                                            const float *__restrict__ logits, int V) {
   __shared__ uint64_t tab[32];
+  __shared__ float lds[kThreads / kWave];
+  __shared__ double lds_d[kThreads / kWave];
   ugk_exp2_stage(tab);
   __syncthreads();
-  const int lane = threadIdx.x & (kWave - 1);
-  const int row = blockIdx.x * kStatsWaves + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const float *lg = logits + (size_t)row * V;
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  const float *lg = logits + (size_t)blockIdx.x * V;
+  const int n4 = V >> 2;  // the long rows: V >= 4
+  const float kNegInf = -__builtin_huge_valf();
+  const UgkExpfAddends add = ugk_expf_addends_vgpr();
+  const auto ex = [&](float d) { return ugk_dev_expf_nooverflow(d, UgkExp2Lds{tab}, add); };
   float m = kNegInit;
   double s = 0.0;
-  for (int v0 = lane; v0 < V; v0 += kWave * kStatsUnroll) {
-    float x[kStatsUnroll];
-#pragma unroll
-    for (int k = 0; k < kStatsUnroll; k++) {
-      const int v = v0 + k * kWave;
-      x[k] = v < V ? ld_nt(lg + v) : kNegInit;
-    }
+  const auto take = [&](const float4 (&x)[kStatsUnroll]) {
     float mb = m;
 #pragma unroll
-    for (int k = 0; k < kStatsUnroll; k++) mb = max_rule(mb, x[k]);
+    for (int k = 0; k < kStatsUnroll; k++)
+      mb = max_rule(max_rule(max_rule(max_rule(mb, x[k].x), x[k].y), x[k].z), x[k].w);
     if (mb != m) {  // rescale the running sum to the new max
-      s *= (double)ugk_expf_t<UGK_EXPF_CONTRACT>(m - mb, UgkExp2Lds{tab});
+      s *= (double)ex(m - mb);
       m = mb;
     }
 #pragma unroll
-    for (int k = 0; k < kStatsUnroll; k++)
-      if (v0 + k * kWave < V) s += (double)ugk_expf_t<UGK_EXPF_CONTRACT>(x[k] - m, UgkExp2Lds{tab});
-  }
-  float M = m;
+    for (int k = 0; k < kStatsUnroll; k++) {
+      s += (double)ex(x[k].x - m);
+      s += (double)ex(x[k].y - m);
+      s += (double)ex(x[k].z - m);
+      s += (double)ex(x[k].w - m);
+    }
+  };
+  const auto load = [&](int q0, float4 (&x)[kStatsUnroll]) {
 #pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) M = max_rule(M, __shfl_xor(M, off));
-  s *= (double)ugk_expf_t<UGK_EXPF_CONTRACT>(m - M, UgkExp2Lds{tab});
+    for (int k = 0; k < kStatsUnroll; k++) {
+      const int q = q0 + k * kThreads;
+      x[k] = ld_nt4(lg + 4 * min(q, n4 - 1));
+      if (q >= n4) x[k] = make_float4(kNegInf, kNegInf, kNegInf, kNegInf);
+    }
+  };
+  constexpr int kStep = kThreads * kStatsUnroll;
+  float4 a[kStatsUnroll], b[kStatsUnroll];
+  load(tid, a);
+  for (int q0 = tid; q0 - tid < n4; q0 += 2 * kStep) {  // the same trip count in every thread
+    load(q0 + kStep, b);
+    take(a);
+    if (q0 - tid + kStep >= n4) break;
+    load(q0 + 2 * kStep, a);
+    take(b);
+  }
+  const int v = 4 * n4 + tid;  // the row's last V % 4 logits
+  if (v < V) {
+    const float x = lg[v], mb = max_rule(m, x);
+    s = s * (double)ex(m - mb) + (double)ex(x - mb);
+    m = mb;
+  }
+  const float M = block_max<kThreads>(m, lds);
+  s *= (double)ex(m - M);
 #pragma unroll
   for (int off = kWave / 2; off > 0; off >>= 1) s += __shfl_xor(s, off);
-  if (lane == 0) stats[row] = make_float2(M, (float)s);
-}
-
-// Long rows, pass 2: a flat map over all rows x V: p = expf(x - max) / sum,
-// and the thread holding a row's target writes its loss.
-constexpr int kNormUnroll = 4;
-__global__ __launch_bounds__(kBlock) void k_softmax_norm(float *__restrict__ losses, float *__restrict__ probs,
-                                                         const float *__restrict__ logits,
-                                                         const int *__restrict__ targets,
-                                                         const float2 *__restrict__ stats, size_t n, int V,
-                                                         double inv_v) {
-  __shared__ uint64_t tab[32];
-  ugk_exp2_stage(tab);
+  if (lane == 0) lds_d[wave] = s;
   __syncthreads();
-  const size_t i0 = (size_t)blockIdx.x * (kBlock * kNormUnroll) + threadIdx.x;
-  float x[kNormUnroll];
-#pragma unroll
-  for (int k = 0; k < kNormUnroll; k++) {
-    const size_t i = i0 + (size_t)k * kBlock;
-    x[k] = i < n ? ld_nt(logits + i) : 0.0f;
-  }
-#pragma unroll
-  for (int k = 0; k < kNormUnroll; k++) {
-    const size_t i = i0 + (size_t)k * kBlock;
-    if (i < n) {
-      const size_t row = row_of(i, (size_t)V, inv_v);
-      const float2 st = stats[row];
-      const float p = ugk_expf_t<UGK_EXPF_CONTRACT>(x[k] - st.x, UgkExp2Lds{tab}) / st.y;
-      st_nt(probs + i, p);
-      if ((int)(i - row * (size_t)V) == targets[row]) losses[row] = neg_logf(p);
-    }
+  if (tid == 0) {
+    for (int w = 1; w < kThreads / kWave; w++) s += lds_d[w];
+    stats[blockIdx.x] = make_float2(M, (float)s);
   }
 }
 
@@ -510,6 +518,7 @@ __global__ __launch_bounds__(kSxThreads) void k_softmax_sum_exact(float2 *__rest
   if (wave == 0 && lane < kSxRows && r0 + lane < rows) stats[r0 + lane] = make_float2(smax[lane], acc[0]);
 }
 
+// The quotients and losses, in the exact mode and for long rows.
 // grid: rows x chunks of kBlock * kSxNormPer logits, the chunks of a row
 // adjacent and laid from the 256-byte boundary of probs at or before the
 // row's start, so that each wavefront's store covers whole lines
@@ -568,6 +577,13 @@ void launch_rows(float *losses, float *probs, const float *logits, const int *ta
                      logits, targets, V);
 }
 
+void launch_norm_rows(float *losses, float *probs, const float *logits, const int *targets, const float2 *stats,
+                      int rows, int V) {
+  const int chunks = (int)grid_for((size_t)V + 63, (size_t)kBlock * kSxNormPer);  // the skew: up to 63
+  launch(k_softmax_norm_rows, dim3((unsigned)((size_t)rows * chunks)), dim3(kBlock), 0, losses, probs, logits, targets,
+         stats, V, chunks);
+}
+
 }  // namespace
 
 // Rows of more than kSplitMaxV logits take the two-pass form, whose row
@@ -592,9 +608,7 @@ int launch_softmax_crossentropy(float *losses, float *probs, const float *logits
                        stream(), stats, logits, rows, V);
     hipLaunchKernelGGL(k_softmax_sum_exact, dim3(grid_for((size_t)rows, kSxRows)), dim3(kSxThreads), 0, stream(),
                        stats, logits, rows, V);
-    const int chunks = (int)grid_for((size_t)V + 63, (size_t)kBlock * kSxNormPer);  // the skew: up to 63
-    hipLaunchKernelGGL(k_softmax_norm_rows, dim3((unsigned)((size_t)rows * chunks)), dim3(kBlock), 0, stream(),
-                       losses, probs, logits, targets, stats, V, chunks);
+    launch_norm_rows(losses, probs, logits, targets, stats, rows, V);
     return check_launch("softmax_crossentropy (exact)");
   }
   // a row takes V + 63 slots at most (the alignment skew)
@@ -614,11 +628,11 @@ int launch_softmax_crossentropy(float *losses, float *probs, const float *logits
     // and a flat normalising pass (12 bytes per logit rather than 8).
     float2 *stats = static_cast<float2 *>(workspace(kRegSoftmax, softmax_scratch(rows, V)));
     if (!stats) return UGK_ENOMEM;
-    hipLaunchKernelGGL(k_softmax_stats, dim3(grid_for((size_t)rows, kStatsWaves)), dim3(kStatsWaves * kWave), 0,
-                       stream(), stats, logits, rows, V);
-    const size_t n = (size_t)rows * V;
-    hipLaunchKernelGGL(k_softmax_norm, dim3(grid_for(n, (size_t)kBlock * kNormUnroll)), dim3(kBlock), 0, stream(),
-                       losses, probs, logits, targets, stats, n, V, 1.0 / (double)V);
+    if (rows >= 1024)
+      launch(k_softmax_stats<256>, dim3(rows), dim3(256), 0, stats, logits, V);
+    else
+      launch(k_softmax_stats<1024>, dim3(rows), dim3(1024), 0, stats, logits, V);
+    launch_norm_rows(losses, probs, logits, targets, stats, rows, V);
   }
   return check_launch("softmax_crossentropy");
 }
