@@ -33,9 +33,8 @@
 // element after another, so that every probability and loss is the CPU's bit
 // for bit (the kernels after the backward's).
 //
-// Backward: dlogits[v] += (probs[v] - (v == target)) * (1 / (B*T)), one
-// workgroup per row streaming float4 (dwords for misaligned arrays);
-// bit-identical to the CPU loop.
+// Backward: dlogits[v] += (probs[v] - (v == target)) * (1 / (B*T)), a flat
+// float4 stream over all rows; bit-identical to the CPU loop.
 #include <atomic>
 #include <type_traits>
 
@@ -336,76 +335,60 @@ __global__ __launch_bounds__(kThreads) void k_softmax_stats(float2 *__restrict__
   }
 }
 
-// Backward over the flat rows x V array, float4 at a time when both arrays
-// start 16-byte aligned (their element offsets agree): each float4 spans at
-// most two rows (V >= 4), so it looks up two targets.
+// Backward over the flat rows x V array, a float4 per thread, at any alignment
+// and length: the slots start at the first element whose address in dlogits is
+// a cache line's, and the elements around them go one by one to a workgroup of
+// their own (as in ugk_map.h). Each float4 spans at most two rows (V >= 4), so
+// it looks up two targets. Memory-bound. Arrays off a 16-byte boundary, and
+// lengths that are no multiple of 4 (any odd number of rows of an odd V), took
+// dwords over a (row, column block) grid before: zeroed, 1,053 rows of 187,239
+// in 385 us, now 242.
 // kZero: dlogits is taken as +0.0 instead of read (callers that zero it before
 // the call); +0.0 + x gives the bits the read of a zero would give.
-constexpr int kBwdThreads = 256, kBwdUnroll = 1;  // measured best: 764 against 846 us with 2 at 8,192 x 50,257
+constexpr int kBwdThreads = 256;  // one float4 per thread measured best: 764 against 846 us with 2 at 8,192 x 50,257
+
+__device__ __forceinline__ float xent_grad(float d, float p, bool hit, float dloss) {
+  return d + (p - (hit ? 1.0f : 0.0f)) * dloss;
+}
+
 template <bool kZero>
 __global__ __launch_bounds__(kBwdThreads) void k_xent_softmax_bwd_flat4(float *__restrict__ dlogits,
                                                                         const float *__restrict__ probs,
                                                                         const int *__restrict__ targets, int rows,
-                                                                        int V, float dloss, size_t n4,
-                                                                        double inv_v) {
-  const float4 *p4 = reinterpret_cast<const float4 *>(probs);
-  float4 *d4 = reinterpret_cast<float4 *>(dlogits);
-  const size_t q0 = (size_t)blockIdx.x * (kBwdThreads * kBwdUnroll) + threadIdx.x;
-  float4 p[kBwdUnroll], d[kBwdUnroll];
-#pragma unroll
-  for (int k = 0; k < kBwdUnroll; k++) {
-    const size_t q = q0 + (size_t)k * kBwdThreads;
-    if (q < n4) {
-      p[k] = ld_nt(p4 + q);
-      d[k] = kZero ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : ld_nt(d4 + q);
+                                                                        int V, float dloss, size_t n4, unsigned full,
+                                                                        unsigned lead, unsigned rest, double inv_v) {
+  if (blockIdx.x == full) {
+    for (unsigned k = threadIdx.x; k < rest; k += kBwdThreads) {
+      const size_t i = k < lead ? k : 4 * n4 + k;
+      const size_t r = row_of(i, (size_t)V, inv_v);
+      dlogits[i] = xent_grad(kZero ? 0.0f : dlogits[i], probs[i], i - r * (size_t)V == (size_t)targets[r], dloss);
     }
+    return;
   }
-#pragma unroll
-  for (int k = 0; k < kBwdUnroll; k++) {
-    const size_t q = q0 + (size_t)k * kBwdThreads;
-    if (q < n4) {
-      const size_t i = 4 * q;
-      const size_t r0 = row_of(i, (size_t)V, inv_v);
-      const size_t t0 = r0 * (size_t)V + (size_t)targets[r0];
-      const size_t t1 = (r0 + 1 < (size_t)rows) ? (r0 + 1) * (size_t)V + (size_t)targets[r0 + 1] : ~(size_t)0;
-      float4 o;
-      o.x = d[k].x + (p[k].x - ((i == t0 || i == t1) ? 1.0f : 0.0f)) * dloss;
-      o.y = d[k].y + (p[k].y - ((i + 1 == t0 || i + 1 == t1) ? 1.0f : 0.0f)) * dloss;
-      o.z = d[k].z + (p[k].z - ((i + 2 == t0 || i + 2 == t1) ? 1.0f : 0.0f)) * dloss;
-      o.w = d[k].w + (p[k].w - ((i + 3 == t0 || i + 3 == t1) ? 1.0f : 0.0f)) * dloss;
-      st_nt(d4 + q, o);
-    }
-  }
+  const size_t q = (size_t)blockIdx.x * kBwdThreads + threadIdx.x;
+  if (q >= n4) return;
+  const size_t i = lead + 4 * q;
+  const float4 p = ld_nt4(probs + i);
+  const float4 d = kZero ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : ld_nt4(dlogits + i);
+  const size_t r0 = row_of(i, (size_t)V, inv_v);
+  const size_t t0 = r0 * (size_t)V + (size_t)targets[r0];
+  const size_t t1 = (r0 + 1 < (size_t)rows) ? (r0 + 1) * (size_t)V + (size_t)targets[r0 + 1] : ~(size_t)0;
+  st_nt4(dlogits + i, make_float4(xent_grad(d.x, p.x, i == t0 || i == t1, dloss),
+                                  xent_grad(d.y, p.y, i + 1 == t0 || i + 1 == t1, dloss),
+                                  xent_grad(d.z, p.z, i + 2 == t0 || i + 2 == t1, dloss),
+                                  xent_grad(d.w, p.w, i + 3 == t0 || i + 3 == t1, dloss)));
 }
 
-// Any alignment: dwords, a (row, column block) grid.
-constexpr int kBwdPer = 4;
+// Rows of fewer than 4 logits: a thread per element.
 template <bool kZero>
 __global__ __launch_bounds__(kBwdThreads) void k_xent_softmax_bwd(float *__restrict__ dlogits,
                                                                   const float *__restrict__ probs,
-                                                                  const int *__restrict__ targets, int V,
+                                                                  const int *__restrict__ targets, int V, size_t n,
                                                                   float dloss) {
-  const size_t row = blockIdx.x;
-  const int tgt = targets[row];
-  const size_t base = row * (size_t)V;
-  const int v0 = blockIdx.y * (kBwdThreads * kBwdPer) + threadIdx.x;
-  float p[kBwdPer], d[kBwdPer];
-#pragma unroll
-  for (int k = 0; k < kBwdPer; k++) {
-    const int v = v0 + k * kBwdThreads;
-    if (v < V) {
-      p[k] = ld_nt(probs + base + v);
-      d[k] = kZero ? 0.0f : ld_nt(dlogits + base + v);
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < kBwdPer; k++) {
-    const int v = v0 + k * kBwdThreads;
-    if (v < V) {
-      const float indicator = (v == tgt) ? 1.0f : 0.0f;
-      st_nt(dlogits + base + v, d[k] + (p[k] - indicator) * dloss);
-    }
-  }
+  const size_t i = (size_t)blockIdx.x * kBwdThreads + threadIdx.x;
+  if (i >= n) return;
+  const size_t r = i / (unsigned)V;
+  dlogits[i] = xent_grad(kZero ? 0.0f : dlogits[i], probs[i], (int)(i - r * (unsigned)V) == targets[r], dloss);
 }
 
 // ---- exact mode: train_bnn.c's order of the row sum ---------------------------
@@ -641,23 +624,21 @@ int launch_crossentropy_softmax_backward(float *dlogits, const float *probs, con
                                          float dloss, bool zeroed) {
   if (rows == 0 || V == 0) return 0;
   const size_t n = (size_t)rows * V;
-  if (V >= 4 && (n & 3) == 0 && aligned16(dlogits) && aligned16(probs)) {
-    const size_t n4 = n / 4;
-    const dim3 grid(grid_for(n4, (size_t)kBwdThreads * kBwdUnroll));
-    if (zeroed)
-      hipLaunchKernelGGL(k_xent_softmax_bwd_flat4<true>, grid, dim3(kBwdThreads), 0, stream(), dlogits, probs, targets,
-                         rows, V, dloss, n4, 1.0 / (double)V);
-    else
-      hipLaunchKernelGGL(k_xent_softmax_bwd_flat4<false>, grid, dim3(kBwdThreads), 0, stream(), dlogits, probs,
-                         targets, rows, V, dloss, n4, 1.0 / (double)V);
+  if (V >= 4) {
+    const size_t lead = (0 - ((uintptr_t)dlogits >> 2)) & 31, first = lead < n ? lead : n, n4 = (n - first) / 4;
+    const unsigned full = grid_for(n4, kBwdThreads), rest = (unsigned)(n - 4 * n4);
+    const auto go = [&](auto k) {
+      launch(k, dim3(full + (rest ? 1 : 0)), dim3(kBwdThreads), 0, dlogits, probs, targets, rows, V, dloss, n4, full,
+             (unsigned)first, rest, 1.0 / (double)V);
+    };
+    if (zeroed) go(k_xent_softmax_bwd_flat4<true>);
+    else go(k_xent_softmax_bwd_flat4<false>);
   } else {
-    const dim3 grid(rows, grid_for((size_t)V, (size_t)kBwdThreads * kBwdPer));
-    if (zeroed)
-      hipLaunchKernelGGL(k_xent_softmax_bwd<true>, grid, dim3(kBwdThreads), 0, stream(), dlogits, probs, targets, V,
-                         dloss);
-    else
-      hipLaunchKernelGGL(k_xent_softmax_bwd<false>, grid, dim3(kBwdThreads), 0, stream(), dlogits, probs, targets, V,
-                         dloss);
+    const auto go = [&](auto k) {
+      launch(k, dim3(grid_for(n, kBwdThreads)), dim3(kBwdThreads), 0, dlogits, probs, targets, V, n, dloss);
+    };
+    if (zeroed) go(k_xent_softmax_bwd<true>);
+    else go(k_xent_softmax_bwd<false>);
   }
   return check_launch("crossentropy_softmax_backward");
 }
