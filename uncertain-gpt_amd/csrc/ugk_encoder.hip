@@ -35,10 +35,11 @@
 //                  added in ascending order, 4 channels per lane, 8 loads in
 //                  flight. The same launch has one more workgroup per
 //                  possible large bucket (K1 lists them with their slots):
-//                  its 256 threads scan the rows' slots in row order, 6,144
+//                  its 256 threads scan the rows' slots in row order, 8,192
 //                  per round, and write the matching row ids, ascending, to a
 //                  list for K3.
-//     K3 large   - workgroups of 16 wavefronts, one per (large bucket, 64
+//     K3 large   - in the exact mode (the default's is k_enc_bwd_blocked)
+//                  workgroups of 16 wavefronts, one per (large bucket, 64
 //                  channels): one wavefront only adds staged rows in order,
 //                  one channel per lane, from one half of a double-buffered
 //                  LDS stage, while three groups of five loader wavefronts
@@ -55,6 +56,7 @@
 //   of calls.
 //   The arrival order inside a bucket depends on scheduling, but it is
 //   discarded: only the set of row ids is used, always in ascending order.
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -161,8 +163,9 @@ __device__ __forceinline__ unsigned hash_slot(int tok, unsigned mask, int shift)
   return ((unsigned)tok * 0x9E3779B1u) >> shift & mask;
 }
 
-// K1: insert the chunk's rows; blocks past the insert range run dwpe.
-template <bool kVec>
+// K1: insert the chunk's rows; blocks past the insert range run dwpe, kB rows
+// of a (t, c) entry in flight.
+template <bool kVec, int kB>
 __global__ __launch_bounds__(kBlock) void k_enc_bwd_insert(EncTable tb, EncShared sh, const int *__restrict__ inp,
                                                            int n, unsigned mask, int shift, int ins_blocks,
                                                            float *dwpe, const float *dout, int B, int T, int C) {
@@ -249,13 +252,15 @@ __global__ __launch_bounds__(kBlock) void k_enc_bwd_insert(EncTable tb, EncShare
     }
     return;
   }
-  // dwpe[t, c] += dout[b, t, c] for b = 0..B-1, in order; 8 rows in flight.
+  // dwpe[t, c] += dout[b, t, c] for b = 0..B-1, in order, kB rows in flight.
   // dout is read with ordinary (cached) loads: K2 reads the same rows again,
   // and finds part of them in the cache (K2 15.8 -> 14.3 us at 8,192 x 768).
   // Each dwpe thread takes two (t, c) entries, one after the other, so half
   // as many dwpe workgroups stream at once and the inserts' round trips are
-  // delayed less (25.6 -> 24.8 us per call at 8,192 x 768).
-  constexpr int kB = 8;
+  // delayed less (25.6 -> 24.8 us per call at 8,192 x 768). Large batches of
+  // short sequences have few entries of many rows: they take one channel per
+  // thread and 32 rows in flight (128 x 64 tokens of 384 channels: 8.7 against
+  // 22.4 us for the launch).
   const size_t pstride = (size_t)(gridDim.x - ins_blocks) * kBlock;
   const size_t n_pe = (size_t)T * (kVec ? C >> 2 : C);
   for (size_t j = (size_t)(blockIdx.x - ins_blocks) * kBlock + threadIdx.x; j < n_pe; j += pstride) {
@@ -301,30 +306,26 @@ __device__ __forceinline__ void wave_lds_sync() {
 }
 
 // K2, scan workgroup of large bucket j: the chunk's row ids whose slot is the
-// bucket's, in row order, to its share of the pool; 6 int4 loads of slots per
-// thread per round (6,144 slots), the round's matches placed by a workgroup
-// prefix over (load, wavefront). Frees the slot after reading its count.
-// (8 loads per round would take K2 from 48 to 58 registers, and from ten
-// wavefronts per SIMD to eight.)
-constexpr int kScanQ = 6;
+// bucket's, in row order, to its share of the pool; 8 int4 loads of slots per
+// thread per round (8,192 slots), the round's matches placed by a workgroup
+// prefix over (load, wavefront). Frees the slot after reading its count. What
+// bounds it is its chain of round trips, so the first round's slots load with
+// the bucket's entry, and its matches are counted while one thread reads the
+// bucket's size and takes its share of the pool (6 int4 per round, all of it
+// one after the other: K2 7.9 us at 8,192 rows of 27 tokens, now 5.3).
+constexpr int kScanQ = 8;
+constexpr int kScanRound = kScanQ * kBlock * 4;
 __device__ __forceinline__ void scan_large(EncTable tb, EncShared sh, int j, int n) {
-  __shared__ int wt[kScanQ][kWavesPerBlock];
+  __shared__ int wt[kScanQ * kWavesPerBlock];
   __shared__ int pool_base, bucket_cnt;
+  constexpr int kCounts = kScanQ * kWavesPerBlock;
+  static_assert(kCounts <= kWave, "one lane per (load, wavefront) count");
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x >> 6;
-  const int4 m = sh.lmeta[j];
-  const int w = m.w;
-  if (threadIdx.x == 0) {
-    const int cnt = slot_cnt(tb.slot[w]);
-    pool_base = atomicAdd(&tb.counters[2], cnt);
-    bucket_cnt = cnt;
-    tb.slot[w] = kFree;
-  }
-  __syncthreads();
-  const int base = pool_base;
   const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (kWave - lane));
+  const int4 m = sh.lmeta[j];
   int run = 0;  // matches in the rounds before this one
-  for (int i0 = 0; i0 < n; i0 += kScanQ * kBlock * 4) {
+  for (int i0 = 0; i0 < n; i0 += kScanRound) {
     int4 sl[kScanQ];
 #pragma unroll
     for (int q = 0; q < kScanQ; q++) {
@@ -338,58 +339,56 @@ __device__ __forceinline__ void scan_large(EncTable tb, EncShared sh, int j, int
         sl[q].w = -1;
       }
     }
+    const int w = m.w;
+    if (i0 == 0 && threadIdx.x == kBlock - 1) {
+      const int cnt = slot_cnt(tb.slot[w]);
+      pool_base = atomicAdd(&tb.counters[2], cnt);
+      bucket_cnt = cnt;
+      tb.slot[w] = kFree;
+    }
 #pragma unroll
     for (int q = 0; q < kScanQ; q++) {
       const int k = __popcll(__ballot(sl[q].x == w)) + __popcll(__ballot(sl[q].y == w)) +
                     __popcll(__ballot(sl[q].z == w)) + __popcll(__ballot(sl[q].w == w));
-      if (lane == 0) wt[q][wave] = k;
+      if (lane == 0) wt[q * kWavesPerBlock + wave] = k;
     }
     __syncthreads();
-    // slots are ordered by (load q, wavefront, lane, element): the matches of
-    // the (q, wavefront) pairs before this one come first
-    int off = run;
+    // slots are ordered by (load q, wavefront, lane, element): lane 4 q + v
+    // gets the matches up to (q, v)
+    const int own = lane < kCounts ? wt[lane] : 0;
+    int incl = own;
+#pragma unroll
+    for (int d = 1; d < kCounts; d <<= 1) {
+      const int t = __shfl_up(incl, d);
+      if (lane >= d) incl += t;
+    }
+    int *const out = sh.pool + pool_base + run;
+#pragma unroll
     for (int q = 0; q < kScanQ; q++) {
-      int o = off;
-#pragma unroll
-      for (int v = 0; v < kWavesPerBlock; v++) o += v < wave ? wt[q][v] : 0;
-#pragma unroll
-      for (int v = 0; v < kWavesPerBlock; v++) off += wt[q][v];
       const int e = i0 + (q * kBlock + (int)threadIdx.x) * 4;
+      int o = __shfl(incl - own, q * kWavesPerBlock + wave);
       o += __popcll(__ballot(sl[q].x == w) & below) + __popcll(__ballot(sl[q].y == w) & below) +
            __popcll(__ballot(sl[q].z == w) & below) + __popcll(__ballot(sl[q].w == w) & below);
-      if (sl[q].x == w) sh.pool[base + o++] = e;
-      if (sl[q].y == w) sh.pool[base + o++] = e + 1;
-      if (sl[q].z == w) sh.pool[base + o++] = e + 2;
-      if (sl[q].w == w) sh.pool[base + o] = e + 3;
+      if (sl[q].x == w) out[o++] = e;
+      if (sl[q].y == w) out[o++] = e + 1;
+      if (sl[q].z == w) out[o++] = e + 2;
+      if (sl[q].w == w) out[o] = e + 3;
     }
-    run = off;
+    run += __shfl(incl, kCounts - 1);
     __syncthreads();  // wt is rewritten by the next round
   }
-  if (threadIdx.x == 0) sh.lmeta[j] = make_int4(base, bucket_cnt, m.z, w);
+  if (threadIdx.x == 0) sh.lmeta[j] = make_int4(pool_base, bucket_cnt, m.z, m.w);
 }
 
-// K2: one scan workgroup per possible large bucket in the first nscan
-// workgroups (dispatched first, so that those with no bucket have left before
-// the adds end), then one wavefront per slot-list entry (covering K1's
-// regions exactly). A small bucket's wavefront frees its slot once it has
-// read it.
+// A wavefront's slot-list entry (wavefront gw of R regions of kBlock entries):
+// a bucket of at most kCap rows is added, and its slot freed. mine: kCap words of LDS of the wavefront's own.
 template <bool kVec>
-__global__ __launch_bounds__(kBlock) void k_enc_bwd_add(EncTable tb, EncShared sh, float *__restrict__ dwte,
-                                                        const float *__restrict__ dout, int C, int n, int nscan) {
-  __shared__ unsigned lds[kWavesPerBlock * kCap];
-  if ((int)blockIdx.x < nscan) {
-    const int j = (int)blockIdx.x;
-    if (j < tb.counters[1]) scan_large(tb, sh, j, n);  // K1 has counted them: the same value in every thread
-    return;
-  }
+__device__ __forceinline__ void add_small(EncTable tb, EncShared sh, float *__restrict__ dwte,
+                                          const float *__restrict__ dout, int C, int gw, int R, unsigned *mine) {
   const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x >> 6;
-  unsigned *mine = lds + (size_t)wave * kCap;
   // Wavefront g takes entry g / R of region g % R (R regions of kBlock
   // entries): the entries of one region (one K1 workgroup's tokens, where a
   // skewed batch puts its frequent tokens early) spread over all workgroups.
-  const int R = ((int)gridDim.x - nscan) * kWavesPerBlock / kBlock;
-  const int gw = ((int)blockIdx.x - nscan) * kWavesPerBlock + wave;
   const int w = sh.list[(gw % R) * kBlock + gw / R];  // this wavefront's slot
   if (w < 0) return;
   // the slot word and the bucket's first row ids in one round trip (ids past
@@ -445,28 +444,46 @@ __global__ __launch_bounds__(kBlock) void k_enc_bwd_add(EncTable tb, EncShared s
   for (int j = 0; j < cnt; j++) rank += (__shfl(id, j) < id) ? 1 : 0;
   if (lane < cnt) mine[rank] = (unsigned)id;
   wave_lds_sync();
-  // rows in ascending order, kBatch loads in flight before their adds
-  constexpr int kBatch = 8;
+  // rows in ascending order, up to kBatch rows of three float4 per lane in
+  // flight before their adds (one float4 and eight rows at a time, three times
+  // the round trips for small buckets: K2 17.7 us at 16,384 Zipf rows x 768, now
+  // 14.5 with the scan's part)
+  constexpr int kCols = 3;
   if (kVec) {
+    constexpr int kBatch = 4;
     const int C4 = C >> 2;
     float4 *row = reinterpret_cast<float4 *>(dwte) + (size_t)tok * C4;
     const float4 *g = reinterpret_cast<const float4 *>(dout);
-    for (int c4 = lane; c4 < C4; c4 += kWave) {
-      float4 acc = row[c4];
-      for (int q0 = 0; q0 < cnt; q0 += kBatch) {
-        float4 d[kBatch];
+    for (int c0 = lane; c0 < C4; c0 += kCols * kWave) {
+      float4 acc[kCols];
 #pragma unroll
-        for (int q = 0; q < kBatch; q++)
-          if (q0 + q < cnt) d[q] = ld_nt(g + (size_t)mine[q0 + q] * C4 + c4);
+      for (int u = 0; u < kCols; u++)
+        if (c0 + u * kWave < C4) acc[u] = row[c0 + u * kWave];
+      for (int q0 = 0; q0 < cnt; q0 += kBatch) {
+        float4 d[kBatch][kCols];
 #pragma unroll
         for (int q = 0; q < kBatch; q++)
           if (q0 + q < cnt) {
-            acc.x += d[q].x; acc.y += d[q].y; acc.z += d[q].z; acc.w += d[q].w;
+            const float4 *gr = g + (size_t)mine[q0 + q] * C4 + c0;
+#pragma unroll
+            for (int u = 0; u < kCols; u++)
+              if (c0 + u * kWave < C4) d[q][u] = ld_nt(gr + u * kWave);
+          }
+#pragma unroll
+        for (int q = 0; q < kBatch; q++)
+          if (q0 + q < cnt) {
+#pragma unroll
+            for (int u = 0; u < kCols; u++) {
+              acc[u].x += d[q][u].x; acc[u].y += d[q][u].y; acc[u].z += d[q][u].z; acc[u].w += d[q][u].w;
+            }
           }
       }
-      row[c4] = acc;
+#pragma unroll
+      for (int u = 0; u < kCols; u++)
+        if (c0 + u * kWave < C4) row[c0 + u * kWave] = acc[u];
     }
   } else {
+    constexpr int kBatch = 8;
     float *row = dwte + (size_t)tok * C;
     for (int c = lane; c < C; c += kWave) {
       float acc = row[c];
@@ -482,6 +499,26 @@ __global__ __launch_bounds__(kBlock) void k_enc_bwd_add(EncTable tb, EncShared s
       row[c] = acc;
     }
   }
+}
+
+// K2: one scan workgroup per possible large bucket in the first nscan
+// workgroups (dispatched first, so that those with no bucket have left before
+// the adds end), then one wavefront per slot-list entry (covering K1's
+// regions exactly). A small bucket's wavefront frees its slot once it has
+// read it.
+template <bool kVec>
+__global__ __launch_bounds__(kBlock, 6) void k_enc_bwd_add(EncTable tb, EncShared sh, float *__restrict__ dwte,
+                                                        const float *__restrict__ dout, int C, int n, int nscan) {
+  __shared__ unsigned lds[kWavesPerBlock * kCap];
+  if ((int)blockIdx.x < nscan) {
+    const int j = (int)blockIdx.x;
+    if (j < tb.counters[1]) scan_large(tb, sh, j, n);  // K1 has counted them: the same value in every thread
+    return;
+  }
+  const int wave = threadIdx.x >> 6;
+  const int R = ((int)gridDim.x - nscan) * kWavesPerBlock / kBlock;
+  add_small<kVec>(tb, sh, dwte, dout, C, ((int)blockIdx.x - nscan) * kWavesPerBlock + wave, R,
+                         lds + (size_t)wave * kCap);
 }
 
 // K3: workgroups take (large bucket, 64-channel slice) work items from a
@@ -638,87 +675,154 @@ __global__ __launch_bounds__(kLargeThreads) void k_enc_bwd_large(EncTable tb, En
   }
 }
 
-// K3, blocked mode (the default): the same (large bucket, 64-channel slice)
-// work items as k_enc_bwd_large, but the bucket's rows, ascending, are cut
-// into blocks of kBlkRows, and the workgroup's 16 wavefronts add blocks
-// w, w + 16, ... in parallel, each block's rows in row order, all its 64
-// rows' loads in flight at once (one float per lane) and the next block's
-// row ids loaded meanwhile. The first block starts from dwte's value, the
-// others from -0.0f (the identity of IEEE addition); the block sums go to
-// LDS, and wavefront 0 adds them in block order:
+// K3, blocked mode (the default): (large bucket, channel slice) work items,
+// taken as k_enc_bwd_large takes its own. The bucket's rows, ascending, are cut
+// into blocks of kBlkRows, and the workgroup's wavefronts add blocks in
+// parallel, each block's rows in row order, one channel per lane, all its 64
+// rows' loads in flight at once. The first block starts from dwte's value, the
+// others from -0.0f (the identity of IEEE addition); the block sums go to LDS,
+// and wavefront 0 adds them in block order:
 //   s_0 = ((dwte + d_0) + d_1) + ... + d_63,  s_k = d_64k + ... + d_64k+63,
 //   dwte = ((s_0 + s_1) + s_2) + ...
 // in rounds of at most kLdsBlocks blocks. The same inputs give the same bits
 // on every run, and a bucket of at most 64 rows gets the CPU's order. A
-// bucket of 2,348 rows is 37 blocks, at most three per wavefront, instead of
-// a chain of 2,348 dependent adds. No state crosses workgroups: the counters
-// and their reset are k_enc_bwd_large's.
+// bucket of 2,348 rows is 37 blocks instead of a chain of 2,348 dependent
+// adds. No state crosses workgroups: the counters and their reset are
+// k_enc_bwd_large's.
+// What bounds it: a frequent token's rows through the few CUs that hold its
+// items (about 60 GB/s each; with 8 wavefronts instead of 16 the kernel takes
+// nearly twice the time). So a bucket of more than kHalfRows rows is cut into
+// slices of 32 channels, a wavefront adding two blocks at a time, one per half
+// (kG = 2), the others into slices of 64 (kG = 1): 8,192 rows of 27 tokens x 384
+// take 11.0 us against 12.6 with 64 channels throughout; 16,384 Zipf rows x 768,
+// whose many smaller buckets fill the chip, 16.6 against 16.0 with the line at
+// 512 rows.
 constexpr int kBlkRows = 64;
-constexpr int kBlockedWaves = 16;
+constexpr int kBlkWaves = 16;
 constexpr int kLdsBlocks = 256;
+constexpr int kHalfRows = 1024;
 
-__device__ __forceinline__ void blocked_items(EncTable tb, EncShared sh, float *__restrict__ dwte,
-                                              const float *__restrict__ dout, int C, int nslices, int total,
-                                              float (*bs)[kWave], int *next_item_p) {
-  int &next_item = *next_item_p;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x >> 6;
-  for (int first = 1;; first = 0) {
-    // a workgroup's first item is its own index, later ones come from the counter
-    if (threadIdx.x == 0) next_item = first ? (int)blockIdx.x : (int)gridDim.x + atomicAdd(&tb.counters[0], 1);
-    __syncthreads();
-    const int wi = next_item;
-    __syncthreads();
-    if (wi >= total) break;
-    const int j = wi / nslices;
-    const int c = (wi % nslices) * kWave + lane;
-    const bool on = c < C;
-    const int cc = on ? c : 0;  // a valid column for the lanes past C, never stored
-    const int4 m = sh.lmeta[j];
-    const int *ids = sh.pool + m.x;
-    const int cnt = m.y;
-    const size_t trow = (size_t)m.z * C + cc;
-    const int nb = (cnt + kBlkRows - 1) / kBlkRows;
-    float t = -0.0f;  // wavefront 0's running total of the block sums
-    for (int r0 = 0; r0 < nb; r0 += kLdsBlocks) {
-      const int r1 = min(nb, r0 + kLdsBlocks);
-      int k = r0 + wave;
-      int id = k < r1 ? ids[k * kBlkRows + min(lane, cnt - k * kBlkRows - 1)] : 0;
-      for (; k < r1; k += kBlockedWaves) {
-        const int nr = min(kBlkRows, cnt - k * kBlkRows);
-        float v[kBlkRows];
+struct BlockedLds {
+  float bs[kLdsBlocks][kWave];
+  unsigned short half[kMaxLarge], whole[kMaxLarge];  // the buckets by slice width
+  int next_item, nhalf, nwhole;
+};
+
+// One item: the bucket m's rows in the 64 / kG channels of slice sl. Offsets of
+// rows are 32-bit unless kFar.
+template <int kG, bool kFar>
+__device__ __forceinline__ void blocked_item(BlockedLds &L, const int *__restrict__ ids, int cnt, float *__restrict__ dtok,
+                                             const float *__restrict__ dout, int C, int sl) {
+  constexpr int kCols = kWave / kG;
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6, half = lane / kCols;
+  const int c = sl * kCols + lane % kCols;
+  const bool on = c < C;
+  const unsigned cc = on ? (unsigned)c : 0u;  // a valid column for the lanes past C, never stored
+  const int nb = (cnt + kBlkRows - 1) / kBlkRows;
+  const float base = wave == 0 ? dtok[cc] : -0.0f;
+  float t = -0.0f;  // wavefront 0's running total of the block sums
+  for (int r0 = 0; r0 < nb; r0 += kLdsBlocks) {
+    const int r1 = min(nb, r0 + kLdsBlocks);
+    for (int k0 = r0 + kG * wave; k0 < r1; k0 += kG * kBlkWaves) {
+      // row offsets of the blocks k0 (.. k0 + kG - 1), one row per lane; past a
+      // block's rows its last one, past the last block that block's
+      unsigned at[kG];
+      int nrow[kG], id[kG];
 #pragma unroll
-        for (int q = 0; q < kBlkRows; q++) v[q] = dout[(size_t)__builtin_amdgcn_readlane(id, min(q, nr - 1)) * C + cc];
-        const int kn = k + kBlockedWaves;  // the next block's row ids, loaded while these rows arrive
-        if (kn < r1) id = ids[kn * kBlkRows + min(lane, cnt - kn * kBlkRows - 1)];
-        float a = k == 0 ? dwte[trow] : -0.0f;
+      for (int g = 0; g < kG; g++) {
+        const int k = min(k0 + g, r1 - 1);
+        nrow[g] = min(kBlkRows, cnt - k * kBlkRows);
+        id[g] = ids[k * kBlkRows + min(lane, nrow[g] - 1)];
+        at[g] = (unsigned)id[g] * (unsigned)C;
+      }
+      const int nr = kG == 1 || half == 0 ? nrow[0] : k0 + 1 < r1 ? nrow[kG - 1] : 0;
+      float v[kBlkRows];
+#pragma unroll
+      for (int q = 0; q < kBlkRows; q++) {
+        if (kG == 1) {
+          v[q] = (dout + (size_t)(unsigned)__builtin_amdgcn_readlane(id[0], q) * C)[cc];
+        } else if (kFar) {
+          const int r0q = __builtin_amdgcn_readlane(id[0], q), r1q = __builtin_amdgcn_readlane(id[kG - 1], q);
+          v[q] = dout[(size_t)(unsigned)(half ? r1q : r0q) * C + cc];
+        } else {
+          const unsigned o0 = __builtin_amdgcn_readlane(at[0], q), o1 = __builtin_amdgcn_readlane(at[kG - 1], q);
+          v[q] = dout[(half ? o1 : o0) + cc];
+        }
+      }
+      float a = k0 == 0 && half == 0 ? base : -0.0f;
+      if (kG == 1) {
 #pragma unroll
         for (int q = 0; q < kBlkRows; q++)
-          if (q < nr) a += v[q];  // the same for the whole wavefront
-        bs[k - r0][lane] = a;
+          if (q < nrow[0]) a += v[q];  // the same for the whole wavefront
+      } else {
+#pragma unroll
+        for (int q = 0; q < kBlkRows; q++) a += q < nr ? v[q] : -0.0f;
       }
-      __syncthreads();
-      if (wave == 0)
-        for (int q = 0; q < r1 - r0; q++) t += bs[q][lane];
-      __syncthreads();  // bs is rewritten by the next round
+      if (k0 + half < r1) L.bs[k0 + half - r0][lane % kCols] = a;
     }
-    if (wave == 0 && on) dwte[trow] = t;
+    __syncthreads();
+    if (wave == 0) {
+      int q = 0;
+      for (; q + 8 <= r1 - r0; q += 8) {
+        float b[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) b[i] = L.bs[q + i][lane % kCols];
+#pragma unroll
+        for (int i = 0; i < 8; i++) t += b[i];
+      }
+      for (; q < r1 - r0; q++) t += L.bs[q][lane % kCols];
+    }
+    if (r1 < nb) __syncthreads();  // bs is rewritten by the next round
   }
+  if (wave == 0 && half == 0 && on) dtok[c] = t;
 }
 
-__global__ __launch_bounds__(kBlockedWaves * kWave) void k_enc_bwd_blocked(EncTable tb, EncShared sh,
-                                                                           float *__restrict__ dwte,
-                                                                           const float *__restrict__ dout, int C,
-                                                                           int nslices) {
-  __shared__ float bs[kLdsBlocks][kWave];
-  __shared__ int next_item;
+template <bool kFar>
+__global__ __launch_bounds__(kBlkWaves * kWave) void k_enc_bwd_blocked(EncTable tb, EncShared sh,
+                                                                       float *__restrict__ dwte,
+                                                                       const float *__restrict__ dout, int C) {
+  __shared__ BlockedLds L;
+  const int grid = (int)gridDim.x, lane = threadIdx.x & (kWave - 1);
   // As k_enc_bwd_large: with no large bucket every counter is still zero;
   // otherwise the last workgroup to arrive resets them after all their reads.
-  const int total = tb.counters[1] * nslices;
-  if (total == 0) return;
-  blocked_items(tb, sh, dwte, dout, C, nslices, total, bs, &next_item);
+  const int count = tb.counters[1];
+  if (count == 0) return;
+  if (threadIdx.x < kWave) {  // the buckets by slice width, each in list order
+    int nh = 0;
+    for (int j0 = 0; j0 < count; j0 += kWave) {
+      const int j = j0 + lane;
+      const bool h = j < count && sh.lmeta[j].y > kHalfRows;
+      const u64 mk = __ballot(h), below = (lane == 0) ? 0ull : (~0ull >> (kWave - lane));
+      const int hb = nh + __popcll(mk & below);
+      if (h) L.half[hb] = (unsigned short)j;
+      else if (j < count) L.whole[j - hb] = (unsigned short)j;
+      nh += __popcll(mk);
+    }
+    if (lane == 0) {
+      L.nhalf = nh;
+      L.nwhole = count - nh;
+    }
+  }
   __syncthreads();
-  if (threadIdx.x == 0 && atomicAdd(&tb.counters[3], 1) == (int)gridDim.x - 1) {
+  const int s2 = (C + kWave / 2 - 1) / (kWave / 2), s1 = (C + kWave - 1) / kWave;
+  const int first1 = L.nhalf * s2, total = first1 + L.nwhole * s1;
+  // a workgroup's first item is its own index, later ones come from the counter
+  for (int wi = (int)blockIdx.x; wi < total;) {
+    const bool h = wi < first1;
+    const int i = h ? wi : wi - first1, j = h ? L.half[i / s2] : L.whole[i / s1];
+    const int4 m = sh.lmeta[j];
+    float *const dtok = dwte + (size_t)m.z * C;
+    if (h)
+      blocked_item<2, kFar>(L, sh.pool + m.x, m.y, dtok, dout, C, i % s2);
+    else
+      blocked_item<1, kFar>(L, sh.pool + m.x, m.y, dtok, dout, C, i % s1);
+    if (total <= grid) break;  // the first items were all
+    if (threadIdx.x == 0) L.next_item = grid + atomicAdd(&tb.counters[0], 1);
+    __syncthreads();
+    wi = L.next_item;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0 && atomicAdd(&tb.counters[3], 1) == grid - 1) {
     tb.counters[0] = 0;
     tb.counters[1] = 0;
     tb.counters[2] = 0;
@@ -889,36 +993,46 @@ int launch_encoder_backward(float *dwte, float *dwpe, const float *dout, const i
     const unsigned mask = (unsigned)tsize - 1u;
     const int shift = 32 - lg;
     const int ins_blocks = (int)grid_for((size_t)n, kBlock);
+    // dwpe, in the first chunk's launch: two float4 entries per thread, or one
+    // entry of one channel where each has many rows
+    const bool deep = B > 16;
     int pe_blocks = 0;
-    if (c0 == 0) pe_blocks = ((int)grid_for((size_t)T * (vec ? C / 4 : C), kBlock) + 1) / 2;
-    if (vec)
-      hipLaunchKernelGGL(k_enc_bwd_insert<true>, dim3(ins_blocks + pe_blocks), dim3(kBlock), 0, stream(), tb,
-                         sh, inp + c0, n, mask, shift, ins_blocks, dwpe, dout, B, T, C);
-    else
-      hipLaunchKernelGGL(k_enc_bwd_insert<false>, dim3(ins_blocks + pe_blocks), dim3(kBlock), 0, stream(), tb,
-                         sh, inp + c0, n, mask, shift, ins_blocks, dwpe, dout, B, T, C);
+    if (c0 == 0)
+      pe_blocks = deep ? (int)grid_for((size_t)T * C, kBlock)
+                       : ((int)grid_for((size_t)T * (vec ? C / 4 : C), kBlock) + 1) / 2;
+    const auto insert = [&](auto k) {
+      launch(k, dim3(ins_blocks + pe_blocks), dim3(kBlock), 0, tb, sh, inp + c0, n, mask, shift, ins_blocks, dwpe, dout,
+             B, T, C);
+    };
+    if (deep) insert(k_enc_bwd_insert<false, 32>);
+    else if (vec) insert(k_enc_bwd_insert<true, 8>);
+    else insert(k_enc_bwd_insert<false, 8>);
     const float *dchunk = dout + (size_t)c0 * C;
     // one workgroup per possible large bucket (at most n / (kCap + 1)), then
     // one wavefront per entry of K1's slot-list regions
     const int nscan = n / (kCap + 1) + 1;
     const dim3 g2((unsigned)(nscan + ins_blocks * (kBlock / kWavesPerBlock)));
     if (vec)
-      hipLaunchKernelGGL(k_enc_bwd_add<true>, g2, dim3(kBlock), 0, stream(), tb, sh, dwte, dchunk, C, n, nscan);
+      launch(k_enc_bwd_add<true>, g2, dim3(kBlock), 0, tb, sh, dwte, dchunk, C, n, nscan);
     else
-      hipLaunchKernelGGL(k_enc_bwd_add<false>, g2, dim3(kBlock), 0, stream(), tb, sh, dwte, dchunk, C, n, nscan);
-    const int max_items = (n / (kCap + 1) + 1) * nslices;
-    const dim3 g3(max_items < kLargeGrid ? max_items : kLargeGrid);
+      launch(k_enc_bwd_add<false>, g2, dim3(kBlock), 0, tb, sh, dwte, dchunk, C, n, nscan);
+    const auto grid_of = [&](int slices, int most) { return std::min((n / (kCap + 1) + 1) * slices, most); };
     if (blocked) {
-      // the same work items, each bucket's blocks spread over the workgroup's
-      // wavefronts; with no large bucket every workgroup returns at once
-      hipLaunchKernelGGL(k_enc_bwd_blocked, g3, dim3(kBlockedWaves * kWave), 0, stream(), tb, sh, dwte, dchunk, C,
-                         nslices);
+      // each bucket's blocks spread over half wavefronts; with no large bucket
+      // every workgroup returns at once
+      // (a bucket's slices of 32 channels are within twice the count of 64)
+      const dim3 g3(grid_of(2 * nslices, kLargeGrid)), block(kBlkWaves * kWave);
+      if ((size_t)n * C > ((size_t)1 << 30))
+        launch(k_enc_bwd_blocked<true>, g3, block, 0, tb, sh, dwte, dchunk, C);
+      else
+        launch(k_enc_bwd_blocked<false>, g3, block, 0, tb, sh, dwte, dchunk, C);
       continue;
     }
     // one round of workgroups (one per CU: each stages 122 KB in LDS) takes
     // the (large bucket, channel slice) work items; with no large bucket
     // every workgroup goes straight to the counter reset
-    hipLaunchKernelGGL(k_enc_bwd_large, g3, dim3(kLargeThreads), 0, stream(), tb, sh, dwte, dchunk, C, nslices);
+    launch(k_enc_bwd_large, dim3(grid_of(nslices, kLargeGrid)), dim3(kLargeThreads), 0, tb, sh, dwte, dchunk, C,
+           nslices);
   }
   return check_launch("encoder_backward");
 }
