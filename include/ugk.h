@@ -353,6 +353,27 @@ int ugk_synchronize(void);
 #define UGK_IDS_SOFTMAX_CROSSENTROPY 4
 #define UGK_IDS_CROSSENTROPY_BACKWARD 5
 int ugk_ids_guard(int *ids, int n, int bound, int fill, int code);
+/* The ops that index a table by ids with that check inside their own kernels:
+ * ugk_ids_guard over the B*T ids (bound V, the fill and code of the op; fill -1
+ * for the encoder backward, else 0) and then the op, without the guard's
+ * launch. V > 0: the rows of wte for the encoder ops, the logits per row for
+ * the others. `zeroed` as ugk_crossentropy_softmax_backward_zeroed. */
+int ugk_encoder_forward_checked(float *out, int *inp, const float *wte,
+                                const float *wpe, int B, int T, int C, int V);
+int ugk_encoder_backward_checked(float *dwte, float *dwpe, const float *dout,
+                                 int *inp, int B, int T, int C, int V);
+int ugk_encoder_layernorm_forward_checked(float *enc, float *out, float *mean,
+                                          float *rstd, int *inp,
+                                          const float *wte, const float *wpe,
+                                          const float *weight,
+                                          const float *bias, int B, int T,
+                                          int C, int V);
+int ugk_softmax_crossentropy_checked(float *losses, float *probs,
+                                     const float *logits, int *targets, int B,
+                                     int T, int V);
+int ugk_crossentropy_softmax_backward_checked(float *dlogits,
+                                              const float *probs, int *targets,
+                                              int B, int T, int V, int zeroed);
 /* Library version, major*10000 + minor*100 + patch. */
 int ugk_version(void);
 

@@ -238,26 +238,96 @@ bool any_same(std::initializer_list<const void *> ps) {
 
 }  // namespace
 
+// The ops that index a table by ids, without the check of the ids (ids.word
+// null; they are then only read) or with it.
+namespace {
+int *unchecked(const int *ids) { return const_cast<int *>(ids); }
+
+// *ids for a table of V rows.
+int id_check(const char *fn, int V, int fill, int code, IdCheck *ids) {
+  if (V <= 0) return bad(fn, "V must be > 0 (the ids index a table of V rows)");
+  int *word = ids_error_word();
+  if (!word) return UGK_EHIP;
+  *ids = IdCheck{(unsigned)V - 1u, fill, code, word};
+  return UGK_OK;
+}
+
+int encoder_forward(const char *fn, float *out, int *inp, const float *wte, const float *wpe, int B, int T, int C,
+                    const IdCheck &ids) {
+  if (int e = check_btc(fn, B, T, C)) return e;
+  if ((long long)B * T * C == 0) return ok();
+  if (any_null({out, inp, wte, wpe})) return bad(fn, "NULL pointer");
+  if (int e = launch_encoder_forward(out, inp, wte, wpe, B, T, C, ids)) return e;
+  return ok();
+}
+
+int encoder_backward(const char *fn, float *dwte, float *dwpe, const float *dout, int *inp, int B, int T, int C,
+                     const IdCheck &ids) {
+  if (int e = check_btc(fn, B, T, C)) return e;
+  if ((long long)B * T * C == 0) return ok();
+  if (any_null({dwte, dwpe, dout, inp})) return bad(fn, "NULL pointer");
+  if (int e = launch_encoder_backward(dwte, dwpe, dout, inp, B, T, C, ids)) return e;
+  return ok();
+}
+
+int encoder_layernorm_forward(const char *fn, float *enc, float *out, float *mean, float *rstd, int *inp,
+                              const float *wte, const float *wpe, const float *weight, const float *bias, int B, int T,
+                              int C, const IdCheck &ids) {
+  if (int e = check_btc(fn, B, T, C)) return e;
+  if ((long long)B * T == 0) return ok();
+  if (C == 0) return bad(fn, "C must be > 0 when B*T > 0 (mean over an empty row)");
+  if (any_null({enc, out, mean, rstd, inp, wte, wpe, weight, bias})) return bad(fn, "NULL pointer");
+  if (int e = launch_encoder_layernorm_forward(enc, out, mean, rstd, inp, wte, wpe, weight, bias, B, T, C, ids))
+    return e;
+  return ok();
+}
+
+int softmax_crossentropy(const char *fn, float *losses, float *probs, const float *logits, int *targets, int B, int T,
+                         int V, const IdCheck &ids) {
+  if (int e = check_btc(fn, B, T, V)) return e;
+  if ((long long)B * T == 0) return ok();
+  if (V == 0) return bad(fn, "V must be > 0 when B*T > 0 (the target indexes the row)");
+  if (any_null({losses, probs, logits, targets})) return bad(fn, "NULL pointer");
+  if ((const void *)probs == (const void *)logits) return bad(fn, "probs and logits must be distinct buffers");
+  if (int e = launch_softmax_crossentropy(losses, probs, logits, targets, B * T, V, ids)) return e;
+  return ok();
+}
+
+int xent_backward(const char *fn, bool zeroed, float *dlogits, const float *probs, int *targets, int B, int T, int V,
+                  const IdCheck &ids) {
+  if (int e = check_btc(fn, B, T, V)) return e;
+  if ((long long)B * T * V == 0) return ok();
+  if (any_null({dlogits, probs, targets})) return bad(fn, "NULL pointer");
+  const float dloss = 1.0f / (B * T);  // train_bnn.c:360
+  if (int e = launch_crossentropy_softmax_backward(dlogits, probs, targets, B * T, V, dloss, zeroed, ids)) return e;
+  return ok();
+}
+}  // namespace
+
 extern "C" {
 
 int ugk_encoder_forward(float *out, const int *inp, const float *wte, const float *wpe, int B, int T,
                         int C) {
-  const char *fn = "ugk_encoder_forward";
-  if (int e = check_btc(fn, B, T, C)) return e;
-  if ((long long)B * T * C == 0) return ok();
-  if (any_null({out, inp, wte, wpe})) return bad(fn, "NULL pointer");
-  if (int e = launch_encoder_forward(out, inp, wte, wpe, B, T, C)) return e;
-  return ok();
+  return encoder_forward("ugk_encoder_forward", out, unchecked(inp), wte, wpe, B, T, C, {});
+}
+
+int ugk_encoder_forward_checked(float *out, int *inp, const float *wte, const float *wpe, int B, int T, int C, int V) {
+  const char *fn = "ugk_encoder_forward_checked";
+  IdCheck ids;
+  if (int e = id_check(fn, V, 0, UGK_IDS_ENCODER_FORWARD, &ids)) return e;
+  return encoder_forward(fn, out, inp, wte, wpe, B, T, C, ids);
 }
 
 int ugk_encoder_backward(float *dwte, float *dwpe, const float *dout, const int *inp, int B, int T,
                          int C) {
-  const char *fn = "ugk_encoder_backward";
-  if (int e = check_btc(fn, B, T, C)) return e;
-  if ((long long)B * T * C == 0) return ok();
-  if (any_null({dwte, dwpe, dout, inp})) return bad(fn, "NULL pointer");
-  if (int e = launch_encoder_backward(dwte, dwpe, dout, inp, B, T, C)) return e;
-  return ok();
+  return encoder_backward("ugk_encoder_backward", dwte, dwpe, dout, unchecked(inp), B, T, C, {});
+}
+
+int ugk_encoder_backward_checked(float *dwte, float *dwpe, const float *dout, int *inp, int B, int T, int C, int V) {
+  const char *fn = "ugk_encoder_backward_checked";
+  IdCheck ids;
+  if (int e = id_check(fn, V, -1, UGK_IDS_ENCODER_BACKWARD, &ids)) return e;
+  return encoder_backward(fn, dwte, dwpe, dout, inp, B, T, C, ids);
 }
 
 int ugk_layernorm_forward(float *out, float *mean, float *rstd, const float *inp, const float *weight,
@@ -304,14 +374,17 @@ int ugk_layernorm_backward_noalloc(float *dinp, float *dweight, float *dbias, co
 int ugk_encoder_layernorm_forward(float *enc, float *out, float *mean, float *rstd, const int *inp,
                                   const float *wte, const float *wpe, const float *weight, const float *bias, int B,
                                   int T, int C) {
-  const char *fn = "ugk_encoder_layernorm_forward";
-  if (int e = check_btc(fn, B, T, C)) return e;
-  if ((long long)B * T == 0) return ok();
-  if (C == 0) return bad(fn, "C must be > 0 when B*T > 0 (mean over an empty row)");
-  if (any_null({enc, out, mean, rstd, inp, wte, wpe, weight, bias})) return bad(fn, "NULL pointer");
-  if (int e = launch_encoder_layernorm_forward(enc, out, mean, rstd, inp, wte, wpe, weight, bias, B, T, C))
-    return e;
-  return ok();
+  return encoder_layernorm_forward("ugk_encoder_layernorm_forward", enc, out, mean, rstd, unchecked(inp), wte, wpe,
+                                   weight, bias, B, T, C, {});
+}
+
+int ugk_encoder_layernorm_forward_checked(float *enc, float *out, float *mean, float *rstd, int *inp, const float *wte,
+                                          const float *wpe, const float *weight, const float *bias, int B, int T,
+                                          int C, int V) {
+  const char *fn = "ugk_encoder_layernorm_forward_checked";
+  IdCheck ids;
+  if (int e = id_check(fn, V, 0, UGK_IDS_ENCODER_LAYERNORM_FORWARD, &ids)) return e;
+  return encoder_layernorm_forward(fn, enc, out, mean, rstd, inp, wte, wpe, weight, bias, B, T, C, ids);
 }
 
 int ugk_residual_layernorm_forward(float *res, float *out, float *mean, float *rstd, const float *x,
@@ -386,35 +459,32 @@ int ugk_bayes_materialize(float *w, const float *mu, const float *rho, const flo
 
 int ugk_softmax_crossentropy(float *losses, float *probs, const float *logits, const int *targets, int B, int T,
                              int V) {
-  const char *fn = "ugk_softmax_crossentropy";
-  if (int e = check_btc(fn, B, T, V)) return e;
-  if ((long long)B * T == 0) return ok();
-  if (V == 0) return bad(fn, "V must be > 0 when B*T > 0 (the target indexes the row)");
-  if (any_null({losses, probs, logits, targets})) return bad(fn, "NULL pointer");
-  if ((const void *)probs == (const void *)logits) return bad(fn, "probs and logits must be distinct buffers");
-  if (int e = launch_softmax_crossentropy(losses, probs, logits, targets, B * T, V)) return e;
-  return ok();
+  return softmax_crossentropy("ugk_softmax_crossentropy", losses, probs, logits, unchecked(targets), B, T, V, {});
 }
 
-namespace {
-int xent_backward(const char *fn, bool zeroed, float *dlogits, const float *probs, const int *targets, int B, int T,
-                  int V) {
-  if (int e = check_btc(fn, B, T, V)) return e;
-  if ((long long)B * T * V == 0) return ok();
-  if (any_null({dlogits, probs, targets})) return bad(fn, "NULL pointer");
-  const float dloss = 1.0f / (B * T);  // train_bnn.c:360
-  if (int e = launch_crossentropy_softmax_backward(dlogits, probs, targets, B * T, V, dloss, zeroed)) return e;
-  return ok();
+int ugk_softmax_crossentropy_checked(float *losses, float *probs, const float *logits, int *targets, int B, int T,
+                                     int V) {
+  const char *fn = "ugk_softmax_crossentropy_checked";
+  IdCheck ids;
+  if (int e = id_check(fn, V, 0, UGK_IDS_SOFTMAX_CROSSENTROPY, &ids)) return e;
+  return softmax_crossentropy(fn, losses, probs, logits, targets, B, T, V, ids);
 }
-}  // namespace
 
 int ugk_crossentropy_softmax_backward(float *dlogits, const float *probs, const int *targets, int B, int T, int V) {
-  return xent_backward("ugk_crossentropy_softmax_backward", false, dlogits, probs, targets, B, T, V);
+  return xent_backward("ugk_crossentropy_softmax_backward", false, dlogits, probs, unchecked(targets), B, T, V, {});
 }
 
 int ugk_crossentropy_softmax_backward_zeroed(float *dlogits, const float *probs, const int *targets, int B, int T,
                                              int V) {
-  return xent_backward("ugk_crossentropy_softmax_backward_zeroed", true, dlogits, probs, targets, B, T, V);
+  return xent_backward("ugk_crossentropy_softmax_backward_zeroed", true, dlogits, probs, unchecked(targets), B, T, V, {});
+}
+
+int ugk_crossentropy_softmax_backward_checked(float *dlogits, const float *probs, int *targets, int B, int T, int V,
+                                              int zeroed) {
+  const char *fn = "ugk_crossentropy_softmax_backward_checked";
+  IdCheck ids;
+  if (int e = id_check(fn, V, 0, UGK_IDS_CROSSENTROPY_BACKWARD, &ids)) return e;
+  return xent_backward(fn, zeroed != 0, dlogits, probs, targets, B, T, V, ids);
 }
 
 int ugk_bayes_sample(float *w, float *eps, const float *mu, const float *rho, size_t n,

@@ -78,15 +78,15 @@ constexpr int kEmpty = -1;
 
 // ---- forward ---------------------------------------------------------------
 
-__global__ __launch_bounds__(kBlock) void k_enc_fwd_vec(float4 *__restrict__ out, const int *__restrict__ inp,
+__global__ __launch_bounds__(kBlock) void k_enc_fwd_vec(float4 *__restrict__ out, int *inp,
                                                         const float4 *__restrict__ wte,
                                                         const float4 *__restrict__ wpe, int BT, int T,
-                                                        int C4) {
+                                                        int C4, IdCheck ids) {
   const int lane = threadIdx.x & (kWave - 1);
   const int bt = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
   if (bt >= BT) return;
   const int t = bt % T;
-  const int ix = inp[bt];
+  const int ix = checked_id(inp, bt, ids);
   const float4 *a = wte + (size_t)ix * C4;
   const float4 *p = wpe + (size_t)t * C4;
   float4 *o = out + (size_t)bt * C4;
@@ -100,13 +100,14 @@ __global__ __launch_bounds__(kBlock) void k_enc_fwd_vec(float4 *__restrict__ out
 // every load of the row issued before the first store (columns past the row
 // load the last one again and are not stored).
 template <int V>
-__global__ __launch_bounds__(kBlock) void k_enc_fwd_row(float4 *__restrict__ out, const int *__restrict__ inp,
+__global__ __launch_bounds__(kBlock) void k_enc_fwd_row(float4 *__restrict__ out, int *inp,
                                                         const float4 *__restrict__ wte,
-                                                        const float4 *__restrict__ wpe, int BT, int T, int C4) {
+                                                        const float4 *__restrict__ wpe, int BT, int T, int C4,
+                                                        IdCheck ids) {
   const int lane = threadIdx.x & (kWave - 1);
   const int bt = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
   if (bt >= BT) return;
-  const size_t ot = (size_t)inp[bt] * C4, op = (size_t)(bt % T) * C4;
+  const size_t ot = (size_t)checked_id(inp, bt, ids) * C4, op = (size_t)(bt % T) * C4;
   float4 x[V], y[V];
 #pragma unroll
   for (int v = 0; v < V; v++) {
@@ -122,13 +123,13 @@ __global__ __launch_bounds__(kBlock) void k_enc_fwd_row(float4 *__restrict__ out
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_enc_fwd_scalar(float *out, const int *inp, const float *wte,
-                                                           const float *wpe, int BT, int T, int C) {
+__global__ __launch_bounds__(kBlock) void k_enc_fwd_scalar(float *out, int *inp, const float *wte,
+                                                           const float *wpe, int BT, int T, int C, IdCheck ids) {
   const int lane = threadIdx.x & (kWave - 1);
   const int bt = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
   if (bt >= BT) return;
   const int t = bt % T;
-  const int ix = inp[bt];
+  const int ix = checked_id(inp, bt, ids);
   for (int c = lane; c < C; c += kWave)
     out[(size_t)bt * C + c] = wte[(size_t)ix * C + c] + wpe[(size_t)t * C + c];
 }
@@ -166,8 +167,7 @@ __device__ __forceinline__ unsigned hash_slot(int tok, unsigned mask, int shift)
 // K1: insert the chunk's rows; blocks past the insert range run dwpe, kB rows
 // of a (t, c) entry in flight.
 template <bool kVec, int kB>
-__global__ __launch_bounds__(kBlock) void k_enc_bwd_insert(EncTable tb, EncShared sh, const int *__restrict__ inp,
-                                                           int n, unsigned mask, int shift, int ins_blocks,
+__global__ __launch_bounds__(kBlock) void k_enc_bwd_insert(EncTable tb, EncShared sh, int *inp, IdCheck ids, int n, unsigned mask, int shift, int ins_blocks,
                                                            float *dwpe, const float *dout, int B, int T, int C) {
   if ((int)blockIdx.x < ins_blocks) {
     constexpr int kL = 2 * kBlock;  // LDS table slots
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(kBlock) void k_enc_bwd_insert(EncTable tb, EncShare
     }
     __syncthreads();
     const int i = blockIdx.x * kBlock + threadIdx.x;
-    const int tok = i < n ? inp[i] : -1;
+    const int tok = i < n ? checked_id(inp, i, ids) : -1;
     int e = -1, lrank = 0;
     if (tok >= 0) {  // at most 256 distinct tokens in 512 slots: always found
       e = (int)hash_slot(tok, kL - 1, 32 - 9);
@@ -935,8 +935,8 @@ int *ids_error_word() {
   return a.ptr;
 }
 
-int launch_encoder_forward(float *out, const int *inp, const float *wte, const float *wpe, int B,
-                           int T, int C) {
+int launch_encoder_forward(float *out, int *inp, const float *wte, const float *wpe, int B, int T, int C,
+                           const IdCheck &ids) {
   const int BT = B * T;
   if (BT == 0 || C == 0) return 0;
   const dim3 grid(grid_for((size_t)BT, kWavesPerBlock)), block(kBlock);
@@ -947,22 +947,22 @@ int launch_encoder_forward(float *out, const int *inp, const float *wte, const f
     switch ((C4 + kWave - 1) / kWave) {
 #define UGK_ENC_ROW(v) \
   case v:              \
-    launch(k_enc_fwd_row<v>, grid, block, 0, o4, inp, te4, pe4, BT, T, C4); \
+    launch(k_enc_fwd_row<v>, grid, block, 0, o4, inp, te4, pe4, BT, T, C4, ids); \
     break;
       UGK_ENC_ROW(1) UGK_ENC_ROW(2) UGK_ENC_ROW(3) UGK_ENC_ROW(4)
       UGK_ENC_ROW(5) UGK_ENC_ROW(6) UGK_ENC_ROW(7) UGK_ENC_ROW(8)
 #undef UGK_ENC_ROW
       default:  // rows beyond 2,048 channels: the lane loop
-        launch(k_enc_fwd_vec, grid, block, 0, o4, inp, te4, pe4, BT, T, C4);
+        launch(k_enc_fwd_vec, grid, block, 0, o4, inp, te4, pe4, BT, T, C4, ids);
     }
   } else {
-    launch(k_enc_fwd_scalar, grid, block, 0, out, inp, wte, wpe, BT, T, C);
+    launch(k_enc_fwd_scalar, grid, block, 0, out, inp, wte, wpe, BT, T, C, ids);
   }
   return check_launch("encoder_forward");
 }
 
-int launch_encoder_backward(float *dwte, float *dwpe, const float *dout, const int *inp, int B,
-                            int T, int C) {
+int launch_encoder_backward(float *dwte, float *dwpe, const float *dout, int *inp, int B, int T, int C,
+                            const IdCheck &ids) {
   const int BT = B * T;
   if (BT == 0 || C == 0) return 0;
   // the bucket state lives in its own workspace region; new memory is cleared
@@ -1001,7 +1001,7 @@ int launch_encoder_backward(float *dwte, float *dwpe, const float *dout, const i
       pe_blocks = deep ? (int)grid_for((size_t)T * C, kBlock)
                        : ((int)grid_for((size_t)T * (vec ? C / 4 : C), kBlock) + 1) / 2;
     const auto insert = [&](auto k) {
-      launch(k, dim3(ins_blocks + pe_blocks), dim3(kBlock), 0, tb, sh, inp + c0, n, mask, shift, ins_blocks, dwpe, dout,
+      launch(k, dim3(ins_blocks + pe_blocks), dim3(kBlock), 0, tb, sh, inp + c0, ids, n, mask, shift, ins_blocks, dwpe, dout,
              B, T, C);
     };
     if (deep) insert(k_enc_bwd_insert<false, 32>);

@@ -167,6 +167,27 @@ __device__ __forceinline__ void chain_add4(float (&s)[kArr], const float4 *const
   }
 }
 
+// The id check inside an op's own kernels, in place of a launch of
+// ugk_ids_guard's: an id beyond `last` is replaced by `fill`, in place, and
+// `code` goes into the error word. An unchecked call has the last unsigned
+// value there, which no id is beyond.
+struct IdCheck {
+  unsigned last = 0xffffffffu;
+  int fill = 0, code = 0;
+  int *word = nullptr;
+};
+// id as read from ids[i], checked. Threads that read the same id find it in
+// range, or replace it by the same value, in any order. (Where the read's
+// latency counts it is made early, and the id checked where it is used.)
+__device__ __forceinline__ int check_id(int id, int *ids, size_t i, const IdCheck &g) {
+  if ((unsigned)id > g.last) {
+    id = ids[i] = g.fill;
+    *g.word = g.code;
+  }
+  return id;
+}
+__device__ __forceinline__ int checked_id(int *ids, size_t i, const IdCheck &g) { return check_id(ids[i], ids, i, g); }
+
 // Launchers, one per kernel family. Each validates nothing (ugk_api.hip does)
 // and returns the launch status through check_launch.
 int launch_residual_forward(float *out, const float *x, const float *y, size_t n);
@@ -214,9 +235,9 @@ int launch_layernorm_backward(float *dinp, float *dweight, float *dbias,
                               const float *mean, const float *rstd, int rows, int C);
 // residual_forward then layernorm_forward of its output, in one pass when the
 // float4 path applies (two launches otherwise).
-int launch_encoder_layernorm_forward(float *enc, float *out, float *mean, float *rstd, const int *inp,
+int launch_encoder_layernorm_forward(float *enc, float *out, float *mean, float *rstd, int *inp,
                                      const float *wte, const float *wpe, const float *weight, const float *bias,
-                                     int B, int T, int C);
+                                     int B, int T, int C, const IdCheck &ids);
 int launch_residual_layernorm_forward(float *res, float *out, float *mean, float *rstd, const float *x,
                                       const float *y, const float *weight, const float *bias, int rows,
                                       int C);
@@ -289,15 +310,14 @@ constexpr int kMaxPartialRows = 1024;  // partial rows the column-sum kernel tak
 constexpr size_t kNoAllocScratchBytes = (size_t)8 << 20;
 float *noalloc_scratch();
 int noalloc_max_blocks(int C);
-int launch_softmax_crossentropy(float *losses, float *probs, const float *logits, const int *targets, int rows,
-                                int V);
-int launch_crossentropy_softmax_backward(float *dlogits, const float *probs, const int *targets, int rows, int V,
-                                         float dloss,
-                                         bool zeroed = false);
-int launch_encoder_forward(float *out, const int *inp, const float *wte,
-                           const float *wpe, int B, int T, int C);
-int launch_encoder_backward(float *dwte, float *dwpe, const float *dout,
-                            const int *inp, int B, int T, int C);
+int launch_softmax_crossentropy(float *losses, float *probs, const float *logits, int *targets, int rows, int V,
+                                const IdCheck &ids);
+int launch_crossentropy_softmax_backward(float *dlogits, const float *probs, int *targets, int rows, int V,
+                                         float dloss, bool zeroed, const IdCheck &ids);
+int launch_encoder_forward(float *out, int *inp, const float *wte, const float *wpe, int B, int T, int C,
+                           const IdCheck &ids);
+int launch_encoder_backward(float *dwte, float *dwpe, const float *dout, int *inp, int B, int T, int C,
+                            const IdCheck &ids);
 // Buckets of more than 32 rows: 0 (default) blocked adds (64-row blocks, each
 // in row order, the block sums in block order), 1 one add per row in row
 // order (bit-identical to train_bnn.c).

@@ -218,7 +218,7 @@ __global__ __launch_bounds__(kBlock) void k_ln_fwd_vec(float *__restrict__ out, 
 template <int V, int RPW, bool kEarly>
 __global__ __launch_bounds__(kBlock) void k_enc_ln_fwd_vec(float *__restrict__ enc, float *__restrict__ out,
                                                            float *__restrict__ mean, float *__restrict__ rstd,
-                                                           const int *__restrict__ inp,
+                                                           int *inp, IdCheck ids,
                                                            const float *__restrict__ wte,
                                                            const float *__restrict__ wpe,
                                                            const float *__restrict__ weight,
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(kBlock) void k_enc_ln_fwd_vec(float *__restrict__ e
   const Cols<V, false> cl(lane, kWave, C);
   float4 xa[V], ya[V];
   {
-    const float *te = wte + (size_t)inp[row0] * C, *pe = wpe + (size_t)(row0 % T) * C;
+    const float *te = wte + (size_t)checked_id(inp, row0, ids) * C, *pe = wpe + (size_t)(row0 % T) * C;
 #pragma unroll
     for (int v = 0; v < V; v++) {
       xa[v] = ld4(te + cl.at[v]);
@@ -243,7 +243,7 @@ __global__ __launch_bounds__(kBlock) void k_enc_ln_fwd_vec(float *__restrict__ e
     float4 xb[V], yb[V];
     if (k + 1 < RPW) {
       const int nx = min(row + 1, rows - 1);
-      const float *te = wte + (size_t)inp[nx] * C, *pe = wpe + (size_t)(nx % T) * C;
+      const float *te = wte + (size_t)checked_id(inp, nx, ids) * C, *pe = wpe + (size_t)(nx % T) * C;
 #pragma unroll
       for (int v = 0; v < V; v++) {
         xb[v] = ld4(te + cl.at[v]);
@@ -1388,20 +1388,20 @@ int launch_residual_layernorm_forward(float *res, float *out, float *mean, float
   return check_launch("residual_layernorm_forward");
 }
 
-int launch_encoder_layernorm_forward(float *enc, float *out, float *mean, float *rstd, const int *inp,
+int launch_encoder_layernorm_forward(float *enc, float *out, float *mean, float *rstd, int *inp,
                                      const float *wte, const float *wpe, const float *weight, const float *bias,
-                                     int B, int T, int C) {
+                                     int B, int T, int C, const IdCheck &ids) {
   const int rows = B * T;
   if (rows == 0) return 0;
   if (layernorm_exact() || !row_in_wave(C) || (C & 3) != 0) {
-    if (int e = launch_encoder_forward(enc, inp, wte, wpe, B, T, C)) return e;
+    if (int e = launch_encoder_forward(enc, inp, wte, wpe, B, T, C, ids)) return e;
     return launch_layernorm_forward(out, mean, rstd, enc, weight, bias, rows, C);
   }
   const int V = slots_of(C, kWave);
   const int rpw = fwd_rpw(rows, C, true);
   const dim3 grid(grid_for((size_t)rows, (size_t)kWavesPerBlock * rpw)), block(kBlock);
   const auto go = [&](auto k) {
-    launch(k, grid, block, 0, enc, out, mean, rstd, inp, wte, wpe, weight, bias, rows, T, C);
+    launch(k, grid, block, 0, enc, out, mean, rstd, inp, ids, wte, wpe, weight, bias, rows, T, C);
   };
   switch (V) {
 #define UGK_ENC_LN(v)                                             \

@@ -95,7 +95,7 @@ __device__ __forceinline__ void store_loss(float *losses, size_t row, const floa
 template <int kThreads, int kPer>
 __global__ __launch_bounds__(kThreads) void k_softmax_xent(float *__restrict__ losses, float *__restrict__ probs,
                                                            const float *__restrict__ logits,
-                                                           const int *__restrict__ targets, int V) {
+                                                           int *targets, IdCheck ids, int V) {
   __shared__ uint64_t tab[32];
   __shared__ float lds[kThreads / kWave];
   ugk_exp2_stage(tab);
@@ -107,6 +107,7 @@ __global__ __launch_bounds__(kThreads) void k_softmax_xent(float *__restrict__ l
   // spans (a misaligned row's stores would write partial cache lines).
   const int skew = (int)(((uintptr_t)pr >> 2) & 63);
   const int tid = threadIdx.x;
+  const int target = targets[row];
   float x[kPer];
 #pragma unroll
   for (int k = 0; k < kPer; k++) {
@@ -139,7 +140,7 @@ __global__ __launch_bounds__(kThreads) void k_softmax_xent(float *__restrict__ l
   };
   if (__all(lo >= kUgkDivRecipKeyMin)) store(std::true_type{});
   else store(std::false_type{});
-  store_loss(losses, row, lg, targets[row], skew, m, s, tab, kThreads);
+  store_loss(losses, row, lg, check_id(target, targets, row, ids), skew, m, s, tab, kThreads);
 }
 
 // The same row computation for rows of up to 51,393 logits, with two rows
@@ -153,7 +154,7 @@ __global__ __launch_bounds__(kThreads) void k_softmax_xent(float *__restrict__ l
 template <int kThreads, int kReg, int kLds>
 __global__ __launch_bounds__(kThreads, 2 * kThreads / kWave / 4) void k_softmax_xent_split(
     float *__restrict__ losses, float *__restrict__ probs, const float *__restrict__ logits,
-    const int *__restrict__ targets, int V) {
+    int *targets, IdCheck ids, int V) {
   // one LDS block with the expf table first, so that its address fits the
   // offset field of the table reads
   __shared__ struct {
@@ -169,6 +170,7 @@ __global__ __launch_bounds__(kThreads, 2 * kThreads / kWave / 4) void k_softmax_
   float *pr = probs + row * (size_t)V;
   const int skew = (int)(((uintptr_t)pr >> 2) & 63);  // as in k_softmax_xent
   const int tid = threadIdx.x, wave = tid / kWave;
+  const int target = targets[row];
   const int v0 = tid - skew;  // element of slot tid; slot tid + k * kThreads holds v0 + k * kThreads
   // Slots outside the row hold -inf: the max rule skips it and expf gives +0,
   // which leaves the sum's bits unchanged, so only the loads and stores test
@@ -239,7 +241,7 @@ __global__ __launch_bounds__(kThreads, 2 * kThreads / kWave / 4) void k_softmax_
   };
   if (__all(lo >= kUgkDivRecipKeyMin)) store(std::true_type{});
   else store(std::false_type{});
-  store_loss(losses, row, lg, targets[row], skew, m, s, tab, kThreads);
+  store_loss(losses, row, lg, check_id(target, targets, row, ids), skew, m, s, tab, kThreads);
 }
 
 // Row of flat element i (rows of V elements): a double-precision quotient,
@@ -354,14 +356,14 @@ __device__ __forceinline__ float xent_grad(float d, float p, bool hit, float dlo
 template <bool kZero>
 __global__ __launch_bounds__(kBwdThreads) void k_xent_softmax_bwd_flat4(float *__restrict__ dlogits,
                                                                         const float *__restrict__ probs,
-                                                                        const int *__restrict__ targets, int rows,
-                                                                        int V, float dloss, size_t n4, unsigned full,
+                                                                        int *targets, IdCheck ids, int rows, int V,
+                                                                        float dloss, size_t n4, unsigned full,
                                                                         unsigned lead, unsigned rest, double inv_v) {
   if (blockIdx.x == full) {
     for (unsigned k = threadIdx.x; k < rest; k += kBwdThreads) {
       const size_t i = k < lead ? k : 4 * n4 + k;
       const size_t r = row_of(i, (size_t)V, inv_v);
-      dlogits[i] = xent_grad(kZero ? 0.0f : dlogits[i], probs[i], i - r * (size_t)V == (size_t)targets[r], dloss);
+      dlogits[i] = xent_grad(kZero ? 0.0f : dlogits[i], probs[i], i - r * (size_t)V == (size_t)checked_id(targets, r, ids), dloss);
     }
     return;
   }
@@ -371,8 +373,10 @@ __global__ __launch_bounds__(kBwdThreads) void k_xent_softmax_bwd_flat4(float *_
   const float4 p = ld_nt4(probs + i);
   const float4 d = kZero ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : ld_nt4(dlogits + i);
   const size_t r0 = row_of(i, (size_t)V, inv_v);
-  const size_t t0 = r0 * (size_t)V + (size_t)targets[r0];
-  const size_t t1 = (r0 + 1 < (size_t)rows) ? (r0 + 1) * (size_t)V + (size_t)targets[r0 + 1] : ~(size_t)0;
+  const bool two = r0 + 1 < (size_t)rows;
+  const int id0 = targets[r0], id1 = targets[two ? r0 + 1 : r0];
+  const size_t t0 = r0 * (size_t)V + (size_t)check_id(id0, targets, r0, ids);
+  const size_t t1 = two ? (r0 + 1) * (size_t)V + (size_t)check_id(id1, targets, r0 + 1, ids) : ~(size_t)0;
   st_nt4(dlogits + i, make_float4(xent_grad(d.x, p.x, i == t0 || i == t1, dloss),
                                   xent_grad(d.y, p.y, i + 1 == t0 || i + 1 == t1, dloss),
                                   xent_grad(d.z, p.z, i + 2 == t0 || i + 2 == t1, dloss),
@@ -382,13 +386,12 @@ __global__ __launch_bounds__(kBwdThreads) void k_xent_softmax_bwd_flat4(float *_
 // Rows of fewer than 4 logits: a thread per element.
 template <bool kZero>
 __global__ __launch_bounds__(kBwdThreads) void k_xent_softmax_bwd(float *__restrict__ dlogits,
-                                                                  const float *__restrict__ probs,
-                                                                  const int *__restrict__ targets, int V, size_t n,
-                                                                  float dloss) {
+                                                                  const float *__restrict__ probs, int *targets,
+                                                                  IdCheck ids, int V, size_t n, float dloss) {
   const size_t i = (size_t)blockIdx.x * kBwdThreads + threadIdx.x;
   if (i >= n) return;
   const size_t r = i / (unsigned)V;
-  dlogits[i] = xent_grad(kZero ? 0.0f : dlogits[i], probs[i], (int)(i - r * (unsigned)V) == targets[r], dloss);
+  dlogits[i] = xent_grad(kZero ? 0.0f : dlogits[i], probs[i], (int)(i - r * (unsigned)V) == checked_id(targets, r, ids), dloss);
 }
 
 // ---- exact mode: train_bnn.c's order of the row sum ---------------------------
@@ -506,9 +509,9 @@ __global__ __launch_bounds__(kSxThreads) void k_softmax_sum_exact(float2 *__rest
 // adjacent and laid from the 256-byte boundary of probs at or before the
 // row's start, so that each wavefront's store covers whole lines
 __global__ __launch_bounds__(kBlock) void k_softmax_norm_rows(float *__restrict__ losses, float *__restrict__ probs,
-                                                              const float *__restrict__ logits,
-                                                              const int *__restrict__ targets,
-                                                              const float2 *__restrict__ stats, int V, int chunks) {
+                                                              const float *__restrict__ logits, int *targets,
+                                                              IdCheck ids, const float2 *__restrict__ stats, int V,
+                                                              int chunks) {
   __shared__ uint64_t tab[32];
   ugk_exp2_stage(tab);
   __syncthreads();
@@ -517,7 +520,7 @@ __global__ __launch_bounds__(kBlock) void k_softmax_norm_rows(float *__restrict_
   const int skew = (int)((reinterpret_cast<uintptr_t>(probs + base) >> 2) & 63);
   const int v0 = (int)(blockIdx.x - (unsigned)row * chunks) * (kBlock * kSxNormPer) + (int)threadIdx.x - skew;
   const float2 st = stats[row];
-  const int tgt = targets[row];
+  const int tgt = checked_id(targets, row, ids);
   float x[kSxNormPer];
 #pragma unroll
   for (int k = 0; k < kSxNormPer; k++) {
@@ -555,16 +558,15 @@ __global__ __launch_bounds__(kBlock) void k_softmax_norm_rows(float *__restrict_
 std::atomic<int> g_softmax_exact{0};
 
 template <int kThreads, int kPer>
-void launch_rows(float *losses, float *probs, const float *logits, const int *targets, int rows, int V) {
-  hipLaunchKernelGGL((k_softmax_xent<kThreads, kPer>), dim3(rows), dim3(kThreads), 0, stream(), losses, probs,
-                     logits, targets, V);
+void launch_rows(float *losses, float *probs, const float *logits, int *targets, const IdCheck &ids, int rows, int V) {
+  launch(k_softmax_xent<kThreads, kPer>, dim3(rows), dim3(kThreads), 0, losses, probs, logits, targets, ids, V);
 }
 
-void launch_norm_rows(float *losses, float *probs, const float *logits, const int *targets, const float2 *stats,
-                      int rows, int V) {
+void launch_norm_rows(float *losses, float *probs, const float *logits, int *targets, const IdCheck &ids,
+                      const float2 *stats, int rows, int V) {
   const int chunks = (int)grid_for((size_t)V + 63, (size_t)kBlock * kSxNormPer);  // the skew: up to 63
   launch(k_softmax_norm_rows, dim3((unsigned)((size_t)rows * chunks)), dim3(kBlock), 0, losses, probs, logits, targets,
-         stats, V, chunks);
+         ids, stats, V, chunks);
 }
 
 }  // namespace
@@ -581,8 +583,8 @@ size_t softmax_scratch(int rows, int V) { return V > 0 ? (size_t)rows * sizeof(f
 void set_softmax_exact(int on) { g_softmax_exact.store(on ? 1 : 0); }
 int softmax_exact() { return g_softmax_exact.load(); }
 
-int launch_softmax_crossentropy(float *losses, float *probs, const float *logits, const int *targets, int rows,
-                                int V) {
+int launch_softmax_crossentropy(float *losses, float *probs, const float *logits, int *targets, int rows, int V,
+                                const IdCheck &ids) {
   if (rows == 0 || V == 0) return 0;
   if (softmax_exact()) {
     float2 *stats = static_cast<float2 *>(workspace(kRegSoftmax, softmax_scratch(rows, V)));
@@ -591,21 +593,20 @@ int launch_softmax_crossentropy(float *losses, float *probs, const float *logits
                        stream(), stats, logits, rows, V);
     hipLaunchKernelGGL(k_softmax_sum_exact, dim3(grid_for((size_t)rows, kSxRows)), dim3(kSxThreads), 0, stream(),
                        stats, logits, rows, V);
-    launch_norm_rows(losses, probs, logits, targets, stats, rows, V);
+    launch_norm_rows(losses, probs, logits, targets, ids, stats, rows, V);
     return check_launch("softmax_crossentropy (exact)");
   }
   // a row takes V + 63 slots at most (the alignment skew)
   const int W = V + 63;
-  if (W <= 64 * 2) launch_rows<64, 2>(losses, probs, logits, targets, rows, V);
-  else if (W <= 256) launch_rows<64, 4>(losses, probs, logits, targets, rows, V);
-  else if (W <= 1024) launch_rows<256, 4>(losses, probs, logits, targets, rows, V);
-  else if (W <= 4096) launch_rows<256, 16>(losses, probs, logits, targets, rows, V);
-  else if (W <= 16384) launch_rows<1024, 16>(losses, probs, logits, targets, rows, V);
-  else if (W <= 32768) launch_rows<1024, 32>(losses, probs, logits, targets, rows, V);
+  if (W <= 64 * 2) launch_rows<64, 2>(losses, probs, logits, targets, ids, rows, V);
+  else if (W <= 256) launch_rows<64, 4>(losses, probs, logits, targets, ids, rows, V);
+  else if (W <= 1024) launch_rows<256, 4>(losses, probs, logits, targets, ids, rows, V);
+  else if (W <= 4096) launch_rows<256, 16>(losses, probs, logits, targets, ids, rows, V);
+  else if (W <= 16384) launch_rows<1024, 16>(losses, probs, logits, targets, ids, rows, V);
+  else if (W <= 32768) launch_rows<1024, 32>(losses, probs, logits, targets, ids, rows, V);
   else if (V <= kSplitMaxV) {  // 42 slots per thread in registers, 25 in LDS: two rows per CU
     static_assert(32768 - 63 >= 768 * 42, "the split kernel's register slots must lie inside every row it takes");
-    hipLaunchKernelGGL((k_softmax_xent_split<768, 42, 25>), dim3(rows), dim3(768), 0, stream(), losses, probs,
-                       logits, targets, V);
+    launch(k_softmax_xent_split<768, 42, 25>, dim3(rows), dim3(768), 0, losses, probs, logits, targets, ids, V);
   } else {
     // Rows too long for the registers of one workgroup: a statistics pass
     // and a flat normalising pass (12 bytes per logit rather than 8).
@@ -615,27 +616,27 @@ int launch_softmax_crossentropy(float *losses, float *probs, const float *logits
       launch(k_softmax_stats<256>, dim3(rows), dim3(256), 0, stats, logits, V);
     else
       launch(k_softmax_stats<1024>, dim3(rows), dim3(1024), 0, stats, logits, V);
-    launch_norm_rows(losses, probs, logits, targets, stats, rows, V);
+    launch_norm_rows(losses, probs, logits, targets, ids, stats, rows, V);
   }
   return check_launch("softmax_crossentropy");
 }
 
-int launch_crossentropy_softmax_backward(float *dlogits, const float *probs, const int *targets, int rows, int V,
-                                         float dloss, bool zeroed) {
+int launch_crossentropy_softmax_backward(float *dlogits, const float *probs, int *targets, int rows, int V,
+                                         float dloss, bool zeroed, const IdCheck &ids) {
   if (rows == 0 || V == 0) return 0;
   const size_t n = (size_t)rows * V;
   if (V >= 4) {
     const size_t lead = (0 - ((uintptr_t)dlogits >> 2)) & 31, first = lead < n ? lead : n, n4 = (n - first) / 4;
     const unsigned full = grid_for(n4, kBwdThreads), rest = (unsigned)(n - 4 * n4);
     const auto go = [&](auto k) {
-      launch(k, dim3(full + (rest ? 1 : 0)), dim3(kBwdThreads), 0, dlogits, probs, targets, rows, V, dloss, n4, full,
+      launch(k, dim3(full + (rest ? 1 : 0)), dim3(kBwdThreads), 0, dlogits, probs, targets, ids, rows, V, dloss, n4, full,
              (unsigned)first, rest, 1.0 / (double)V);
     };
     if (zeroed) go(k_xent_softmax_bwd_flat4<true>);
     else go(k_xent_softmax_bwd_flat4<false>);
   } else {
     const auto go = [&](auto k) {
-      launch(k, dim3(grid_for(n, kBwdThreads)), dim3(kBwdThreads), 0, dlogits, probs, targets, V, n, dloss);
+      launch(k, dim3(grid_for(n, kBwdThreads)), dim3(kBwdThreads), 0, dlogits, probs, targets, ids, V, n, dloss);
     };
     if (zeroed) go(k_xent_softmax_bwd<true>);
     else go(k_xent_softmax_bwd<false>);

@@ -130,6 +130,11 @@ _SIGS = {
     "ugk_diag_stream": [_fp, _sz, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int],
     "ugk_diag_layernorm_partial_rows": [_i, _i, _i, ctypes.POINTER(_i), ctypes.POINTER(_i)],
     "ugk_ids_guard": [_fp, _i, _i, _i, _i],
+    "ugk_encoder_forward_checked": [_fp, _fp, _fp, _fp, _i, _i, _i, _i],
+    "ugk_encoder_backward_checked": [_fp, _fp, _fp, _fp, _i, _i, _i, _i],
+    "ugk_encoder_layernorm_forward_checked": [_fp] * 9 + [_i, _i, _i, _i],
+    "ugk_softmax_crossentropy_checked": [_fp, _fp, _fp, _fp, _i, _i, _i],
+    "ugk_crossentropy_softmax_backward_checked": [_fp, _fp, _fp, _i, _i, _i, _i],
     "ugk_diag_layernorm_tail": [_i],
     "ugk_loader_open": [ctypes.POINTER(_fp), ctypes.c_char_p],
     "ugk_loader_count": [ctypes.c_char_p, ctypes.POINTER(ctypes.c_long)],
@@ -187,14 +192,13 @@ def _ptr(x, what: str, need: int, dtype: str):
 
 # Token and target ids index tables (rows of wte, logits of a row): an id out of range would make a
 # kernel read or write outside them. The reference leaves 0 <= id < V to its callers unchecked.
-# Here each tensor of ids goes through ugk_ids_guard on the device first, on the library's stream:
-# ids out of range are replaced in place (so no kernel indexes outside its table; ids in range are
+# Here a tensor of ids goes to the op's _checked entry point, whose kernels check each id as they read
+# it: ids out of range are replaced in place (so no kernel indexes outside its table; ids in range are
 # not written), and the library records the op, which the next synchronize() raises as UgkError.
-# No host round trip, so the calls stay asynchronous and may be captured in a graph.
+# No host round trip and no launch of its own (which cost a small call about 4 us on the GPU), so the
+# calls stay asynchronous and may be captured in a graph.
 # set_sync_checks(True) checks on the host instead (reading the ids back, a device synchronisation
 # per call) and raises ValueError at once, leaving the ids untouched.
-_IDS_CODE = {"encoder_forward": 1, "encoder_backward": 2, "encoder_layernorm_forward": 3, "softmax_crossentropy": 4,
-             "crossentropy_softmax_backward": 5, "crossentropy_softmax_backward_zeroed": 5}
 _sync_checks = False
 
 
@@ -205,48 +209,45 @@ def set_sync_checks(on: bool) -> None:
     _sync_checks = bool(on)
 
 
-def _guard_ids(ids, n: int, bound: int, fill: int, what: str) -> None:
-    """Guard a device tensor of ids (see above); a device address, or a tensor that the argument
-    checks reject, is left alone."""
+def _guarded(ids, n: int, bound: int, what: str) -> bool:
+    """Whether a device tensor of ids goes to the checked entry point (see above); a device address,
+    or a tensor that the argument checks reject, does not."""
     import torch
     if not (isinstance(ids, torch.Tensor) and ids.is_cuda and ids.dtype == torch.int32 and ids.is_contiguous()):
-        return
-    if n <= 0 or ids.numel() < n:
-        return  # nothing to index, or the size check of the call rejects it
+        return False
+    if n <= 0 or bound <= 0 or ids.numel() < n:
+        return False  # nothing to index, or the size checks of the call reject it
     if _sync_checks and not torch.cuda.is_current_stream_capturing():
         t = ids.reshape(-1)[:n]
         lo, hi = int(t.min()), int(t.max())
         if lo < 0 or hi >= bound:
             raise ValueError(f"{what}: ids must lie in [0, {bound}), got [{lo}, {hi}]")
-        return
-    _check(lib.ugk_ids_guard(ids.data_ptr(), n, bound, fill, _IDS_CODE[what]))
+        return False
+    return True
 
 
-def _check_tokens(inp, table, C: int, n: int, what: str, fill: int = 0) -> None:
-    """Token ids index rows of ``table`` (``table.numel() // C`` rows)."""
+def _rows(table, C: int) -> int:
+    """Rows of a device tensor of C channels (0 if it is none: its ids then go unchecked)."""
     import torch
-    if isinstance(table, torch.Tensor) and table.is_cuda and C:
-        _guard_ids(inp, n, table.numel() // C, fill, what)
-
-
-def _check_targets(targets, V: int, rows: int, what: str) -> None:
-    """Target ids index a row of V logits."""
-    _guard_ids(targets, rows, V, 0, what)
+    return table.numel() // C if isinstance(table, torch.Tensor) and table.is_cuda and C else 0
 
 
 def encoder_forward(out, inp, wte, wpe, B: int, T: int, C: int) -> None:
     """train_bnn.c:41-65. ``out[b,t,:] = wte[inp[b,t],:] + wpe[t,:]``."""
-    _check_tokens(inp, wte, C, B * T, "encoder_forward")
-    _check(lib.ugk_encoder_forward(_ptr(out, "out", B * T * C, "f32"), _ptr(inp, "inp", B * T, "i32"),
-                                   _ptr(wte, "wte", C, "f32"), _ptr(wpe, "wpe", T * C, "f32"), B, T, C))
+    V = _rows(wte, C)
+    checked = _guarded(inp, B * T, V, "encoder_forward")
+    args = (_ptr(out, "out", B * T * C, "f32"), _ptr(inp, "inp", B * T, "i32"), _ptr(wte, "wte", C, "f32"),
+            _ptr(wpe, "wpe", T * C, "f32"), B, T, C)
+    _check(lib.ugk_encoder_forward_checked(*args, V) if checked else lib.ugk_encoder_forward(*args))
 
 
 def encoder_backward(dwte, dwpe, dout, inp, B: int, T: int, C: int) -> None:
     """train_bnn.c:647-662. ``dwte[inp[b,t],:] += dout[b,t,:]``; ``dwpe[t,:] += dout[b,t,:]``."""
-    _check_tokens(inp, dwte, C, B * T, "encoder_backward", fill=-1)  # a negative id: the row is skipped
-    _check(lib.ugk_encoder_backward(_ptr(dwte, "dwte", C, "f32"), _ptr(dwpe, "dwpe", T * C, "f32"),
-                                    _ptr(dout, "dout", B * T * C, "f32"), _ptr(inp, "inp", B * T, "i32"),
-                                    B, T, C))
+    V = _rows(dwte, C)
+    checked = _guarded(inp, B * T, V, "encoder_backward")  # out of range: -1, the row is skipped
+    args = (_ptr(dwte, "dwte", C, "f32"), _ptr(dwpe, "dwpe", T * C, "f32"), _ptr(dout, "dout", B * T * C, "f32"),
+            _ptr(inp, "inp", B * T, "i32"), B, T, C)
+    _check(lib.ugk_encoder_backward_checked(*args, V) if checked else lib.ugk_encoder_backward(*args))
 
 
 def layernorm_forward(out, mean, rstd, inp, weight, bias, B: int, T: int, C: int) -> None:
@@ -269,12 +270,12 @@ def layernorm_backward(dinp, dweight, dbias, dout, inp, weight, mean, rstd, B: i
 
 def encoder_layernorm_forward(enc, out, mean, rstd, inp, wte, wpe, weight, bias, B: int, T: int, C: int) -> None:
     """``encoder_forward(enc, inp, wte, wpe)`` then ``layernorm_forward(out, mean, rstd, enc, ...)``, one pass."""
-    n, rows = B * T * C, B * T
-    _check_tokens(inp, wte, C, rows, "encoder_layernorm_forward")
-    _check(lib.ugk_encoder_layernorm_forward(
-        _ptr(enc, "enc", n, "f32"), _ptr(out, "out", n, "f32"), _ptr(mean, "mean", rows, "f32"),
-        _ptr(rstd, "rstd", rows, "f32"), _ptr(inp, "inp", rows, "i32"), _ptr(wte, "wte", C, "f32"),
-        _ptr(wpe, "wpe", T * C, "f32"), _ptr(weight, "weight", C, "f32"), _ptr(bias, "bias", C, "f32"), B, T, C))
+    n, rows, V = B * T * C, B * T, _rows(wte, C)
+    checked = _guarded(inp, rows, V, "encoder_layernorm_forward")
+    args = (_ptr(enc, "enc", n, "f32"), _ptr(out, "out", n, "f32"), _ptr(mean, "mean", rows, "f32"),
+            _ptr(rstd, "rstd", rows, "f32"), _ptr(inp, "inp", rows, "i32"), _ptr(wte, "wte", C, "f32"),
+            _ptr(wpe, "wpe", T * C, "f32"), _ptr(weight, "weight", C, "f32"), _ptr(bias, "bias", C, "f32"), B, T, C)
+    _check(lib.ugk_encoder_layernorm_forward_checked(*args, V) if checked else lib.ugk_encoder_layernorm_forward(*args))
 
 
 def residual_layernorm_forward(res, out, mean, rstd, x, y, weight, bias, B: int, T: int, C: int) -> None:
@@ -329,28 +330,29 @@ def bayes_materialize(w, mu, rho, eps, n: int) -> None:
 def softmax_crossentropy(losses, probs, logits, targets, B: int, T: int, V: int) -> None:
     """train_bnn.c:279-304. ``probs`` = row softmax of ``logits``; ``losses`` = -log probs[target]."""
     rows, n = B * T, B * T * V
-    _check_targets(targets, V, rows, "softmax_crossentropy")
-    _check(lib.ugk_softmax_crossentropy(_ptr(losses, "losses", rows, "f32"), _ptr(probs, "probs", n, "f32"),
-                                        _ptr(logits, "logits", n, "f32"), _ptr(targets, "targets", rows, "i32"),
-                                        B, T, V))
+    f = lib.ugk_softmax_crossentropy_checked if _guarded(targets, rows, V, "softmax_crossentropy") \
+        else lib.ugk_softmax_crossentropy
+    _check(f(_ptr(losses, "losses", rows, "f32"), _ptr(probs, "probs", n, "f32"), _ptr(logits, "logits", n, "f32"),
+             _ptr(targets, "targets", rows, "i32"), B, T, V))
 
 
 def crossentropy_softmax_backward(dlogits, probs, targets, B: int, T: int, V: int) -> None:
     """train_bnn.c:358-378. ``dlogits += (probs - onehot(target)) / (B*T)``."""
-    rows, n = B * T, B * T * V
-    _check_targets(targets, V, rows, "crossentropy_softmax_backward")
-    _check(lib.ugk_crossentropy_softmax_backward(_ptr(dlogits, "dlogits", n, "f32"), _ptr(probs, "probs", n, "f32"),
-                                                 _ptr(targets, "targets", rows, "i32"), B, T, V))
+    _xent_backward("crossentropy_softmax_backward", dlogits, probs, targets, B, T, V, 0)
 
 
 def crossentropy_softmax_backward_zeroed(dlogits, probs, targets, B: int, T: int, V: int) -> None:
     """crossentropy_softmax_backward for a dlogits that is zero before the call (the arms' memset of
     the activation gradients): it is written, not read."""
+    _xent_backward("crossentropy_softmax_backward_zeroed", dlogits, probs, targets, B, T, V, 1)
+
+
+def _xent_backward(name, dlogits, probs, targets, B: int, T: int, V: int, zeroed: int) -> None:
     rows, n = B * T, B * T * V
-    _check_targets(targets, V, rows, "crossentropy_softmax_backward_zeroed")
-    _check(lib.ugk_crossentropy_softmax_backward_zeroed(_ptr(dlogits, "dlogits", n, "f32"),
-                                                        _ptr(probs, "probs", n, "f32"),
-                                                        _ptr(targets, "targets", rows, "i32"), B, T, V))
+    checked = _guarded(targets, rows, V, name)
+    args = (_ptr(dlogits, "dlogits", n, "f32"), _ptr(probs, "probs", n, "f32"), _ptr(targets, "targets", rows, "i32"),
+            B, T, V)
+    _check(lib.ugk_crossentropy_softmax_backward_checked(*args, zeroed) if checked else getattr(lib, "ugk_" + name)(*args))
 
 
 def bayes_sample(w, eps, mu, rho, n: int, seed: int, step: int) -> None:
