@@ -169,13 +169,33 @@ def _check(status: int) -> None:
         raise UgkError(status, lib.ugk_last_error().decode(errors="replace"))
 
 
+# torch (plumbing only: device memory), imported when the first tensor arrives, and what _ptr's
+# first line asks of a tensor
+_torch = _Tensor = _DTYPES = None
+
+
+def _import_torch():
+    global _torch, _Tensor, _DTYPES
+    if _torch is None:
+        import torch
+        _torch, _Tensor, _DTYPES = torch, torch.Tensor, {"f32": torch.float32, "i32": torch.int32}
+    return _torch
+
+
 def _ptr(x, what: str, need: int, dtype: str):
-    """Device address of ``x`` after checking it can hold ``need`` elements of ``dtype``."""
+    """Device address of ``x`` after checking it can hold ``need`` elements of ``dtype``. A call has up to
+    14 of these: what passes is decided in one line, the rest (addresses, subclasses, errors) by _ptr_or_raise."""
+    if type(x) is _Tensor and x.dtype is _DTYPES[dtype] and x.is_cuda and x.numel() >= need and x.is_contiguous():
+        return x.data_ptr()
+    return _ptr_or_raise(x, what, need, dtype)
+
+
+def _ptr_or_raise(x, what: str, need: int, dtype: str):
     if x is None:
         return None
     if isinstance(x, int):
         return x
-    import torch  # plumbing only: device memory
+    torch = _import_torch()
     want = {"f32": torch.float32, "i32": torch.int32}[dtype]
     if not isinstance(x, torch.Tensor):
         raise TypeError(f"{what}: expected a torch tensor or a device address, got {type(x)!r}")
@@ -212,7 +232,7 @@ def set_sync_checks(on: bool) -> None:
 def _guarded(ids, n: int, bound: int, what: str) -> bool:
     """Whether a device tensor of ids goes to the checked entry point (see above); a device address,
     or a tensor that the argument checks reject, does not."""
-    import torch
+    torch = _torch or _import_torch()
     if not (isinstance(ids, torch.Tensor) and ids.is_cuda and ids.dtype == torch.int32 and ids.is_contiguous()):
         return False
     if n <= 0 or bound <= 0 or ids.numel() < n:
@@ -228,7 +248,7 @@ def _guarded(ids, n: int, bound: int, what: str) -> bool:
 
 def _rows(table, C: int) -> int:
     """Rows of a device tensor of C channels (0 if it is none: its ids then go unchecked)."""
-    import torch
+    torch = _torch or _import_torch()
     return table.numel() // C if isinstance(table, torch.Tensor) and table.is_cuda and C else 0
 
 
