@@ -1,7 +1,7 @@
 """GPU: the encoder backward at the edges of its kernels, with the bit-exact checks of test_parity_gpu.py's
 enc_case: batches on both sides of 16 sequences (how many dwpe rows a thread has in flight), buckets on
 both sides of 1,024 rows (32- or 64-channel slices) and of 256 blocks of 64 rows (one or more rounds of
-block sums), more than 8,192 rows (rounds of the slot scan), small buckets of every size up to 33 rows, and
+block sums), more than 8,192 rows (rounds of the slot scan), up to 1,024 rows (one launch), small buckets of every size up to 33 rows, and
 widths around the slices and the three float4 a lane adds at a time."""
 import numpy as np
 import pytest
@@ -30,6 +30,13 @@ def test_bucket_sizes(gpu, oracle, C):
     counts = list(range(34)) + [63, 64, 65, 128, 129, 1024, 1025, 2500]
     inp = counts_to_tokens(counts, C)
     enc_case(gpu, oracle, 1, inp.size, C, len(counts), inp, C)
+
+
+@pytest.mark.parametrize("B,T", [(1, 1), (1, 63), (1, 65), (4, 128), (1, 513), (8, 128), (25, 41)])
+@pytest.mark.parametrize("C,V", [(5, 1), (64, 2), (384, 27), (768, 5000)])
+def test_few_rows(gpu, oracle, B, T, C, V):
+    """Up to 512 and 1,024 rows in one launch, and one row more: tokens with up to all of the rows."""
+    enc_case(gpu, oracle, B, T, C, V, gen.tokens_zipf(gen.rng(B + T), B * T, V), B * T + C, reps=2)
 
 
 @pytest.mark.parametrize("rows", [8191, 8192, 8193, 20500])

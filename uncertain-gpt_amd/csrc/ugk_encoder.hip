@@ -59,6 +59,7 @@
 #include <algorithm>
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include "ugk_internal.h"
 
@@ -164,6 +165,56 @@ __device__ __forceinline__ unsigned hash_slot(int tok, unsigned mask, int shift)
   return ((unsigned)tok * 0x9E3779B1u) >> shift & mask;
 }
 
+// Workgroup blk of nblk of the dwpe adds.
+template <bool kVec, int kB>
+__device__ __forceinline__ void add_dwpe(float *dwpe, const float *dout, int blk, int nblk, int B, int T, int C) {
+  // dwpe[t, c] += dout[b, t, c] for b = 0..B-1, in order, kB rows in flight.
+  // dout is read with ordinary (cached) loads: K2 reads the same rows again,
+  // and finds part of them in the cache (K2 15.8 -> 14.3 us at 8,192 x 768).
+  // Each dwpe thread takes two (t, c) entries, one after the other, so half
+  // as many dwpe workgroups stream at once and the inserts' round trips are
+  // delayed less (25.6 -> 24.8 us per call at 8,192 x 768). Large batches of
+  // short sequences have few entries of many rows: they take one channel per
+  // thread and 32 rows in flight (128 x 64 tokens of 384 channels: 8.7 against
+  // 22.4 us for the launch).
+  const size_t pstride = (size_t)nblk * kBlock;
+  const size_t n_pe = (size_t)T * (kVec ? C >> 2 : C);
+  for (size_t j = (size_t)blk * kBlock + threadIdx.x; j < n_pe; j += pstride) {
+    if (kVec) {
+      const int C4 = C >> 2;
+      const int t = (int)(j / C4), c4 = (int)(j % C4);
+      float4 *p = reinterpret_cast<float4 *>(dwpe) + j;
+      const float4 *g = reinterpret_cast<const float4 *>(dout) + (size_t)t * C4 + c4;
+      float4 acc = *p;
+      for (int b0 = 0; b0 < B; b0 += kB) {
+        float4 d[kB];
+#pragma unroll
+        for (int q = 0; q < kB; q++)
+          if (b0 + q < B) d[q] = g[(size_t)(b0 + q) * T * C4];
+#pragma unroll
+        for (int q = 0; q < kB; q++)
+          if (b0 + q < B) {
+            acc.x += d[q].x; acc.y += d[q].y; acc.z += d[q].z; acc.w += d[q].w;
+          }
+      }
+      *p = acc;
+    } else {
+      const int t = (int)(j / C), c = (int)(j % C);
+      float acc = dwpe[j];
+      for (int b0 = 0; b0 < B; b0 += kB) {
+        float d[kB];
+#pragma unroll
+        for (int q = 0; q < kB; q++)
+          if (b0 + q < B) d[q] = dout[((size_t)(b0 + q) * T + t) * C + c];
+#pragma unroll
+        for (int q = 0; q < kB; q++)
+          if (b0 + q < B) acc += d[q];
+      }
+      dwpe[j] = acc;
+    }
+  }
+}
+
 // K1: insert the chunk's rows; blocks past the insert range run dwpe, kB rows
 // of a (t, c) entry in flight.
 template <bool kVec, int kB>
@@ -252,51 +303,7 @@ __global__ __launch_bounds__(kBlock) void k_enc_bwd_insert(EncTable tb, EncShare
     }
     return;
   }
-  // dwpe[t, c] += dout[b, t, c] for b = 0..B-1, in order, kB rows in flight.
-  // dout is read with ordinary (cached) loads: K2 reads the same rows again,
-  // and finds part of them in the cache (K2 15.8 -> 14.3 us at 8,192 x 768).
-  // Each dwpe thread takes two (t, c) entries, one after the other, so half
-  // as many dwpe workgroups stream at once and the inserts' round trips are
-  // delayed less (25.6 -> 24.8 us per call at 8,192 x 768). Large batches of
-  // short sequences have few entries of many rows: they take one channel per
-  // thread and 32 rows in flight (128 x 64 tokens of 384 channels: 8.7 against
-  // 22.4 us for the launch).
-  const size_t pstride = (size_t)(gridDim.x - ins_blocks) * kBlock;
-  const size_t n_pe = (size_t)T * (kVec ? C >> 2 : C);
-  for (size_t j = (size_t)(blockIdx.x - ins_blocks) * kBlock + threadIdx.x; j < n_pe; j += pstride) {
-    if (kVec) {
-      const int C4 = C >> 2;
-      const int t = (int)(j / C4), c4 = (int)(j % C4);
-      float4 *p = reinterpret_cast<float4 *>(dwpe) + j;
-      const float4 *g = reinterpret_cast<const float4 *>(dout) + (size_t)t * C4 + c4;
-      float4 acc = *p;
-      for (int b0 = 0; b0 < B; b0 += kB) {
-        float4 d[kB];
-#pragma unroll
-        for (int q = 0; q < kB; q++)
-          if (b0 + q < B) d[q] = g[(size_t)(b0 + q) * T * C4];
-#pragma unroll
-        for (int q = 0; q < kB; q++)
-          if (b0 + q < B) {
-            acc.x += d[q].x; acc.y += d[q].y; acc.z += d[q].z; acc.w += d[q].w;
-          }
-      }
-      *p = acc;
-    } else {
-      const int t = (int)(j / C), c = (int)(j % C);
-      float acc = dwpe[j];
-      for (int b0 = 0; b0 < B; b0 += kB) {
-        float d[kB];
-#pragma unroll
-        for (int q = 0; q < kB; q++)
-          if (b0 + q < B) d[q] = dout[((size_t)(b0 + q) * T + t) * C + c];
-#pragma unroll
-        for (int q = 0; q < kB; q++)
-          if (b0 + q < B) acc += d[q];
-      }
-      dwpe[j] = acc;
-    }
-  }
+  add_dwpe<kVec, kB>(dwpe, dout, (int)blockIdx.x - ins_blocks, (int)gridDim.x - ins_blocks, B, T, C);
 }
 
 __device__ __forceinline__ void wave_lds_sync() {
@@ -830,6 +837,84 @@ __global__ __launch_bounds__(kBlkWaves * kWave) void k_enc_bwd_blocked(EncTable 
   }
 }
 
+// The whole backward of at most kFew rows in one launch, without the bucket
+// table, whose three launches' latencies made up the time of a small batch: per
+// call 256 rows of 27 tokens x 384 5.6 against 17.0 us, 512 of 50,257 x 768 5.8
+// against 16, 1,024 of 27 x 384 13.4 against 20.5, 1,024 of 50,257 x 768 11.3
+// against 16.7 (every wavefront's look at every id grows with the square of the
+// rows: more rows go to the table). One wavefront per (row, 64 channels)
+// reads every id and leaves if an earlier row has its row's token; the first
+// row's wavefront lists the token's rows, ascending, in LDS and adds them in the
+// order of the mode (blocks of kBlkRows and then the block sums, or one chain),
+// up to 64 rows in flight, one channel per lane. The workgroups past them add
+// dwpe. Ids out of range match no row's token, before or after their own
+// wavefront has replaced them.
+template <int kFew>
+__global__ __launch_bounds__(kBlock) void k_enc_bwd_few(float *__restrict__ dwte, float *dwpe, const float *dout,
+                                                        int *inp, IdCheck ids, int nslices, int add_blocks, int exact,
+                                                        int B, int T, int C) {
+  if ((int)blockIdx.x >= add_blocks) {
+    add_dwpe<false, 16>(dwpe, dout, (int)blockIdx.x - add_blocks, (int)gridDim.x - add_blocks, B, T, C);
+    return;
+  }
+  __shared__ unsigned short list[kWavesPerBlock][kFew];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int n = B * T;
+  const int item = __builtin_amdgcn_readfirstlane((int)blockIdx.x * kWavesPerBlock + (int)(threadIdx.x >> 6));
+  const int i = item / nslices, slice = item - i * nslices;
+  if (i >= n) return;
+  unsigned short *mine = list[threadIdx.x >> 6];
+  int all[kFew / kWave];
+#pragma unroll
+  for (int j = 0; j < kFew / kWave; j++) {
+    const int r = j * kWave + lane;
+    all[j] = inp[min(r, n - 1)];
+    if (r >= n) all[j] = -1;
+  }
+  int tok = inp[i];
+  if ((unsigned)tok > ids.last && lane == 0 && slice == 0) check_id(tok, inp, i, ids);
+  tok = __builtin_amdgcn_readfirstlane(tok);
+  if (tok < 0 || (unsigned)tok > ids.last) return;  // skipped
+  const u64 below = (lane == 0) ? 0ull : (~0ull >> (kWave - lane));
+  int cnt = 0;
+#pragma unroll
+  for (int j = 0; j < kFew / kWave; j++) {
+    const bool hit = all[j] == tok;
+    const u64 mk = __ballot(hit);
+    if (cnt == 0 && mk && j * kWave + (__ffsll((long long)mk) - 1) < i) return;  // not the token's first row
+    if (hit) mine[cnt + __popcll(mk & below)] = (unsigned short)(j * kWave + lane);
+    cnt += __popcll(mk);
+  }
+  wave_lds_sync();
+  const int c = slice * kWave + lane;
+  const bool on = c < C;
+  const unsigned cc = on ? (unsigned)c : 0u;  // a valid column for the lanes past C, never stored
+  float *const dst = dwte + (size_t)tok * C + cc;
+  float acc = *dst, t = -0.0f;  // t: the sum of the finished blocks
+  for (int k = 0; k < cnt; k += kBlkRows) {
+    const int nr = min(kBlkRows, cnt - k);  // the same for the whole wavefront
+    if (k > 0 && !exact) {
+      t += acc;
+      acc = -0.0f;
+    }
+    const int id = mine[k + min(lane, nr - 1)];
+    const auto rows = [&](auto most) {
+      constexpr int kN = decltype(most)::value;
+      float v[kN];
+#pragma unroll
+      for (int q = 0; q < kN; q++) v[q] = (dout + (size_t)(unsigned)__builtin_amdgcn_readlane(id, q) * C)[cc];
+#pragma unroll
+      for (int q = 0; q < kN; q++)
+        if (q < nr) acc += v[q];
+    };
+    if (nr <= 4) rows(std::integral_constant<int, 4>{});
+    else if (nr <= 16) rows(std::integral_constant<int, 16>{});
+    else rows(std::integral_constant<int, kBlkRows>{});
+  }
+  if (cnt > kBlkRows && !exact) acc = t + acc;
+  if (on) *dst = acc;
+}
+
 __global__ void k_enc_init(EncTable t) {
   const int h = blockIdx.x * kBlock + threadIdx.x;
   if (h < kTableMax) t.slot[h] = kFree;
@@ -986,6 +1071,17 @@ int launch_encoder_backward(float *dwte, float *dwpe, const float *dout, int *in
   const bool vec = (C & 3) == 0 && aligned16(dwte) && aligned16(dwpe) && aligned16(dout);
   const int nslices = (C + kWave - 1) / kWave;
   const bool blocked = !encoder_exact();
+  if (BT <= 1024) {
+    const int add_blocks = (int)grid_for((size_t)BT * nslices, kWavesPerBlock);
+    const int pe_blocks = (int)grid_for((size_t)T * C, kBlock);
+    const auto few = [&](auto k) {
+      launch(k, dim3(add_blocks + pe_blocks), dim3(kBlock), 0, dwte, dwpe, dout, inp, ids, nslices, add_blocks,
+             blocked ? 0 : 1, B, T, C);
+    };
+    if (BT <= 512) few(k_enc_bwd_few<512>);
+    else few(k_enc_bwd_few<1024>);
+    return check_launch("encoder_backward");
+  }
   for (int c0 = 0; c0 < BT; c0 += kChunk) {
     const int n = BT - c0 < kChunk ? BT - c0 : kChunk;
     int tsize = 64, lg = 6;
