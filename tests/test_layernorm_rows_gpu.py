@@ -73,3 +73,40 @@ def test_writes_nothing_outside(gpu, rows, C, offset):
     for k, t in bufs.items():
         lo, hi = 16 + offset, 16 + offset + t.numel() - 64
         assert bool((t[:lo] == guard).all()) and bool((t[hi:] == guard).all()), k
+
+
+@pytest.mark.parametrize("rows,C,offset", [(256, 384, 0), (512, 768, 1), (300, 771, 0), (128, 8192, 0), (513, 768, 0)])
+@pytest.mark.parametrize("pair", [False, True])
+def test_in_place(gpu, rows, C, offset, pair):
+    """dinp (for the pair dx) over dout: a row's terms are those of dout as it was. Another kernel may
+    take the call then, with its sums in another order, so the results agree to the bound of two orders
+    of 32-bit additions (n terms: n 2^-24 of their absolute sum, each)."""
+    g = gen.rng(rows * 13 + C)
+    n = rows * C
+    x, dout, w, b, dw0, db0 = (gen.normal(g, (k,)) for k in (n, n, C, C, C, C))
+    tx, tw, tb = (put(a, offset) for a in (x, w, b))
+    out, m, r = (put(np.zeros(k, np.float32), offset) for k in (n, rows, rows))
+    gpu.layernorm_forward(out, m, r, tx, tw, tb, 1, rows, C)
+    got = []
+    for same in (True, False):
+        do = put(dout, offset)
+        over = do if same else put(dout, offset)
+        di, dy = put(np.zeros(n, np.float32), offset), put(dout, offset)
+        dw, db = put(dw0, offset), put(db0, offset)
+        if pair:
+            gpu.layernorm_residual_backward(di, dw, db, over, dy, do, tx, tw, m, r, 1, rows, C)
+        else:
+            gpu.layernorm_backward(over, dw, db, do, tx, tw, m, r, 1, rows, C)
+        got.append([host(t) for t in (over, di, dy, dw, db)])
+    u, d64 = 2.0 ** -24, dout.reshape(rows, C).astype(np.float64)
+    r64 = host(r).astype(np.float64)[:, None]
+    xhat = np.abs((x.reshape(rows, C) - host(m).astype(np.float64)[:, None]) * r64)
+    dn = np.abs(d64 * w)
+    # of a row's two means, and of the rounding of dinp's and dx's own few terms
+    means = 2 * C * u * (dn.mean(1, keepdims=True) + xhat * (dn * xhat).mean(1, keepdims=True))
+    row = r64 * (means + 16 * u * (dn + dn.mean(1, keepdims=True) + xhat * (dn * xhat).mean(1, keepdims=True)))
+    row += 8 * u * np.abs(d64)
+    for k, bound in ((0, row), (1, row), (2, row), (3, 2 * rows * u * ((np.abs(d64) * xhat).sum(0) + np.abs(dw0))),
+                     (4, 2 * rows * u * (np.abs(d64).sum(0) + np.abs(db0)))):
+        diff = np.abs(got[0][k].astype(np.float64) - got[1][k]).reshape(bound.shape)
+        assert (diff <= bound).all(), k

@@ -922,11 +922,10 @@ __global__ void k_enc_init(EncTable t) {
 }
 
 // ---- id guard -----------------------------------------------------------------
-// The Python binding checks token and target ids with this kernel before a
-// kernel indexes a table with them: ids outside [0, bound) are replaced in
-// place by `fill` and recorded in the per-device error word, which
-// ugk_synchronize reports. Ids in range are not written. No host round trip,
-// so the calls stay asynchronous (and capturable).
+// ugk_ids_guard: ids outside [0, bound) are replaced in place by `fill` and
+// recorded in the per-device error word, which ugk_synchronize reports. Ids in
+// range are not written. No host round trip, so the calls stay asynchronous
+// (and capturable). The _checked ops do the same as they read the ids (IdCheck).
 }  // namespace
 }  // namespace ugk
 

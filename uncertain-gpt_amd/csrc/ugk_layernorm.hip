@@ -1953,6 +1953,20 @@ void set_layernorm_tail(int on) { g_ln_tail.store(on ? 1 : 0); }
 int layernorm_tail() { return g_ln_tail.load(); }
 
 namespace {
+// Whether a backward writes over its own dout or inp (dinp = dout, say). The
+// kernels above read all of a row before they write it, and take its column
+// terms from the registers; the column workgroups beside the small path's rows
+// would read it at any time.
+bool in_place(const float *dinp, const float *dx, const float *dy, const float *dout, const float *inp, size_t n) {
+  const auto overlap = [n](const float *a, const float *b) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return a && (x < y ? y - x : x - y) < n * sizeof(float);
+  };
+  for (const float *w : {dinp, dx, dy})
+    if (overlap(w, dout) || overlap(w, inp)) return true;
+  return false;
+}
+
 // The backward of small_path(rows, C); without the columns if dweight is null.
 template <bool kRes>
 void launch_ln_bwd_small(float *dinp, float *dweight, float *dbias, float *dx, float *dy, const float *dout,
@@ -2005,7 +2019,7 @@ int launch_layernorm_backward_partials(float *dinp, float *partial, float *dweig
     return set_error(UGK_EINVAL, "layernorm_backward: unsupported dinp mode %d with assign %d", dinp_mode,
                      (int)assign_res);
   const LnBwdMode md{dinp_mode != kDinpNone, dinp_mode == kDinpRw, assign_res, dx == dy};
-  if (small_path(rows, C)) {
+  if (small_path(rows, C) && !(dweight && in_place(dinp, dx, dy, dout, inp, (size_t)rows * C))) {
     if (res)
       launch_ln_bwd_small<true>(dinp, dweight, dbias, dx, dy, dout, inp, weight, mean, rstd, rows, C, md);
     else
@@ -2052,7 +2066,7 @@ int launch_layernorm_reduce(const LnReduceJob *jobs, int njobs, int rows, int C)
     LnReduceBatch b{};
     const int n = njobs - j0 < kMaxReduceJobs ? njobs - j0 : kMaxReduceJobs;
     for (int k = 0; k < n; k++) b.job[k] = jobs[j0 + k];
-    if (small_path(rows, C)) {
+    if (b.job[0].nblk == 0) {  // no partial rows; the same for all jobs of a batch
       launch(k_ln_small_cols_batch, dim3(grid_for((size_t)C, kSmallCols), n), dim3(kBlock), 0, b, rows, C);
       continue;
     }
