@@ -108,14 +108,17 @@ __global__ __launch_bounds__(kBlock) void k_enc_fwd_row(float4 *__restrict__ out
   const int lane = threadIdx.x & (kWave - 1);
   const int bt = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
   if (bt >= BT) return;
-  const size_t ot = (size_t)checked_id(inp, bt, ids) * C4, op = (size_t)(bt % T) * C4;
+  // the row of wpe loads while the id is on its way (the check's branch would
+  // otherwise hold it back)
+  int id = inp[bt];
+  const size_t op = (size_t)(bt % T) * C4;
   float4 x[V], y[V];
 #pragma unroll
-  for (int v = 0; v < V; v++) {
-    const int c = min(lane + v * kWave, C4 - 1);
-    x[v] = wte[ot + c];
-    y[v] = wpe[op + c];
-  }
+  for (int v = 0; v < V; v++) y[v] = wpe[op + min(lane + v * kWave, C4 - 1)];
+  id = check_id(__builtin_amdgcn_readfirstlane(id), inp, bt, ids);
+  const size_t ot = (size_t)id * C4;
+#pragma unroll
+  for (int v = 0; v < V; v++) x[v] = wte[ot + min(lane + v * kWave, C4 - 1)];
   float4 *o = out + (size_t)bt * C4;
 #pragma unroll
   for (int v = 0; v < V; v++) {

@@ -228,13 +228,19 @@ __global__ __launch_bounds__(kBlock) void k_enc_ln_fwd_vec(float *__restrict__ e
   if (row0 >= rows) return;
   const Cols<V, false> cl(lane, kWave, C);
   float4 xa[V], ya[V];
-  {
-    const float *te = wte + (size_t)checked_id(inp, row0, ids) * C, *pe = wpe + (size_t)(row0 % T) * C;
+  // every id of the wavefront, and the first row of wpe, on their way before the
+  // first check: its branch, and the store in it, would hold back what comes after
+  int id[RPW];
 #pragma unroll
-    for (int v = 0; v < V; v++) {
-      xa[v] = ld4(te + cl.at[v]);
-      ya[v] = ld4(pe + cl.at[v]);
-    }
+  for (int k = 0; k < RPW; k++) id[k] = inp[min(row0 + k, rows - 1)];
+  {
+    const float *pe = wpe + (size_t)(row0 % T) * C;
+#pragma unroll
+    for (int v = 0; v < V; v++) ya[v] = ld4(pe + cl.at[v]);
+    const int ix = check_id(__builtin_amdgcn_readfirstlane(id[0]), inp, row0, ids);
+    const float *te = wte + (size_t)ix * C;
+#pragma unroll
+    for (int v = 0; v < V; v++) xa[v] = ld4(te + cl.at[v]);
   }
 #pragma unroll
   for (int k = 0; k < RPW; k++) {
@@ -243,7 +249,8 @@ __global__ __launch_bounds__(kBlock) void k_enc_ln_fwd_vec(float *__restrict__ e
     float4 xb[V], yb[V];
     if (k + 1 < RPW) {
       const int nx = min(row + 1, rows - 1);
-      const float *te = wte + (size_t)checked_id(inp, nx, ids) * C, *pe = wpe + (size_t)(nx % T) * C;
+      const int ix = check_id(__builtin_amdgcn_readfirstlane(id[k + 1 < RPW ? k + 1 : k]), inp, nx, ids);
+      const float *te = wte + (size_t)ix * C, *pe = wpe + (size_t)(nx % T) * C;
 #pragma unroll
       for (int v = 0; v < V; v++) {
         xb[v] = ld4(te + cl.at[v]);
