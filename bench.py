@@ -104,11 +104,16 @@ KERNEL_KEYS = [  # (substring of the rocprof kernel name, short name)
     ("k_ln_bwd_reduce_batch", "layernorm_backward (batched column sums)"),
     ("k_ln_bwd_reduce", "layernorm_backward (reduce)"),
     ("k_ln_fwd_exact", "layernorm_forward (exact form)"),
+    ("k_ln_bwd_wide", "layernorm_backward (main, a workgroup per row)"),
+    ("k_ln_bwd_small", "layernorm_backward (few rows)"),
+    ("k_ln_small_cols_batch", "layernorm_backward (few rows, batched columns)"),
+    ("k_ln_fwd_wide", "layernorm_forward (a workgroup per row)"),
     ("k_ln_bwd_exact", "layernorm_backward (exact form: rows and columns in one launch)"),
     ("k_ln_fwd_vec", "layernorm_forward"),
     ("k_enc_fwd_vec", "encoder_forward"),
     ("k_enc_fwd_row", "encoder_forward"),
     ("k_enc_ln_fwd_vec", "encoder_layernorm_forward"),
+    ("k_enc_bwd_few", "encoder_backward (few rows, one launch)"),
     ("k_enc_bwd_insert", "encoder_backward (insert + dwpe)"),
     ("k_enc_bwd_add", "encoder_backward (add)"),
     ("k_enc_bwd_large", "encoder_backward (large buckets, exact order)"),
@@ -128,8 +133,7 @@ KERNEL_KEYS = [  # (substring of the rocprof kernel name, short name)
     ("k_softmax_xent<", "softmax_crossentropy"),
     ("k_softmax_xent_split<", "softmax_crossentropy"),
     ("k_softmax_stats", "softmax_crossentropy (row statistics)"),
-    ("k_softmax_norm_rows", "softmax_crossentropy (exact form, normalise)"),
-    ("k_softmax_norm", "softmax_crossentropy (normalise)"),
+    ("k_softmax_norm_rows", "softmax_crossentropy (normalise)"),
     ("k_softmax_rowmax", "softmax_crossentropy (exact form, row max)"),
     ("k_softmax_sum_exact", "softmax_crossentropy (exact form, serial row sums)"),
     ("k_xent_softmax_bwd_flat4<true>", "crossentropy_softmax_backward (dlogits not read)"),
