@@ -75,7 +75,8 @@ def test_writes_nothing_outside(gpu, rows, C, offset):
         assert bool((t[:lo] == guard).all()) and bool((t[hi:] == guard).all()), k
 
 
-@pytest.mark.parametrize("rows,C,offset", [(256, 384, 0), (512, 768, 1), (300, 771, 0), (128, 8192, 0), (513, 768, 0)])
+@pytest.mark.parametrize("rows,C,offset", [(256, 384, 0), (512, 768, 1), (300, 771, 0), (128, 8192, 0), (513, 768, 0),
+                                           (70, 3, 0), (40, 8193, 0)])
 @pytest.mark.parametrize("pair", [False, True])
 def test_in_place(gpu, rows, C, offset, pair):
     """dinp (for the pair dx) over dout: a row's terms are those of dout as it was. Another kernel may

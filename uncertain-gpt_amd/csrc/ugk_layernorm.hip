@@ -1067,8 +1067,10 @@ __global__ __launch_bounds__(kBlock) void k_ln_bwd_small(float *__restrict__ din
 }
 
 // Backward for the rows that no kernel above takes (C < 4 or beyond 8,192).
-// Phase 1: one wavefront per row writes
-// dinp. Phase 2: thread-per-channel column sums over the workgroup's rows.
+// Phase 1: thread-per-channel column sums over the workgroup's rows. Phase 2:
+// one wavefront per row writes dinp. The columns come first because both read
+// dout and inp from memory, and dinp may be one of them: a row's terms are
+// those of the arrays as they were.
 __global__ __launch_bounds__(kBlock) void k_ln_bwd_scalar(float *dinp, float *partial, const float *dout,
                                                           const float *inp, const float *weight,
                                                           const float *mean, const float *rstd, int rows,
@@ -1078,6 +1080,19 @@ __global__ __launch_bounds__(kBlock) void k_ln_bwd_scalar(float *dinp, float *pa
   const float Cf = (float)C;
   const int row0 = blockIdx.x * rpb;
   const int row1 = min(row0 + rpb, rows);
+  float *prow = partial + (size_t)blockIdx.x * 2 * C;
+  for (int c = threadIdx.x; c < C; c += kBlock) {
+    float g = 0.0f, b = 0.0f;
+    for (int row = row0; row < row1; row++) {
+      const float dy = dout[(size_t)row * C + c];
+      const float xhat = (inp[(size_t)row * C + c] - mean[row]) * rstd[row];
+      b += dy;
+      g += dy * xhat;
+    }
+    prow[c] = g;
+    prow[C + c] = b;
+  }
+  __syncthreads();
   for (int row = row0 + wave; row < row1; row += kWavesPerBlock) {
     const float *x = inp + (size_t)row * C;
     const float *dy = dout + (size_t)row * C;
@@ -1098,18 +1113,6 @@ __global__ __launch_bounds__(kBlock) void k_ln_bwd_scalar(float *dinp, float *pa
       const float dnorm = dy[c] * weight[c];
       dx[c] += r * (dnorm - dnm - xhat * dnxm);
     }
-  }
-  float *prow = partial + (size_t)blockIdx.x * 2 * C;
-  for (int c = threadIdx.x; c < C; c += kBlock) {
-    float g = 0.0f, b = 0.0f;
-    for (int row = row0; row < row1; row++) {
-      const float dy = dout[(size_t)row * C + c];
-      const float xhat = (inp[(size_t)row * C + c] - mean[row]) * rstd[row];
-      b += dy;
-      g += dy * xhat;
-    }
-    prow[c] = g;
-    prow[C + c] = b;
   }
 }
 
