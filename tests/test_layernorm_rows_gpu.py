@@ -75,13 +75,8 @@ def test_writes_nothing_outside(gpu, rows, C, offset):
         assert bool((t[:lo] == guard).all()) and bool((t[hi:] == guard).all()), k
 
 
-@pytest.mark.parametrize("rows,C,offset", [(256, 384, 0), (512, 768, 1), (300, 771, 0), (128, 8192, 0), (513, 768, 0),
-                                           (70, 3, 0), (40, 8193, 0)])
-@pytest.mark.parametrize("pair", [False, True])
-def test_in_place(gpu, rows, C, offset, pair):
-    """dinp (for the pair dx) over dout: a row's terms are those of dout as it was. Another kernel may
-    take the call then, with its sums in another order, so the results agree to the bound of two orders
-    of 32-bit additions (n terms: n 2^-24 of their absolute sum, each)."""
+def in_place_results(gpu, rows, C, offset, pair):
+    """dinp (for the pair dx) over dout, and in an array of its own: [dinp or dx, dinp, dy, dweight, dbias] of both."""
     g = gen.rng(rows * 13 + C)
     n = rows * C
     x, dout, w, b, dw0, db0 = (gen.normal(g, (k,)) for k in (n, n, C, C, C, C))
@@ -99,9 +94,20 @@ def test_in_place(gpu, rows, C, offset, pair):
         else:
             gpu.layernorm_backward(over, dw, db, do, tx, tw, m, r, 1, rows, C)
         got.append([host(t) for t in (over, di, dy, dw, db)])
+    return got, x, dout, w, dw0, db0, host(m), host(r)
+
+
+@pytest.mark.parametrize("rows,C,offset", [(256, 384, 0), (512, 768, 1), (300, 771, 0), (128, 8192, 0), (513, 768, 0),
+                                           (70, 3, 0), (40, 8193, 0)])
+@pytest.mark.parametrize("pair", [False, True])
+def test_in_place(gpu, rows, C, offset, pair):
+    """dinp (for the pair dx) over dout: a row's terms are those of dout as it was. Another kernel may
+    take the call then, with its sums in another order, so the results agree to the bound of two orders
+    of 32-bit additions (n terms: n 2^-24 of their absolute sum, each)."""
+    got, x, dout, w, dw0, db0, m, r = in_place_results(gpu, rows, C, offset, pair)
     u, d64 = 2.0 ** -24, dout.reshape(rows, C).astype(np.float64)
-    r64 = host(r).astype(np.float64)[:, None]
-    xhat = np.abs((x.reshape(rows, C) - host(m).astype(np.float64)[:, None]) * r64)
+    r64 = r.astype(np.float64)[:, None]
+    xhat = np.abs((x.reshape(rows, C) - m.astype(np.float64)[:, None]) * r64)
     dn = np.abs(d64 * w)
     # of a row's two means, and of the rounding of dinp's and dx's own few terms
     means = 2 * C * u * (dn.mean(1, keepdims=True) + xhat * (dn * xhat).mean(1, keepdims=True))
@@ -111,3 +117,17 @@ def test_in_place(gpu, rows, C, offset, pair):
                      (4, 2 * rows * u * (np.abs(d64).sum(0) + np.abs(db0)))):
         diff = np.abs(got[0][k].astype(np.float64) - got[1][k]).reshape(bound.shape)
         assert (diff <= bound).all(), k
+
+
+@pytest.mark.parametrize("rows,C,offset", [(256, 384, 0), (300, 771, 1), (70, 3, 0)])
+@pytest.mark.parametrize("pair", [False, True])
+def test_in_place_exact(gpu, rows, C, offset, pair):
+    """The exact mode in place: the same bits."""
+    prev = gpu.layernorm_exact()
+    gpu.set_layernorm_exact(True)
+    try:
+        got = in_place_results(gpu, rows, C, offset, pair)[0]
+    finally:
+        gpu.set_layernorm_exact(prev)
+    for k, (a, c) in enumerate(zip(*got)):
+        assert_bits(a, c, str(k))

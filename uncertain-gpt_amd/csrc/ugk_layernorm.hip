@@ -1859,16 +1859,38 @@ int launch_layernorm_forward_exact(float *out, float *mean, float *rstd, const f
   return check_launch("layernorm_forward (exact)");
 }
 
+namespace {
+// Whether a backward writes over its own dout or inp (dinp = dout, say). A
+// row's terms are then those of the arrays as they were, so the kernels whose
+// column workgroups run beside the row workgroups (few rows, and the exact
+// form) cannot take the call as it is. The others read all that a workgroup's
+// column terms need of its rows before they write them.
+bool in_place(const float *dinp, const float *dx, const float *dy, const float *dout, const float *inp, size_t n) {
+  const auto overlap = [n](const float *a, const float *b) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return a && (x < y ? y - x : x - y) < n * sizeof(float);
+  };
+  for (const float *w : {dinp, dx, dy})
+    if (overlap(w, dout) || overlap(w, inp)) return true;
+  return false;
+}
+}  // namespace
+
 int launch_layernorm_backward_exact(float *dinp, float *dweight, float *dbias, const float *dout, const float *inp,
                                     const float *weight, const float *mean, const float *rstd, int rows, int C) {
   if (rows == 0 || C == 0) return 0;
   const bool vec = C % 4 == 0 && aligned16(dinp) && aligned16(dout) && aligned16(inp) && aligned16(weight);
   const int nrow = (int)grid_for((size_t)rows, kExRows), ncol = (int)grid_for((size_t)C, kExCols);
-  const dim3 grid(nrow + ncol), block(kExThreads);
-  if (vec)
-    launch(k_ln_bwd_exact<true>, grid, block, 0, dinp, dweight, dbias, dout, inp, weight, mean, rstd, rows, C, nrow);
-  else
-    launch(k_ln_bwd_exact<false>, grid, block, 0, dinp, dweight, dbias, dout, inp, weight, mean, rstd, rows, C, nrow);
+  const auto go = [&](int blocks, int row_blocks) {
+    launch(vec ? k_ln_bwd_exact<true> : k_ln_bwd_exact<false>, dim3(blocks), dim3(kExThreads), 0, dinp, dweight, dbias,
+           dout, inp, weight, mean, rstd, rows, C, row_blocks);
+  };
+  if (in_place(dinp, nullptr, nullptr, dout, inp, (size_t)rows * C)) {
+    go(ncol, 0);  // all columns before any row is written
+    go(nrow, nrow);
+  } else {
+    go(nrow + ncol, nrow);
+  }
   return check_launch("layernorm_backward (exact)");
 }
 
@@ -1963,20 +1985,6 @@ void set_layernorm_tail(int on) { g_ln_tail.store(on ? 1 : 0); }
 int layernorm_tail() { return g_ln_tail.load(); }
 
 namespace {
-// Whether a backward writes over its own dout or inp (dinp = dout, say). The
-// kernels above read all of a row before they write it, and take its column
-// terms from the registers; the column workgroups beside the small path's rows
-// would read it at any time.
-bool in_place(const float *dinp, const float *dx, const float *dy, const float *dout, const float *inp, size_t n) {
-  const auto overlap = [n](const float *a, const float *b) {
-    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
-    return a && (x < y ? y - x : x - y) < n * sizeof(float);
-  };
-  for (const float *w : {dinp, dx, dy})
-    if (overlap(w, dout) || overlap(w, inp)) return true;
-  return false;
-}
-
 // The backward of small_path(rows, C); without the columns if dweight is null.
 template <bool kRes>
 void launch_ln_bwd_small(float *dinp, float *dweight, float *dbias, float *dx, float *dy, const float *dout,
