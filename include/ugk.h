@@ -542,7 +542,9 @@ int ugk_gpt2_layers_forward(float *acts, const float *params, const int *inputs,
  * LayerNorm dweight/dbias column sums are completed by one launch at the end,
  * and their partial rows live in the workspace's LayerNorm region meanwhile,
  * so the dense callbacks must not call ugk_layernorm_backward or
- * ugk_layernorm_residual_backward (the other entry points use other regions). */
+ * ugk_layernorm_residual_backward (the other entry points use other regions).
+ * A callback may overwrite the gradient of a LayerNorm whose backward has run:
+ * with callbacks, no later launch reads it. */
 int ugk_gpt2_layers_backward(float *grads, float *grads_acts, const float *acts,
                              const float *params, const int *inputs,
                              ugk_config cfg, const ugk_dense_ops *ops);

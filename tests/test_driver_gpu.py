@@ -350,6 +350,52 @@ def test_step_driver_dense_callbacks(gpu, B, T, C, NH, L):
     assert d.calls[len(fwd):] == bwd, "backward dense calls differ from gpt2_kernels.cuh:852-891"
 
 
+class ReusingDense(TorchDense):
+    """TorchDense whose attention backward also overwrites the gradients that the LayerNorm backwards
+    before it have read for the last time: the final LayerNorm's, this block's ln2o and the block above's
+    lno."""
+
+    def bind_backward(self, grads, grads_acts, lay=None):
+        super().bind_backward(grads, grads_acts)
+        self.lay, self.l = lay, lay.L - 1
+
+    def attn_bwd(self, dqkv, dout, qkv, B, T, C):
+        TorchDense.attn_bwd(dqkv, dout, qkv, B, T, C)
+        lay, ga = self.lay, self.bases["grads_acts"]
+        done = [lay.a["flo"], lay.aa(self.l, "ln2o")] + ([lay.aa(self.l + 1, "lno")] if self.l + 1 < lay.L else [])
+        for off in done:
+            ga[off:off + lay.NB] = 3.0
+        self.l -= 1
+
+
+@pytest.mark.parametrize("B,T", [(2, 32), (2, 520)])
+@pytest.mark.parametrize("zeroed", [False, True])
+def test_callbacks_may_reuse_finished_gradients(gpu, B, T, zeroed):
+    """A LayerNorm's dweight and dbias are those of its gradient when its backward runs, at few rows and
+    at many, whatever a later dense op does with that buffer."""
+    C, V, NH, L = 384, 27, 6, 3
+    prev = gpu.lib.ugk_get_stream()
+    gpu.set_stream(torch.cuda.current_stream().cuda_stream)
+    try:
+        cfg = gpu.Config(B=B, T=T, C=C, V=V, NH=NH, maxT=T, L=L)
+        lay = Layout(B, T, C, V, T, L)
+        params, acts, inputs, ga0 = make_inputs(gpu, lay, seed=5 + T)
+        gpu.gpt2_layers_forward(acts, params, inputs, cfg)
+        ga0[lay.a["blk0"]:lay.a["blk0"] + L * lay.a["bstride"]] = 0
+        fn = gpu.gpt2_layers_backward_zeroed if zeroed else gpu.gpt2_layers_backward
+        out = []
+        for dense in (TorchDense(params, acts), ReusingDense(params, acts)):
+            g, ga = torch.zeros(lay.p["total"], device=DEV), ga0.clone()
+            dense.bind_backward(g, ga, *([lay] if isinstance(dense, ReusingDense) else []))
+            fn(g, ga, acts, params, inputs, cfg, dense.ops)
+            torch.cuda.synchronize()
+            dense.raise_errors()
+            out.append(g)
+        bits_equal_dev(out[1], out[0], "parameter gradients")
+    finally:
+        gpu.set_stream(prev)
+
+
 def test_step_driver_reports_a_failing_callback(gpu):
     """A dense op that returns nonzero stops the driver with an error naming the op."""
     B, T, C, NH, L, V = 1, 8, 64, 2, 1, 11

@@ -999,6 +999,9 @@ int layers_backward(const char *fn, bool zeroed, float *grads, float *grads_acts
   std::vector<LnReduceJob> jobs;
   jobs.reserve((size_t)nln);
   const bool exact = layernorm_exact() != 0;
+  // A dense callback may reuse the gradient of a LayerNorm whose backward has
+  // run: every sum over it is then taken before the next callback.
+  const LnCols cols = ops ? kColsPartial : kColsLater;
   auto ln_bwd = [&](float *dinp, float *dw, float *db, float *dx, float *dy, const float *dout, const float *inp,
                     const float *w, const float *mean, const float *rstd, int dinp_mode = kDinpRead) -> int {
     if (exact)  // the reference's LayerNorm backward then residual_backward, each in its own order
@@ -1011,8 +1014,8 @@ int layers_backward(const char *fn, bool zeroed, float *grads, float *grads_acts
     // in gpt2_backward nothing reads it after the residual_backward that
     // splits it into dx and dy (res1 of every block and each block's resa).
     if (int e = timed(dx ? UGK_OP_LAYERNORM_RESIDUAL_BACKWARD_MAIN : UGK_OP_LAYERNORM_BACKWARD_MAIN, [&] {
-          return launch_layernorm_backward_partials(dinp, part, nullptr, nullptr, dx, dy, dout, inp, w, mean, rstd,
-                                                    M, C, slot_rows, &nblk, dx ? dinp_mode : kDinpRw,
+          return launch_layernorm_backward_partials(dinp, part, cols, nullptr, nullptr, dx, dy, dout, inp, w, mean,
+                                                    rstd, M, C, slot_rows, &nblk, dx ? dinp_mode : kDinpRw,
                                                     zeroed && dx != nullptr);
         }))
       return e;

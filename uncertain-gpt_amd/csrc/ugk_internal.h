@@ -250,14 +250,18 @@ int launch_layernorm_residual_backward(float *dinp, float *dweight, float *dbias
 // non-null, applies residual_backward(dx, dy, dinp)) and *nblk partial rows
 // of the dweight/dbias column sums to `partial`; launch_layernorm_reduce then
 // adds each job's column totals into its dweight/dbias, many jobs per launch.
-// (Few rows have no partial rows: *nblk = 0, and the main pass adds the column
-// totals itself if dweight and dbias are given, else launch_layernorm_reduce
-// takes them from the job's dout, inp, mean and rstd.)
+// Few rows have no partial rows of their own; `cols` says what becomes of their
+// column totals.
 struct LnReduceJob {
   const float *partial;
   float *dweight, *dbias;
   int nblk;
   const float *dout, *inp, *mean, *rstd;
+};
+enum LnCols {
+  kColsAdd,      // the main pass adds them to dweight and dbias (*nblk = 0)
+  kColsPartial,  // the main pass stores them as one partial row (*nblk = 1)
+  kColsLater     // launch_layernorm_reduce takes them from the job's dout, inp, mean and rstd (*nblk = 0)
 };
 // What a fused LayerNorm -> residual backward does with its dinp (the
 // float4 path; the scalar path always reads and writes it):
@@ -270,10 +274,10 @@ enum LnDinp {
 // scalar path up to 512). With dx non-null, dinp_mode says what happens to
 // dinp, and assign_res takes dx and dy as +0.0 instead of reading them (float4
 // path; the scalar path reads and writes everything).
-int launch_layernorm_backward_partials(float *dinp, float *partial, float *dweight, float *dbias, float *dx, float *dy,
-                                       const float *dout, const float *inp, const float *weight, const float *mean,
-                                       const float *rstd, int rows, int C, int max_blocks, int *nblk,
-                                       int dinp_mode = kDinpRw, bool assign_res = false);
+int launch_layernorm_backward_partials(float *dinp, float *partial, LnCols cols, float *dweight, float *dbias,
+                                       float *dx, float *dy, const float *dout, const float *inp,
+                                       const float *weight, const float *mean, const float *rstd, int rows, int C,
+                                       int max_blocks, int *nblk, int dinp_mode = kDinpRw, bool assign_res = false);
 int launch_layernorm_reduce(const LnReduceJob *jobs, int njobs, int rows, int C);
 // The per-op LayerNorm backward (launch_layernorm_residual_backward_into) on
 // the float4 path finishes its column sums in its main launch (1) or in a

@@ -946,14 +946,17 @@ __global__ __launch_bounds__(W * kWave) void k_ln_bwd_wide(float *__restrict__ d
 
 // Backward of few rows without partial rows. What bounds it is latency: a
 // launch, one round trip to memory, the reductions. A call's first workgroups
-// finish dweight and dbias by themselves, 16 columns each, reading x and dout
+// sum dweight and dbias by themselves, 16 columns each, reading x and dout
 // once more (they are in the caches): 64 groups of consecutive rows, each
 // added in row order, every eighth group together, then those eight sums as a
-// tree, then onto the arrays' values.
-// The others write dinp (and the residual targets), P wavefronts per row, every
-// row's loads in flight at once. The step driver's calls have the row
-// workgroups alone (ncol = 0), and one launch at its end takes the columns of
-// all its LayerNorms (k_ln_small_cols_batch). Per call, against the two launches
+// tree, then onto the arrays' values, or (add false) as the call's only partial
+// row. The others write dinp (and the residual targets), P wavefronts per row,
+// every row's loads in flight at once. The step driver's calls leave the columns
+// out (ncol = 0) where nothing but its own kernels runs before its end, and one
+// launch there takes them for all its LayerNorms (k_ln_small_cols_batch: 154
+// against 175 us for a step of 13 LayerNorms of 256 x 384); with dense
+// callbacks, which may write to the gradients again, each call sums its own, as
+// a partial row. Per call, against the two launches
 // of the larger shapes' kernels: 256 x 384 3.6 against 8.6 us, 512 x 768 4.1
 // against 9.7, 1,024 x 384 6.4 against 9.0. Too few column workgroups then
 // stream too much each: 768 x 768 10.1 against 10.4, 1,024 x 768 13.4 against
@@ -964,7 +967,7 @@ constexpr int kSmallCols = 16, kSmallSlots = kSmallCols / 4, kSmallGroups = kBlo
 __device__ __forceinline__ void ln_small_cols(float (*red)[2][kSmallCols], int blk, float *__restrict__ dweight,
                                               float *__restrict__ dbias, const float *__restrict__ dout,
                                               const float *__restrict__ inp, const float *__restrict__ mean,
-                                              const float *__restrict__ rstd, int rows, int C) {
+                                              const float *__restrict__ rstd, int rows, int C, bool add) {
   const int l = threadIdx.x % kSmallSlots, g = threadIdx.x / kSmallSlots;
   const Cols<1, true> cl(blk * kSmallSlots + l, 0, C);
   // the adder thread's column: component col % 4 of slot col / 4, if that is the slot's own
@@ -972,7 +975,7 @@ __device__ __forceinline__ void ln_small_cols(float (*red)[2][kSmallCols], int b
   const Cols<1, true> cc(blk * kSmallSlots + col / 4, 0, C);
   const bool adder = (int)threadIdx.x < 2 * kSmallCols && cc.own(0, col & 3);
   float *const dst = (which ? dbias : dweight) + cc.at[0] + (col & 3);
-  const float prev = adder ? *dst : 0.0f;
+  const float prev = adder && add ? *dst : -0.0f;
   float4 ag = zero4(), ab = zero4();
   const int J = (rows + kSmallGroups - 1) / kSmallGroups;
   const int j0 = min(g * J, rows), j1 = min(j0 + J, rows);
@@ -1016,11 +1019,11 @@ __global__ __launch_bounds__(kBlock) void k_ln_bwd_small(float *__restrict__ din
                                                          const float *__restrict__ weight,
                                                          const float *__restrict__ mean,
                                                          const float *__restrict__ rstd, int rows, int C, int ncol,
-                                                         float *__restrict__ rdx, float *__restrict__ rdy,
+                                                         int add, float *__restrict__ rdx, float *__restrict__ rdy,
                                                          LnBwdMode md) {
   __shared__ __align__(16) float red[kSmallGroups][2][kSmallCols];
   if ((int)blockIdx.x < ncol) {
-    ln_small_cols(red, blockIdx.x, dweight, dbias, dout, inp, mean, rstd, rows, C);
+    ln_small_cols(red, blockIdx.x, dweight, dbias, dout, inp, mean, rstd, rows, C, add != 0);
     return;
   }
   constexpr int T = kWavesPerBlock / P;  // rows per workgroup
@@ -1176,7 +1179,7 @@ __global__ __launch_bounds__(kRedCols * kRedGroups) void k_ln_bwd_reduce_batch(L
 __global__ __launch_bounds__(kBlock) void k_ln_small_cols_batch(LnReduceBatch b, int rows, int C) {
   __shared__ __align__(16) float red[kSmallGroups][2][kSmallCols];
   const LnReduceJob &j = b.job[blockIdx.y];
-  ln_small_cols(red, blockIdx.x, j.dweight, j.dbias, j.dout, j.inp, j.mean, j.rstd, rows, C);
+  ln_small_cols(red, blockIdx.x, j.dweight, j.dbias, j.dout, j.inp, j.mean, j.rstd, rows, C, true);
 }
 
 // Which kernels take rows of C channels, at any alignment: one wavefront per
@@ -1985,17 +1988,18 @@ void set_layernorm_tail(int on) { g_ln_tail.store(on ? 1 : 0); }
 int layernorm_tail() { return g_ln_tail.load(); }
 
 namespace {
-// The backward of small_path(rows, C); without the columns if dweight is null.
+// The backward of small_path(rows, C): the column totals are added to dweight
+// and dbias, or stored there (add false), or left out (dweight null).
 template <bool kRes>
-void launch_ln_bwd_small(float *dinp, float *dweight, float *dbias, float *dx, float *dy, const float *dout,
+void launch_ln_bwd_small(float *dinp, float *dweight, float *dbias, bool add, float *dx, float *dy, const float *dout,
                          const float *inp, const float *weight, const float *mean, const float *rstd, int rows, int C,
                          LnBwdMode md) {
   const bool wide = row_in_block(C);
   const int ncol = dweight ? (int)grid_for((size_t)C, kSmallCols) : 0;
   const int nrow = wide ? rows : (int)grid_for((size_t)rows, kWavesPerBlock);
   const auto go = [&](auto k) {
-    launch(k, dim3(ncol + nrow), dim3(kBlock), 0, dinp, dweight, dbias, dout, inp, weight, mean, rstd, rows, C, ncol, dx,
-           dy, md);
+    launch(k, dim3(ncol + nrow), dim3(kBlock), 0, dinp, dweight, dbias, dout, inp, weight, mean, rstd, rows, C, ncol,
+           add ? 1 : 0, dx, dy, md);
   };
   switch (slots_of(C, wide ? kBlock : kWave)) {
 #define UGK_LN_SMALL(v)                              \
@@ -2026,10 +2030,10 @@ void launch_ln_bwd_wide(float *dinp, float *partial, float *dx, float *dy, const
 }
 }  // namespace
 
-int launch_layernorm_backward_partials(float *dinp, float *partial, float *dweight, float *dbias, float *dx, float *dy,
-                                       const float *dout, const float *inp, const float *weight, const float *mean,
-                                       const float *rstd, int rows, int C, int max_blocks, int *nblk, int dinp_mode,
-                                       bool assign_res) {
+int launch_layernorm_backward_partials(float *dinp, float *partial, LnCols cols, float *dweight, float *dbias,
+                                       float *dx, float *dy, const float *dout, const float *inp,
+                                       const float *weight, const float *mean, const float *rstd, int rows, int C,
+                                       int max_blocks, int *nblk, int dinp_mode, bool assign_res) {
   *nblk = 0;
   if (rows == 0) return 0;
   const bool res = dx != nullptr;
@@ -2037,11 +2041,14 @@ int launch_layernorm_backward_partials(float *dinp, float *partial, float *dweig
     return set_error(UGK_EINVAL, "layernorm_backward: unsupported dinp mode %d with assign %d", dinp_mode,
                      (int)assign_res);
   const LnBwdMode md{dinp_mode != kDinpNone, dinp_mode == kDinpRw, assign_res, dx == dy};
-  if (small_path(rows, C) && !(dweight && in_place(dinp, dx, dy, dout, inp, (size_t)rows * C))) {
+  if (small_path(rows, C) && !in_place(dinp, dx, dy, dout, inp, (size_t)rows * C)) {
+    const bool add = cols == kColsAdd;
+    float *const g = add ? dweight : cols == kColsPartial ? partial : nullptr, *const b = add ? dbias : partial + C;
     if (res)
-      launch_ln_bwd_small<true>(dinp, dweight, dbias, dx, dy, dout, inp, weight, mean, rstd, rows, C, md);
+      launch_ln_bwd_small<true>(dinp, g, b, add, dx, dy, dout, inp, weight, mean, rstd, rows, C, md);
     else
-      launch_ln_bwd_small<false>(dinp, dweight, dbias, dx, dy, dout, inp, weight, mean, rstd, rows, C, md);
+      launch_ln_bwd_small<false>(dinp, g, b, add, dx, dy, dout, inp, weight, mean, rstd, rows, C, md);
+    if (cols == kColsPartial) *nblk = 1;
     return check_launch("layernorm_backward");
   }
   if (row_in_wave(C)) {
@@ -2080,16 +2087,21 @@ int launch_layernorm_backward_partials(float *dinp, float *partial, float *dweig
 }
 
 int launch_layernorm_reduce(const LnReduceJob *jobs, int njobs, int rows, int C) {
-  for (int j0 = 0; j0 < njobs; j0 += kMaxReduceJobs) {
-    LnReduceBatch b{};
-    const int n = njobs - j0 < kMaxReduceJobs ? njobs - j0 : kMaxReduceJobs;
-    for (int k = 0; k < n; k++) b.job[k] = jobs[j0 + k];
-    if (b.job[0].nblk == 0) {  // no partial rows; the same for all jobs of a batch
-      launch(k_ln_small_cols_batch, dim3(grid_for((size_t)C, kSmallCols), n), dim3(kBlock), 0, b, rows, C);
-      continue;
+  LnReduceBatch sums{}, cols{};  // jobs with partial rows, and without
+  int nsums = 0, ncols = 0;
+  for (int j = 0; j < njobs; j++) {
+    const bool later = jobs[j].nblk == 0, last = j + 1 == njobs;
+    if (later) cols.job[ncols++] = jobs[j];
+    else sums.job[nsums++] = jobs[j];
+    if (nsums == kMaxReduceJobs || (last && nsums > 0)) {
+      launch(k_ln_bwd_reduce_batch, dim3(grid_for((size_t)2 * C, kRedCols), nsums), dim3(kRedCols * kRedGroups), 0,
+             sums, C);
+      nsums = 0;
     }
-    launch(k_ln_bwd_reduce_batch, dim3(grid_for((size_t)2 * C, kRedCols), n), dim3(kRedCols * kRedGroups), 0, b,
-           C);
+    if (ncols == kMaxReduceJobs || (last && ncols > 0)) {
+      launch(k_ln_small_cols_batch, dim3(grid_for((size_t)C, kSmallCols), ncols), dim3(kBlock), 0, cols, rows, C);
+      ncols = 0;
+    }
   }
   return check_launch("layernorm_backward (column sums)");
 }
@@ -2115,8 +2127,8 @@ int launch_layernorm_residual_backward_into(float *partial, int max_blocks, floa
     return check_launch("layernorm_backward");
   }
   int nblk;
-  if (int e = launch_layernorm_backward_partials(dinp, partial, dweight, dbias, dx, dy, dout, inp, weight, mean, rstd,
-                                                 rows, C, max_blocks, &nblk))
+  if (int e = launch_layernorm_backward_partials(dinp, partial, kColsAdd, dweight, dbias, dx, dy, dout, inp, weight,
+                                                 mean, rstd, rows, C, max_blocks, &nblk))
     return e;
   if (nblk == 0) return 0;  // the launch has added the column sums
   const LnReduceJob job{partial, dweight, dbias, nblk, dout, inp, mean, rstd};
