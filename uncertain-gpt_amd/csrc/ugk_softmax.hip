@@ -375,8 +375,11 @@ __global__ __launch_bounds__(kBwdThreads) void k_xent_softmax_bwd_flat4(float *_
   const size_t r0 = row_of(i, (size_t)V, inv_v);
   const bool two = r0 + 1 < (size_t)rows;
   const int id0 = targets[r0], id1 = targets[two ? r0 + 1 : r0];
-  const size_t t0 = r0 * (size_t)V + (size_t)check_id(id0, targets, r0, ids);
-  const size_t t1 = two ? (r0 + 1) * (size_t)V + (size_t)check_id(id1, targets, r0 + 1, ids) : ~(size_t)0;
+  const auto element = [&](size_t r, int id) {  // a target outside its row is no element
+    id = check_id(id, targets, r, ids);
+    return (unsigned)id < (unsigned)V ? r * (size_t)V + (unsigned)id : ~(size_t)0;
+  };
+  const size_t t0 = element(r0, id0), t1 = two ? element(r0 + 1, id1) : ~(size_t)0;
   st_nt4(dlogits + i, make_float4(xent_grad(d.x, p.x, i == t0 || i == t1, dloss),
                                   xent_grad(d.y, p.y, i + 1 == t0 || i + 1 == t1, dloss),
                                   xent_grad(d.z, p.z, i + 2 == t0 || i + 2 == t1, dloss),
