@@ -131,3 +131,30 @@ def test_in_place_exact(gpu, rows, C, offset, pair):
         gpu.set_layernorm_exact(prev)
     for k, (a, c) in enumerate(zip(*got)):
         assert_bits(a, c, str(k))
+
+
+def test_column_sums_no_further_from_64_bits(gpu):
+    """dweight and dbias of many rows off a 16-byte boundary (959 partial rows) are no further from the
+    64-bit sums than the same terms in chains of 32 rows, 16 groups of 30 such chains and the groups,
+    each in order, as the lane loops would add them."""
+    rows, C, offset = 15345, 768, 2
+    g = gen.rng(3)
+    n = rows * C
+    x, dout, w = (gen.normal(g, (k,)) for k in (n, n, C))
+    tx, tw, td, tb = (put(a, offset) for a in (x, w, dout, w))
+    out, m, r, di, dw, db = (put(np.zeros(k, np.float32), offset) for k in (n, rows, rows, n, C, C))
+    gpu.layernorm_forward(out, m, r, tx, tw, tb, 1, rows, C)
+    gpu.layernorm_backward(di, dw, db, td, tx, tw, m, r, 1, rows, C)
+    x2, d2, m2, r2 = x.reshape(rows, C), dout.reshape(rows, C), host(m)[:, None], host(r)[:, None]
+    terms = {"dweight": ((x2 - m2) * r2 * d2, (x2.astype(np.float64) - m2) * r2 * d2, host(dw)),
+             "dbias": (d2, d2.astype(np.float64), host(db))}
+    for k, (t, t64, got) in terms.items():
+        pad = np.zeros((16 * 30 * 32, C), np.float32)
+        pad[:rows] = t
+        rung = pad.reshape(16, 30, 32, C)
+        for axis in (2, 1, 0):  # np.add.accumulate over a leading axis is a float32 chain in order
+            rung = np.add.accumulate(rung, axis=axis, dtype=np.float32).take(-1, axis=axis)
+        want = t64.sum(0)
+        off = [np.linalg.norm(a - want) / np.linalg.norm(want) for a in (got, rung)]
+        print(k, off)
+        assert off[0] <= off[1], k

@@ -16,7 +16,7 @@
 // wavefront adds the dweight/dbias terms of its rows, in row order, in
 // registers; after one barrier the workgroup's W per-wavefront sums are added
 // column by column in wavefront order into one partial row per workgroup, and
-// a second, small kernel adds the partial rows in index order into
+// a second, small kernel adds the partial rows in a fixed order into
 // dweight/dbias. No atomics, so the result is identical run to run.
 //
 // The float4 paths take rows at any alignment (gfx950 accepts a 16-byte access
@@ -360,8 +360,7 @@ __device__ __forceinline__ float4 zero4() { return make_float4(0.0f, 0.0f, 0.0f,
 // column sums themselves, in the order the column-sum kernel uses (so with the
 // same bits): the partial rows form kTailGroups groups of J = ceil(nblk / 16)
 // consecutive rows; the last workgroup of a group to finish adds the group's
-// rows in index order, starting from +0.0f, and writes the sum over the
-// group's first row; the last group to finish adds the group sums in group
+// rows (RowChains) and writes the sum over the group's first row; the last group to finish adds the group sums in group
 // order (an empty group adds +0.0f) into dweight/dbias.
 //
 // Publishing without a cache write-back: the rows and group sums are written
@@ -401,6 +400,23 @@ __device__ __forceinline__ void st_dev(float *p, float v) {
 __device__ __forceinline__ float ld_dev(float *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// A column's sum over the partial rows of a group: four chains, every fourth
+// row to each, in index order, then the chains in pairs. One chain of up to 64
+// rows is further from the 64-bit sums the more partial rows a call has:
+// dweight of 15,345 x 768 (959 partial rows) was 1.75e-7 off with one chain (in
+// the 2-norm, relative) and is 1.33e-7 off with four, at the same time.
+struct RowChains {
+  float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  // the next rows of the group, `left` of them up to its end
+  template <int N>
+  __device__ __forceinline__ void add(const float (&v)[N], int left) {
+    static_assert(N % 4 == 0, "a batch starts on the first chain");
+#pragma unroll
+    for (int q = 0; q < N; q++) s[q & 3] += q < left ? v[q] : -0.0f;
+  }
+  __device__ __forceinline__ float sum() const { return (s[0] + s[1]) + (s[2] + s[3]); }
+};
+
 // Called by every thread of a workgroup (NT threads) after it has written its
 // partial row with st_dev.
 template <int NT>
@@ -421,15 +437,14 @@ __device__ __forceinline__ void ln_bwd_tail(float *partial, int nblk, int C, flo
   __syncthreads();
   if (!last) return;
   for (int c = threadIdx.x; c < C2; c += NT) {
-    float acc = 0.0f;
+    RowChains acc;
     for (int b = j0; b < j1; b += kBatch) {
       float v[kBatch];
 #pragma unroll
       for (int q = 0; q < kBatch; q++) v[q] = ld_dev(partial + (size_t)min(b + q, j1 - 1) * C2 + c);
-#pragma unroll
-      for (int q = 0; q < kBatch; q++) acc += b + q < j1 ? v[q] : -0.0f;
+      acc.add(v, j1 - b);
     }
-    st_dev(partial + (size_t)j0 * C2 + c, acc);
+    st_dev(partial + (size_t)j0 * C2 + c, acc.sum());
   }
   wait_stores();
   __syncthreads();
@@ -1121,7 +1136,7 @@ __global__ __launch_bounds__(kBlock) void k_ln_bwd_scalar(float *dinp, float *pa
 
 // Column totals of the partial rows, added to dweight (columns [0,C)) and
 // dbias (columns [C,2C)). Workgroup: 32 columns x 16 groups; group k sums the
-// partial rows [k*J, (k+1)*J), J = ceil(nblk/16) <= 64, in index order, 32
+// partial rows [k*J, (k+1)*J), J = ceil(nblk/16) <= 64 (RowChains), 32
 // loads in flight per batch; the 16 group sums are then added in group order.
 // 32 columns rather than 64 spread one LayerNorm's totals over twice the
 // workgroups (48 at C = 768): the per-op backward at 8,192 x 768 took 22.3-22.6
@@ -1145,15 +1160,14 @@ __device__ __forceinline__ void ln_bwd_reduce_tile(float *dweight, float *dbias,
   // after them (one memory round trip fewer at the end)
   float* const dst = col < C ? dweight + col : dbias + (cc - C);
   const float prev = g == 0 && col < C2 ? *dst : 0.0f;
-  float acc = 0.0f;
+  RowChains acc;
   for (int b = j0; b < j1; b += kRedBatch) {
     float v[kRedBatch];
 #pragma unroll
     for (int q = 0; q < kRedBatch; q++) v[q] = partial[(size_t)min(b + q, j1 - 1) * C2 + cc];
-#pragma unroll
-    for (int q = 0; q < kRedBatch; q++) acc += b + q < j1 ? v[q] : -0.0f;
+    acc.add(v, j1 - b);
   }
-  red[g][cl] = acc;
+  red[g][cl] = acc.sum();
   __syncthreads();
   if (g == 0 && col < C2) {
     float t = red[0][cl];
