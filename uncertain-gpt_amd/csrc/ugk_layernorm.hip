@@ -971,12 +971,11 @@ __global__ __launch_bounds__(W * kWave) void k_ln_bwd_wide(float *__restrict__ d
 // launch there takes them for all its LayerNorms (k_ln_small_cols_batch: 154
 // against 175 us for a step of 13 LayerNorms of 256 x 384); with dense
 // callbacks, which may write to the gradients again, each call sums its own, as
-// a partial row. Per call, against the two launches
-// of the larger shapes' kernels: 256 x 384 3.6 against 8.6 us, 512 x 768 4.1
-// against 9.7, 1,024 x 384 6.4 against 9.0. Too few column workgroups then
-// stream too much each: 768 x 768 10.1 against 10.4, 1,024 x 768 13.4 against
-// 9.9 (8 or 32 columns a workgroup, and longer batches, moved that by 2 us at
-// most), hence small_path.
+// a partial row. Per call, captured and cold, against the two launches of the
+// larger shapes' kernels: 256 x 384 3.8 against 7.6 us, 512 x 768 6.4 against
+// 10.3, 640 x 384 4.9 against 8.2. With more rows the few column workgroups
+// stream too much each (8 or 32 columns a workgroup, and longer batches, moved
+// that by 2 us at most), hence small_path.
 constexpr int kSmallCols = 16, kSmallSlots = kSmallCols / 4, kSmallGroups = kBlock / kSmallSlots, kSmallBatch = 4;
 
 __device__ __forceinline__ void ln_small_cols(float (*red)[2][kSmallCols], int blk, float *__restrict__ dweight,
@@ -1301,11 +1300,25 @@ void wide_shape(int rows, int max_blocks, int *nblk, int *rpw) {
   *nblk = (rows + *rpw - 1) / *rpw;
 }
 
-// The backward without partial rows (k_ln_bwd_small, which has the timings on
-// both sides of the line).
-bool small_path(int rows, int C) {
+// The backward without partial rows (k_ln_bwd_small). The lines are where it
+// meets the two launches, captured and cold, the plain backward and the pair:
+//   up to 512 rows      of 1,024 channels 8.3 against 8.3 and 9.6 against 10.3
+//                       us, 768 6.4 against 10.3, but 1,280 8.8 against 8.3;
+//                       beyond 1,536 the two launches are slower again: 2,048
+//                       9.1 against 10.2, 256 x 4,096 7.8 against 11.9;
+//   up to 1,024, cols'  1,024 x 256 6.6 against 7.5, 640 x 384 4.9 against
+//   arrays aligned      8.2, but 1,024 x 320 10.8 against 8.3, 896 x 320 8.5
+//                       against 8.3;
+//   the same, at other  768 x 256 6.4 against 7.5 and 9.4 against 8.1, but
+//   addresses or widths 896 x 256 10.7 against 7.6, 640 x 384 9.0 against 8.4
+//                       (the column workgroups' 64 bytes of a row then lie in
+//                       two lines as often as not).
+bool small_path(int rows, int C, const float *dout, const float *inp) {
   if (!row_in_wave(C) && !row_in_block(C)) return false;
-  return rows <= 512 ? (size_t)rows * C <= ((size_t)1 << 20) : rows <= 1024 && C <= 384;
+  const size_t n = (size_t)rows * C;
+  if (rows <= 512) return n <= ((size_t)1 << 19) || (C > 1536 && n <= ((size_t)1 << 20));
+  const bool aligned = (C & 3) == 0 && aligned16(dout) && aligned16(inp);
+  return rows <= 1024 && n <= (size_t)(aligned ? 4 : 3) << 16;
 }
 
 // Rows per wavefront of the fused forward: two while one wavefront per row
@@ -2002,7 +2015,7 @@ void set_layernorm_tail(int on) { g_ln_tail.store(on ? 1 : 0); }
 int layernorm_tail() { return g_ln_tail.load(); }
 
 namespace {
-// The backward of small_path(rows, C): the column totals are added to dweight
+// The backward of small_path: the column totals are added to dweight
 // and dbias, or stored there (add false), or left out (dweight null).
 template <bool kRes>
 void launch_ln_bwd_small(float *dinp, float *dweight, float *dbias, bool add, float *dx, float *dy, const float *dout,
@@ -2055,7 +2068,7 @@ int launch_layernorm_backward_partials(float *dinp, float *partial, LnCols cols,
     return set_error(UGK_EINVAL, "layernorm_backward: unsupported dinp mode %d with assign %d", dinp_mode,
                      (int)assign_res);
   const LnBwdMode md{dinp_mode != kDinpNone, dinp_mode == kDinpRw, assign_res, dx == dy};
-  if (small_path(rows, C) && !in_place(dinp, dx, dy, dout, inp, (size_t)rows * C)) {
+  if (small_path(rows, C, dout, inp) && !in_place(dinp, dx, dy, dout, inp, (size_t)rows * C)) {
     const bool add = cols == kColsAdd;
     float *const g = add ? dweight : cols == kColsPartial ? partial : nullptr, *const b = add ? dbias : partial + C;
     if (res)
@@ -2131,7 +2144,7 @@ int launch_layernorm_residual_backward_into(float *partial, int max_blocks, floa
       return e;
     return res ? launch_residual_backward(dx, dy, dinp, (size_t)rows * C) : 0;
   }
-  if (layernorm_tail() && row_in_wave(C) && (C & 3) == 0 && !small_path(rows, C)) {
+  if (layernorm_tail() && row_in_wave(C) && (C & 3) == 0 && !small_path(rows, C, dout, inp)) {
     if (res)
       launch_ln_bwd_vec<true, kDinpRw, false>(dinp, partial, dout, inp, weight, mean, rstd, rows, C, dx, dy,
                                               max_blocks, true, dweight, dbias);
