@@ -590,6 +590,12 @@ __global__ __launch_bounds__(W * kWave, MINW) void k_ln_bwd_vec(
     }
 #pragma unroll
     for (int q = 0; q < R; q++) {
+      // The plain backward waits for dinp's loads here, once. Left to itself the
+      // compiler waits before each slot's store, counting the stores before it as
+      // if they were loads (8,192 x 2,048 59.1 against 57.7 us, 16,384 x 384 23.6
+      // against 22.9, 1,100 x 257 8.7 against 8.0; the pair, with more to wait
+      // for, is the slower for it at 8,192 x 2,048: 111 against 108).
+      if (q == 0 && !kRes) __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
       const bool live = q < nr;  // rows past nr repeat row nr-1: computed, neither stored nor summed
       const float dnm = s1[q] / Cf, dnxm = s2[q] / Cf;
 #pragma unroll
