@@ -39,6 +39,15 @@ def test_few_rows(gpu, oracle, B, T, C, V):
     enc_case(gpu, oracle, B, T, C, V, gen.tokens_zipf(gen.rng(B + T), B * T, V), B * T + C, reps=2)
 
 
+@pytest.mark.parametrize("rows,C", [(1024, 768), (1024, 772), (1000, 1100), (1024, 1600), (1024, 1601), (601, 2650),
+                                    (512, 3201), (30, 16448)])
+@pytest.mark.parametrize("V", [27, 50257])
+def test_few_rows_of_many_channels(gpu, oracle, rows, C, V):
+    """One, two and three slices of 64 channels per wavefront, the last group of them not full, and
+    one row slice more than the one launch takes."""
+    enc_case(gpu, oracle, 1, rows, C, V, gen.tokens_zipf(gen.rng(C), rows, V), rows + C, modes=("blocked",))
+
+
 @pytest.mark.parametrize("rows", [8191, 8192, 8193, 20500])
 def test_one_frequent_token(gpu, oracle, rows):
     inp = np.zeros(rows, np.int32)

@@ -844,8 +844,7 @@ __global__ __launch_bounds__(kBlkWaves * kWave) void k_enc_bwd_blocked(EncTable 
 // table, whose three launches' latencies made up the time of a small batch: per
 // call 256 rows of 27 tokens x 384 5.6 against 17.0 us, 512 of 50,257 x 768 5.8
 // against 16, 1,024 of 27 x 384 13.4 against 20.5, 1,024 of 50,257 x 768 11.3
-// against 16.7 (every wavefront's look at every id grows with the square of the
-// rows: more rows go to the table). One wavefront per (row, 64 channels)
+// against 16.7. One wavefront per row and group of `per` slices of 64 channels
 // reads every id and leaves if an earlier row has its row's token; the first
 // row's wavefront lists the token's rows, ascending, in LDS and adds them in the
 // order of the mode (blocks of kBlkRows and then the block sums, or one chain),
@@ -854,8 +853,8 @@ __global__ __launch_bounds__(kBlkWaves * kWave) void k_enc_bwd_blocked(EncTable 
 // wavefront has replaced them.
 template <int kFew>
 __global__ __launch_bounds__(kBlock) void k_enc_bwd_few(float *__restrict__ dwte, float *dwpe, const float *dout,
-                                                        int *inp, IdCheck ids, int nslices, int add_blocks, int exact,
-                                                        int B, int T, int C) {
+                                                        int *inp, IdCheck ids, int per, int ngroups, int add_blocks,
+                                                        int exact, int B, int T, int C) {
   if ((int)blockIdx.x >= add_blocks) {
     add_dwpe<false, 16>(dwpe, dout, (int)blockIdx.x - add_blocks, (int)gridDim.x - add_blocks, B, T, C);
     return;
@@ -864,7 +863,7 @@ __global__ __launch_bounds__(kBlock) void k_enc_bwd_few(float *__restrict__ dwte
   const int lane = threadIdx.x & (kWave - 1);
   const int n = B * T;
   const int item = __builtin_amdgcn_readfirstlane((int)blockIdx.x * kWavesPerBlock + (int)(threadIdx.x >> 6));
-  const int i = item / nslices, slice = item - i * nslices;
+  const int i = item / ngroups, group = item - i * ngroups;
   if (i >= n) return;
   unsigned short *mine = list[threadIdx.x >> 6];
   int all[kFew / kWave];
@@ -875,7 +874,7 @@ __global__ __launch_bounds__(kBlock) void k_enc_bwd_few(float *__restrict__ dwte
     if (r >= n) all[j] = -1;
   }
   int tok = inp[i];
-  if ((unsigned)tok > ids.last && lane == 0 && slice == 0) check_id(tok, inp, i, ids);
+  if ((unsigned)tok > ids.last && lane == 0 && group == 0) check_id(tok, inp, i, ids);
   tok = __builtin_amdgcn_readfirstlane(tok);
   if (tok < 0 || (unsigned)tok > ids.last) return;  // skipped
   const u64 below = (lane == 0) ? 0ull : (~0ull >> (kWave - lane));
@@ -889,33 +888,35 @@ __global__ __launch_bounds__(kBlock) void k_enc_bwd_few(float *__restrict__ dwte
     cnt += __popcll(mk);
   }
   wave_lds_sync();
-  const int c = slice * kWave + lane;
-  const bool on = c < C;
-  const unsigned cc = on ? (unsigned)c : 0u;  // a valid column for the lanes past C, never stored
-  float *const dst = dwte + (size_t)tok * C + cc;
-  float acc = *dst, t = -0.0f;  // t: the sum of the finished blocks
-  for (int k = 0; k < cnt; k += kBlkRows) {
-    const int nr = min(kBlkRows, cnt - k);  // the same for the whole wavefront
-    if (k > 0 && !exact) {
-      t += acc;
-      acc = -0.0f;
+  for (int c0 = group * per * kWave, end = min(c0 + per * kWave, C); c0 < end; c0 += kWave) {
+    const int c = c0 + lane;
+    const bool on = c < C;
+    const unsigned cc = on ? (unsigned)c : 0u;  // a valid column for the lanes past C, never stored
+    float *const dst = dwte + (size_t)tok * C + cc;
+    float acc = *dst, t = -0.0f;  // t: the sum of the finished blocks
+    for (int k = 0; k < cnt; k += kBlkRows) {
+      const int nr = min(kBlkRows, cnt - k);  // the same for the whole wavefront
+      if (k > 0 && !exact) {
+        t += acc;
+        acc = -0.0f;
+      }
+      const int id = mine[k + min(lane, nr - 1)];
+      const auto rows = [&](auto most) {
+        constexpr int kN = decltype(most)::value;
+        float v[kN];
+#pragma unroll
+        for (int q = 0; q < kN; q++) v[q] = (dout + (size_t)(unsigned)__builtin_amdgcn_readlane(id, q) * C)[cc];
+#pragma unroll
+        for (int q = 0; q < kN; q++)
+          if (q < nr) acc += v[q];
+      };
+      if (nr <= 4) rows(std::integral_constant<int, 4>{});
+      else if (nr <= 16) rows(std::integral_constant<int, 16>{});
+      else rows(std::integral_constant<int, kBlkRows>{});
     }
-    const int id = mine[k + min(lane, nr - 1)];
-    const auto rows = [&](auto most) {
-      constexpr int kN = decltype(most)::value;
-      float v[kN];
-#pragma unroll
-      for (int q = 0; q < kN; q++) v[q] = (dout + (size_t)(unsigned)__builtin_amdgcn_readlane(id, q) * C)[cc];
-#pragma unroll
-      for (int q = 0; q < kN; q++)
-        if (q < nr) acc += v[q];
-    };
-    if (nr <= 4) rows(std::integral_constant<int, 4>{});
-    else if (nr <= 16) rows(std::integral_constant<int, 16>{});
-    else rows(std::integral_constant<int, kBlkRows>{});
+    if (cnt > kBlkRows && !exact) acc = t + acc;
+    if (on) *dst = acc;
   }
-  if (cnt > kBlkRows && !exact) acc = t + acc;
-  if (on) *dst = acc;
 }
 
 __global__ void k_enc_init(EncTable t) {
@@ -1022,6 +1023,22 @@ int *ids_error_word() {
   return a.ptr;
 }
 
+namespace {
+// How many slices of 64 channels a wavefront of k_enc_bwd_few takes, 0 if the
+// call goes to the table: up to 1,024 rows, of at most 25,600 row slices (dwords
+// one slice after another there, float4 rows by the table), and as few slices as
+// keep the ids that all wavefronts look at within 12 * 2^20. Captured, few rows
+// against the table, uniform tokens (the worst for it) and Zipf's: 1,024 x 768
+// 12.7 against 13.2 us and 10.4 against 28, 1,024 x 1,600 16.2 against 14.7 and
+// 19.3 against 30.9, 1,024 x 2,048 19.3 against 15.9. With a slice per wavefront
+// 1,024 x 1,600 took 22.7 and 18.3, 1,024 x 1,024 15.8 against now 12.3.
+int few_slices(int n, int nslices) {
+  if (n > 1024 || n * nslices > 25600) return 0;
+  const int most = (12 << 20) / (n * n);  // wavefronts per row
+  return (nslices + most - 1) / most;
+}
+}  // namespace
+
 int launch_encoder_forward(float *out, int *inp, const float *wte, const float *wpe, int B, int T, int C,
                            const IdCheck &ids) {
   const int BT = B * T;
@@ -1073,11 +1090,12 @@ int launch_encoder_backward(float *dwte, float *dwpe, const float *dout, int *in
   const bool vec = (C & 3) == 0 && aligned16(dwte) && aligned16(dwpe) && aligned16(dout);
   const int nslices = (C + kWave - 1) / kWave;
   const bool blocked = !encoder_exact();
-  if (BT <= 1024) {
-    const int add_blocks = (int)grid_for((size_t)BT * nslices, kWavesPerBlock);
+  if (const int per = few_slices(BT, nslices)) {
+    const int ngroups = (nslices + per - 1) / per;
+    const int add_blocks = (int)grid_for((size_t)BT * ngroups, kWavesPerBlock);
     const int pe_blocks = (int)grid_for((size_t)T * C, kBlock);
     const auto few = [&](auto k) {
-      launch(k, dim3(add_blocks + pe_blocks), dim3(kBlock), 0, dwte, dwpe, dout, inp, ids, nslices, add_blocks,
+      launch(k, dim3(add_blocks + pe_blocks), dim3(kBlock), 0, dwte, dwpe, dout, inp, ids, per, ngroups, add_blocks,
              blocked ? 0 : 1, B, T, C);
     };
     if (BT <= 512) few(k_enc_bwd_few<512>);
