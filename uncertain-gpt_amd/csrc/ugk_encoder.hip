@@ -316,19 +316,18 @@ __device__ __forceinline__ void wave_lds_sync() {
 }
 
 // K2, scan workgroup of large bucket j: the chunk's row ids whose slot is the
-// bucket's, in row order, to its share of the pool; 8 int4 loads of slots per
-// thread per round (8,192 slots), the round's matches placed by a workgroup
+// bucket's, in row order, to its share of the pool; kScanQ int4 loads of slots per
+// thread per round (8: 8,192 slots), the round's matches placed by a workgroup
 // prefix over (load, wavefront). Frees the slot after reading its count. What
 // bounds it is its chain of round trips, so the first round's slots load with
 // the bucket's entry, and its matches are counted while one thread reads the
 // bucket's size and takes its share of the pool (6 int4 per round, all of it
 // one after the other: K2 7.9 us at 8,192 rows of 27 tokens, now 5.3).
-constexpr int kScanQ = 8;
-constexpr int kScanRound = kScanQ * kBlock * 4;
+template <int kScanQ>
 __device__ __forceinline__ void scan_large(EncTable tb, EncShared sh, int j, int n) {
   __shared__ int wt[kScanQ * kWavesPerBlock];
   __shared__ int pool_base, bucket_cnt;
-  constexpr int kCounts = kScanQ * kWavesPerBlock;
+  constexpr int kCounts = kScanQ * kWavesPerBlock, kScanRound = kScanQ * kBlock * 4;
   static_assert(kCounts <= kWave, "one lane per (load, wavefront) count");
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x >> 6;
@@ -399,15 +398,15 @@ __device__ __forceinline__ void add_small(EncTable tb, EncShared sh, float *__re
   // Wavefront g takes entry g / R of region g % R (R regions of kBlock
   // entries): the entries of one region (one K1 workgroup's tokens, where a
   // skewed batch puts its frequent tokens early) spread over all workgroups.
-  const int w = sh.list[(gw % R) * kBlock + gw / R];  // this wavefront's slot
+  const int w = __builtin_amdgcn_readfirstlane(sh.list[(gw % R) * kBlock + gw / R]);  // this wavefront's slot
   if (w < 0) return;
   // the slot word and the bucket's first row ids in one round trip (ids past
   // the count are stale and ignored)
   const u64 sw = tb.slot[w];
   const int id_raw = sh.rows[(size_t)w * kCap + (lane & (kCap - 1))];
   asm volatile("" ::"v"(id_raw));  // keeps the compiler from sinking the ids load below the branch
-  const int cnt = slot_cnt(sw);
-  const int tok = slot_tok(sw);
+  const int cnt = __builtin_amdgcn_readfirstlane(slot_cnt(sw));
+  const int tok = __builtin_amdgcn_readfirstlane(slot_tok(sw));
   // A large bucket belongs to its scan workgroup, which may already have
   // freed the slot (the word then reads count 0).
   if (cnt == 0 || cnt > kCap) return;
@@ -474,7 +473,8 @@ __device__ __forceinline__ void add_small(EncTable tb, EncShared sh, float *__re
 #pragma unroll
         for (int q = 0; q < kBatch; q++)
           if (q0 + q < cnt) {
-            const float4 *gr = g + (size_t)mine[q0 + q] * C4 + c0;
+            const unsigned id = __builtin_amdgcn_readfirstlane((int)mine[q0 + q]);
+            const float4 *gr = g + (size_t)id * C4 + c0;
 #pragma unroll
             for (int u = 0; u < kCols; u++)
               if (c0 + u * kWave < C4) d[q][u] = ld_nt(gr + u * kWave);
@@ -517,12 +517,12 @@ __device__ __forceinline__ void add_small(EncTable tb, EncShared sh, float *__re
 // regions exactly). A small bucket's wavefront frees its slot once it has
 // read it.
 template <bool kVec>
-__global__ __launch_bounds__(kBlock, 6) void k_enc_bwd_add(EncTable tb, EncShared sh, float *__restrict__ dwte,
+__global__ __launch_bounds__(kBlock, kVec ? 6 : 8) void k_enc_bwd_add(EncTable tb, EncShared sh, float *__restrict__ dwte,
                                                         const float *__restrict__ dout, int C, int n, int nscan) {
   __shared__ unsigned lds[kWavesPerBlock * kCap];
   if ((int)blockIdx.x < nscan) {
     const int j = (int)blockIdx.x;
-    if (j < tb.counters[1]) scan_large(tb, sh, j, n);  // K1 has counted them: the same value in every thread
+    if (j < tb.counters[1]) scan_large<kVec ? 8 : 6>(tb, sh, j, n);  // K1 has counted them: the same value in every thread
     return;
   }
   const int wave = threadIdx.x >> 6;
