@@ -1,14 +1,16 @@
 """The elementwise kernels' float4 slots start at a cache line of the first output and the elements
-around them go one by one: results at every mix of offsets and at sizes around the edges are those of
-the same call on aligned copies (each element is computed alone, so bit for bit), and nothing outside
-the arrays is written."""
+around them go one by one, and few elements at a misaligned address take a thread each: results at
+every mix of offsets and at sizes around the edges, and on both sides of each operator's line between
+the two, are those of the same call on aligned copies (each element is computed alone, so bit for bit),
+and nothing outside the arrays is written."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
 GUARD = 7.25
-SIZES = [1, 2, 3, 4, 5, 31, 32, 33, 35, 36, 127, 2049, 4096 + 31, 3 * 4096 + 2]
+SIZES = [1, 2, 3, 4, 5, 31, 32, 33, 35, 36, 127, 2049, 4096 + 31, 3 * 4096 + 2, 1 << 19, (1 << 19) + 1, (5 << 17) + 2,
+         (3 << 18) + 3, (1 << 20) + 33]
 
 
 def ops(ugk):
@@ -21,14 +23,17 @@ def ops(ugk):
         "bayes_materialize": (4, lambda a, n: ugk.bayes_materialize(a[0], a[1], a[2], a[3], n)),
         "bayes_sample": (4, lambda a, n: ugk.bayes_sample(a[0], a[1], a[2], a[3], n, 0x5EED, 3)),
         "adamw_update": (4, lambda a, n: ugk.adamw_update(a[0], a[1], a[2], a[3], n, *adam)),
+        "bayes_backward_philox": (4, lambda a, n: ugk.bayes_backward_philox(a[0], a[1], a[2], a[3], n, 0x5EED, 3)),
+        "bbb_step_fused": (8, lambda a, n: ugk.bbb_step_fused(*a, n, 0x5EED, 3, 0.1, 1e-6, 0.3, 0.003, *adam[1:])),
     }
 
 
 @pytest.mark.parametrize("name", ["residual_forward", "residual_backward", "gelu_backward", "bayes_materialize",
-                                  "bayes_sample", "adamw_update"])
+                                  "bayes_sample", "adamw_update", "bayes_backward_philox", "bbb_step_fused"])
 @pytest.mark.parametrize("offsets", [(0, 0, 0, 0), (1, 1, 1, 1), (0, 2, 1, 3), (3, 0, 2, 1), (29, 4, 31, 2)])
 def test_offsets_and_ends(gpu, name, offsets):
     k, call = ops(gpu)[name]
+    offsets = (offsets * 2)[:k]
     g = torch.Generator(device="cuda")
     g.manual_seed(5)
     for n in SIZES:

@@ -64,6 +64,7 @@ template <bool kFast>
 struct BayesSample : MapOp {
   static constexpr int kLoads = 2, kStores = 1;
   static constexpr bool kIndexed = true;
+  static constexpr size_t kEachTo = (size_t)3 << 18;
   static constexpr bool kTable = !kFast;
   static constexpr int kUnroll = 1;
   // eps for all four of a thread's elements while mu and rho load: with the
@@ -110,6 +111,7 @@ template <bool kFast>
 struct BayesBackwardPhilox : MapOp {
   static constexpr int kLoads = 4, kStores = 2;
   static constexpr bool kIndexed = true;
+  static constexpr size_t kEachTo = (size_t)5 << 17;
   // measured best of the map shapes: 512 threads for the glibc-exact form, 1024
   // for the fast one (506 us at 512, 515 at 256, 484 at 1024 over 124.4M)
   static constexpr int kUnroll = 1, kThreads = kFast ? 1024 : 512;
@@ -193,6 +195,7 @@ template <bool kFast>
 struct BbbStepFused : MapOp {
   static constexpr int kLoads = 7, kStores = 8;
   static constexpr bool kIndexed = true;
+  static constexpr size_t kEachTo = ~(size_t)0;
   static constexpr bool kTable = !kFast;
   static constexpr int kUnroll = 1;
   // The fast form fits 8 wavefronts per SIMD in its registers but runs best at

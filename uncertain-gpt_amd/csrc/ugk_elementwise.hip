@@ -97,6 +97,7 @@ struct GeluBwdZero : MapOp {  // loads inp, dout
 
 struct Materialize : MapOp {  // train_bnn.c:831-835; loads mu, rho, eps
   static constexpr int kLoads = 3, kStores = 1;
+  static constexpr size_t kEachTo = (size_t)1 << 20;
   static constexpr int kUnroll = 1, kThreads = 256;  // measured best of the map shapes
   static constexpr bool kTable = true;  // expf's 2^(i/32) table staged in LDS
   __device__ static void apply(const float *ld, float *st, const uint64_t *tab, size_t, Params) {

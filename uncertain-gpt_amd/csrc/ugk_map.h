@@ -10,18 +10,27 @@
 // with and without nt) put nt loads and stores with unroll 1-2 and 256-512
 // threads on top; each operator picks its own (the spread is a few percent).
 //
-// Any address and any n take this path, in one launch. gfx950 accepts a
+// Any n takes this path, in one launch, and any address beyond kEachTo
+// elements. gfx950 accepts a
 // 16-byte access at a 4-byte address, so the slots start at the first element
 // whose address in the first output is a cache line's (full lines are then
 // written there whatever the streams' offsets: 478 against 482 us for a whole
 // block of layer kernels whose arrays are 8 bytes off, with the slots started at
 // element 0 instead), and the up to 31 elements before them and 3 after them
 // are taken one by one by a workgroup of their own, told from the others by a
-// scalar compare. Both were separate paths before: misaligned arrays took
-// dwords (residual forward over 11.8M elements 32 against 22.9 us, its
-// backward 42.3 against 39.0), and a ragged end took a second launch, which cost
-// 4.4-4.8 us per call (six such calls over 11,061,531 parameters: 281 against
-// 268 us).
+// scalar compare. Against dwords for misaligned arrays: residual forward over
+// 11.1M elements 23.0 against 31.6 us, its backward 37.4 against 45.1; against a
+// second launch for a ragged end: 4.4-4.8 us less per call (six such calls over
+// 11,061,531 parameters: 281 against 268 us).
+//
+// Few elements at a misaligned address go one to a thread instead (k_map_each):
+// the chip is not filled then, and a thread with four elements takes longer.
+// The operators whose element is long notice (98,305 elements 8 bytes off:
+// AdamW 3.5 against 5.0 us, materialize 3.1 against 4.4), the others don't
+// either way. Where the two meet is the operator's kEachTo, 1,000,000 elements
+// at most (AdamW 6.1 against 5.7 us at 600,000, materialize 4.8 against 5.5) but for
+// the one-pass update: fifteen misaligned streams of 16-byte accesses from
+// element 0 on are slower at any size (40M elements 543 against 524 us).
 //
 // An operator is a struct with
 //   kLoads, kStores          stream counts;
@@ -36,6 +45,8 @@
 //                            element, which the ops that draw eps are short of
 //                            the cycles for);
 //   apply(ld, st, tab, i, p) the per-element body; i is the element index;
+//   kEachTo                  up to how many elements misaligned arrays take one
+//                            thread per element;
 //   kPre, Pre, pre(i, p)     optionally (kPre true), the part of the body that
 //                            reads no stream (a Philox draw): the kernel
 //                            computes it for all of a thread's elements while
@@ -56,6 +67,7 @@ struct MapOp {
   static constexpr int kThreads = kBlock;
   static constexpr unsigned kLdsReserve = 0;
   static constexpr bool kIndexed = false;
+  static constexpr size_t kEachTo = (size_t)1 << 19;
   static constexpr bool kPre = false;
   struct Pre {};
 };
@@ -143,9 +155,32 @@ __global__ __launch_bounds__(Op::kThreads) void k_map_vec4(Streams<Op> s, size_t
   }
 }
 
+// One element per thread (and more where that would take over kEachBlocks workgroups).
+constexpr unsigned kEachBlocks = 65536;
+template <class Op>
+__global__ __launch_bounds__(kBlock) void k_map_each(Streams<Op> s, size_t n) {
+  __shared__ uint64_t tab[Op::kTable ? 32 : 1];
+  if (Op::kTable) {
+    ugk_exp2_stage(tab);
+    __syncthreads();
+  }
+  for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock)
+    map_one<Op>(s, (ptrdiff_t)i, tab);
+}
+
 template <class Op>
 int run_map(Streams<Op> s, size_t n, const char *name) {
   if (n == 0) return 0;
+  if (n <= Op::kEachTo) {
+    bool aligned = true;
+    for (int l = 0; l < Op::kLoads; l++) aligned = aligned && aligned16(s.ld[l]);
+    for (int o = 0; o < Op::kStores; o++) aligned = aligned && aligned16(s.st[o]);
+    if (!aligned) {
+      const size_t blocks = (n - 1) / kBlock + 1;
+      launch(k_map_each<Op>, dim3(blocks < kEachBlocks ? (unsigned)blocks : kEachBlocks), dim3(kBlock), 0, s, n);
+      return check_launch(name);
+    }
+  }
   size_t lead = Op::kIndexed ? 0 : (0 - ((uintptr_t)s.st[0] >> 2)) & (kLine - 1);
   if (lead > n) lead = n;
   for (int l = 0; l < Op::kLoads; l++) s.ld[l] += lead;
