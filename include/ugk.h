@@ -77,7 +77,8 @@ int ugk_encoder_forward(float *out, const int *inp, const float *wte,
  * captured in a HIP graph and replayed any number of times. New workspace
  * memory is cleared by ugk_set_workspace and ugk_reserve_config, or else by
  * the first call; that first call, if made under graph capture, is refused
- * (UGK_EINVAL) rather than leave the clearing inside the graph alone. */
+ * (UGK_EINVAL) rather than leave the clearing inside the graph alone. (A call
+ * of few rows, up to 1,024, does not use the table; the same holds for it.) */
 int ugk_encoder_backward(float *dwte, float *dwpe, const float *dout,
                          const int *inp, int B, int T, int C);
 
@@ -435,13 +436,18 @@ int ugk_diag_philox(unsigned *out, const unsigned *in, size_t n);
  * to what its access pattern allows. Asynchronous. */
 int ugk_diag_stream(float *buf, size_t n, int nr, int nw, int per_thread, int block);
 /* The partial rows (workgroups) a LayerNorm backward of rows x C writes
- * (fused: the LayerNorm -> residual pair), and the bound the workspace's
- * LayerNorm slots are sized by, which covers every call with at most `rows`
- * rows. Host arithmetic only; no HIP call. */
+ * (fused: the LayerNorm -> residual pair) where its column sums take a second
+ * launch, and the bound the workspace's LayerNorm slots are sized by, which
+ * covers every call with at most `rows` rows. (A call of few rows writes none,
+ * or one in the step driver, unless its dinp, dx or dy overlaps its dout or
+ * inp; its workspace is sized by the same bound.) Host arithmetic only; no
+ * HIP call. */
 int ugk_diag_layernorm_partial_rows(int rows, int C, int fused, int *actual, int *bound);
 /* How the per-op LayerNorm backward entry points (ugk_layernorm_backward,
  * ugk_layernorm_residual_backward, ugk_layernorm_backward_noalloc) finish
- * their dweight/dbias column sums on the float4 path: on 0 (the default) a
+ * their dweight/dbias column sums with C a multiple of 4 up to 2,048 and more
+ * rows than the one-launch form takes (a call of few rows adds them beside its
+ * rows in either mode): on 0 (the default) a
  * second launch adds the partial rows; on 1 the main launch's workgroups add
  * them themselves, the last of each group of rows and then the last group,
  * through device-scope stores and loads and a counter, without an L2

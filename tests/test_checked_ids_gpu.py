@@ -1,5 +1,5 @@
 """GPU: the id check inside the ops' own kernels, over every kernel that reads ids: out-of-range ids (below,
-at and beyond the bound; first, middle and last row) are replaced in place, the others not written, the
+at and beyond the bound; the first two rows, the middle and the last) are replaced in place, the others not written, the
 outputs are those of the replaced ids, and the next synchronize names the op, once."""
 import pytest
 import torch
@@ -12,9 +12,9 @@ def planted(n, V, seed):
     g = torch.Generator(DEV).manual_seed(seed)
     ids = torch.randint(0, V, (n,), device=DEV, dtype=torch.int32, generator=g)
     bad = ids.clone()
-    at = sorted({0, n // 2, n - 1})
+    at = sorted({0, 1, n // 2, n - 1})
     for k, i in enumerate(at):
-        bad[i] = (V, -1, 0x7fffffff)[k]
+        bad[i] = (V, -1, 0x7fffffff, V + 7)[k]
     return g, bad, at
 
 
@@ -60,7 +60,10 @@ def test_head(gpu, rows, V, exact):
         assert same(*d)
 
 
-@pytest.mark.parametrize("B,T,C", [(1, 5, 7), (2, 9, 384), (1, 40, 2052), (20, 3, 64)])
+# few rows; the bucket table, with dwpe of few and of many sequences and rows in a second chunk; the fused
+# forward with two rows per wavefront, an odd number of them
+@pytest.mark.parametrize("B,T,C", [(1, 5, 7), (2, 9, 384), (1, 40, 2052), (20, 3, 64), (5, 257, 384), (20, 60, 30),
+                                   (1, 70001, 16), (3, 1367, 384), (1, 2049, 1600)])
 def test_encoder(gpu, B, T, C):
     V, n = 11, B * T
     g, bad, at = planted(n, V, n + C)

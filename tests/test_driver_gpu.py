@@ -198,6 +198,10 @@ def run_driver_vs_replay(gpu, B, T, C, V, NH, maxT, L, seed, dense_factory=None)
     (2, 32, 384, 27, 0),        # no block: the encoder -> LayerNorm pass writes the final LayerNorm
     (2, 16, 1024, 27, 2),       # four float4 per lane (GPT-2 medium's width)
     (1, 16, 2048, 11, 1),       # eight, the widest row held in registers
+    (2, 520, 384, 27, 2),       # more rows than the few-row backward takes, at two, four, seven
+    (2, 520, 1024, 27, 1),      # and eight float4 per lane
+    (2, 520, 1600, 27, 1),
+    (2, 520, 2048, 11, 1),
 ])
 def test_step_driver_equals_per_op_replay_at_shape(gpu, B, T, C, V, L):
     print(f"driver vs replay B={B} T={T} C={C} V={V} L={L}", flush=True)
@@ -424,12 +428,19 @@ def first_write_regions(lay):
 
 @pytest.mark.parametrize("B,T,C,V,L,garbage", [
     (8, 1024, 768, 50257, 12, True),  # the benchmark's step
-    (2, 64, 768, 50, 3, True),        # row teams, few rows
-    (2, 32, 384, 27, 6, True),        # the two-rows-per-wavefront kernels (C = 384)
-    (2, 16, 1024, 27, 2, True),       # four float4 per lane
-    (1, 16, 2048, 11, 1, True),       # eight float4 per lane
+    (2, 64, 768, 50, 3, True),        # few rows, at three,
+    (2, 32, 384, 27, 6, True),        # two,
+    (2, 16, 1024, 27, 2, True),       # four
+    (1, 16, 2048, 11, 1, True),       # and eight float4 per lane
+    (2, 520, 384, 27, 2, True),       # the two-rows-per-wavefront kernels
+    (2, 520, 768, 27, 2, True),       # row teams
+    (2, 520, 1024, 27, 2, True),      # four,
+    (2, 520, 1600, 27, 1, True),      # seven
+    (2, 520, 2048, 11, 1, True),      # and eight float4 per lane
     (2, 32, 384, 27, 0, False),       # no block: the final LayerNorm reads enc
-    (2, 16, 30, 11, 2, False),        # C = 30: the scalar LayerNorm path reads its residual targets
+    (2, 16, 30, 11, 2, False),        # a width that is no multiple of 4, few rows
+    (2, 520, 30, 11, 2, False),       # and many, whose kernel reads its residual targets
+    (2, 16, 2, 11, 2, False),         # the lane loops
 ])
 def test_zeroed_driver_equals_driver(gpu, B, T, C, V, L, garbage):
     """ugk_gpt2_layers_backward_zeroed on a grads_acts that is zero where the layer kernels write first

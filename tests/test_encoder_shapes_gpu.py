@@ -19,8 +19,8 @@ def counts_to_tokens(counts, seed):
     return t
 
 
-@pytest.mark.parametrize("B,T,C,V", [(16, 64, 96, 27), (17, 33, 100, 27), (32, 8, 33, 5), (65, 16, 64, 27), (128, 64, 384, 27),
-                                     (33, 7, 13, 3)])
+@pytest.mark.parametrize("B,T,C,V", [(16, 65, 96, 27), (17, 64, 100, 27), (32, 33, 33, 5), (65, 16, 64, 27), (128, 64, 384, 27),
+                                     (33, 40, 13, 3)])
 def test_batches(gpu, oracle, B, T, C, V):
     enc_case(gpu, oracle, B, T, C, V, gen.tokens_zipf(gen.rng(B), B * T, V), B + T, reps=2)
 
@@ -40,8 +40,8 @@ def test_few_rows(gpu, oracle, B, T, C, V):
 
 
 @pytest.mark.parametrize("rows,C", [(1024, 768), (1024, 772), (1000, 1100), (1024, 1600), (1024, 1601), (601, 2650),
-                                    (512, 3201), (30, 16448)])
-@pytest.mark.parametrize("V", [27, 50257])
+                                    (512, 3201)])
+@pytest.mark.parametrize("V", [27, 5000])
 def test_few_rows_of_many_channels(gpu, oracle, rows, C, V):
     """One, two and three slices of 64 channels per wavefront, the last group of them not full, and
     one row slice more than the one launch takes."""

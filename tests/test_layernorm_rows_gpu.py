@@ -2,7 +2,8 @@
 of each: one wavefront per row (4 to 2,048 channels), a workgroup per row (to 8,192), the lane loops
 (beyond, and below 4); widths that are no multiple of 4, whose last slot of four columns overlaps the
 one before it; rows at any alignment; the few-row backward, which adds its column sums without partial
-rows, on both sides of its rule (512 rows of 2^20 elements, 1,024 rows of 384 channels).
+rows, on both sides of its rule (512 rows of 2^19 elements, or of 2^20 beyond 1,536 channels; 1,024 rows
+of 2^18 elements, or of 3 2^16 off a 16-byte boundary); every number of float4 per lane above it.
 
 Against the CPU oracle with the bars of test_parity_gpu.py's ln_case; the fused pairs against the ops
 in sequence, bit for bit; and nothing written outside the arrays."""
@@ -21,6 +22,9 @@ SHAPES = [  # rows, C, offset
     (520, 2048, 2), (5, 2049, 0), (64, 2052, 1), (40, 3001, 0), (515, 4096, 0), (30, 4097, 3), (129, 6144, 0),
     (60, 8191, 0), (128, 8192, 1), (4, 8193, 0),
     (512, 768, 1), (513, 768, 2), (1024, 384, 0), (1025, 384, 0), (1024, 385, 0), (512, 2048, 0), (257, 4096, 0),
+    (512, 1024, 0), (512, 1028, 0), (512, 1540, 0), (1024, 256, 0), (1025, 256, 0), (1024, 260, 0), (768, 256, 1),
+    (769, 256, 1), (600, 1280, 0), (600, 1600, 0), (600, 1792, 0), (200, 6144, 0), (300, 4099, 0), (140, 8191, 0),
+    (2100, 771, 0),
 ]
 
 

@@ -14,7 +14,10 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 SHAPES = [(1, 3, 768), (2, 5, 16), (4, 64, 384), (1, 2, 2048), (1, 9, 516), (2, 50, 600), (3, 7, 4),
-          (4, 256, 1024), (8, 1024, 768), (16, 1024, 768), (2, 1000, 2048), (1, 70000, 64)]
+          (4, 256, 1024), (8, 1024, 768), (16, 1024, 768), (2, 1000, 2048), (1, 70000, 64),
+          # the seven of few rows above take one launch without partial rows in either mode; these do not,
+          # with 65 partial rows (13 of the 16 groups) and more
+          (1, 1025, 4), (2, 520, 16), (3, 400, 384), (2, 515, 516), (1, 1100, 600), (1, 1025, 768), (1, 530, 2048)]
 
 
 def inputs(B, T, C, seed):

@@ -40,19 +40,22 @@ def enc_case(g, B, T, C, V, hot):
     return (inp, gen.normal(g, (B * T * C,)), gen.normal(g, (V * C,), 0, 0.02), gen.normal(g, (T * C,), 0, 0.01))
 
 
+# few rows (no bucket state); the bucket table, with a large bucket in 64-channel slices and in 32-channel
+# ones (more than 1,024 rows)
+@pytest.mark.parametrize("B,T,hot", [(4, 64, 100), (8, 256, 100), (8, 256, 1300)])
 @pytest.mark.parametrize("exact", [True, False])
-def test_encoder_backward_graph_replays(gpu, oracle, lib_stream, exact):
+def test_encoder_backward_graph_replays(gpu, oracle, lib_stream, exact, B, T, hot):
     with encoder_mode(gpu, exact):
-        graph_replays(gpu, oracle, lib_stream, exact)
+        graph_replays(gpu, oracle, lib_stream, exact, B, T, hot)
 
 
-def graph_replays(gpu, oracle, lib_stream, exact):
+def graph_replays(gpu, oracle, lib_stream, exact, B, T, hot):
     """Exact mode: the CPU's order (oracle); blocked mode: its numpy restatement (test_parity_gpu),
-    whose per-(bucket, slice) counters must also return to zero within each replay."""
+    whose work counters must also return to zero within each replay."""
     backward = oracle.encoder_backward if exact else blocked_encoder_backward
-    B, T, C, V = 4, 64, 384, 1000
+    C, V = 384, 1000
     g = gen.rng(2718)
-    inp, dout, dwte0, dwpe0 = enc_case(g, B, T, C, V, hot=100)
+    inp, dout, dwte0, dwpe0 = enc_case(g, B, T, C, V, hot=hot)
     inp2, dout2, dwte2, dwpe2 = enc_case(g, B, T, C, V, hot=40)
     s = lib_stream
     t_inp, t_dout, t_dwte, t_dwpe = dev(inp), dev(dout), dev(dwte0), dev(dwpe0)
@@ -109,8 +112,9 @@ def run_ops(gpu, cfg, seed):
     return [dinp, dw, db, dwte, dwpe, acts, grads, ga], kl
 
 
-def test_caller_owned_workspace(gpu):
-    cfg = gpu.Config(B=2, T=64, C=384, V=500, NH=6, maxT=64, L=2)
+@pytest.mark.parametrize("B,T,L", [(2, 64, 2), (5, 256, 1)])  # few rows; the bucket table and LayerNorm partial rows
+def test_caller_owned_workspace(gpu, B, T, L):
+    cfg = gpu.Config(B=B, T=T, C=384, V=500, NH=6, maxT=T, L=L)
     gpu.set_workspace(None, cfg)
     want, kl_want = run_ops(gpu, cfg, seed=31)
     nbytes = gpu.workspace_bytes(cfg)
@@ -155,10 +159,10 @@ def test_reserve_config_then_no_growth(gpu):
     assert gpu.scratch_bytes() == held
 
 
-@pytest.mark.parametrize("C,NH,L", [(384, 6, 2), (384, 6, 16), (13, 1, 2)])
+@pytest.mark.parametrize("C,NH,L", [(384, 6, 2), (384, 6, 16), (13, 1, 2), (3, 1, 2)])
 def test_op_timer_records_the_driver_sequence(gpu, C, NH, L):
     """One record per op, in issue order, also for ops of several kernels: at L = 16 the batched
-    column sums take two launches, at C = 13 (scalar path) the fused LayerNorm backward pair does."""
+    column sums take two launches, at C = 3 (the lane loops) the fused LayerNorm backward pair does."""
     B, T, V = 2, 64, 100
     cfg = gpu.Config(B=B, T=T, C=C, V=V, NH=NH, maxT=T, L=L)
     g = torch.Generator(device=DEV)
@@ -210,12 +214,13 @@ def test_workspace_sized_for_more_rows_serves_fewer(gpu):
         gpu.set_workspace(None, cfg)
 
 
-def test_encoder_backward_capture_needs_prepared_state(gpu, oracle, lib_stream):
+@pytest.mark.parametrize("B,T", [(4, 64), (8, 256)])  # the first would not use the state; refused alike
+def test_encoder_backward_capture_needs_prepared_state(gpu, oracle, lib_stream, B, T):
     """The encoder backward's state must be allocated and cleared outside a graph capture: with the
     library's regions just freed, a first call under capture is refused before it launches anything;
     after ugk_set_workspace (which clears the state at once) a first call may be captured, and its
     replays accumulate what the oracle's calls do."""
-    B, T, C, V = 4, 64, 384, 1000
+    C, V = 384, 1000
     cfg = gpu.Config(B=B, T=T, C=C, V=V, NH=6, maxT=T, L=1)
     g = gen.rng(1618)
     inp, dout, dwte0, dwpe0 = enc_case(g, B, T, C, V, hot=70)

@@ -36,8 +36,8 @@
 //                  flight. The same launch has one more workgroup per
 //                  possible large bucket (K1 lists them with their slots):
 //                  its 256 threads scan the rows' slots in row order, 8,192
-//                  per round, and write the matching row ids, ascending, to a
-//                  list for K3.
+//                  per round (6,144 beside dword adds), and write the matching
+//                  row ids, ascending, to a list for K3.
 //     K3 large   - in the exact mode (the default's is k_enc_bwd_blocked)
 //                  workgroups of 16 wavefronts, one per (large bucket, 64
 //                  channels): one wavefront only adds staged rows in order,
@@ -176,10 +176,15 @@ __device__ __forceinline__ void add_dwpe(float *dwpe, const float *dout, int blk
   // and finds part of them in the cache (K2 15.8 -> 14.3 us at 8,192 x 768).
   // Each dwpe thread takes two (t, c) entries, one after the other, so half
   // as many dwpe workgroups stream at once and the inserts' round trips are
-  // delayed less (25.6 -> 24.8 us per call at 8,192 x 768). Large batches of
-  // short sequences have few entries of many rows: they take one channel per
-  // thread and 32 rows in flight (128 x 64 tokens of 384 channels: 8.7 against
-  // 22.4 us for the launch).
+  // delayed less (25.6 -> 24.8 us per call at 8,192 x 768).
+  // An entry's rows, one per sequence, are a chain of round trips, so from 17
+  // sequences on a thread takes one channel with 32 rows in flight, however many
+  // entries there are. Whole call by this form against the other, captured, Zipf
+  // tokens: 17 x 64 tokens of 384 channels 21.0 against 21.3 us, 17 x 256 x 384
+  // 22.5 against 25.0, 17 x 1,024 x 768 44.1 against 44.5, 32 x 64 x 384 22.9
+  // against 26.5, 32 x 1,024 x 768 71.5 against 71.7, 128 x 64 x 384 24.1 against
+  // 38.1; below the line 12 x 1,024 x 768 35.3 against 35.0, 8 x 1,024 x 768 30.9
+  // against 29.7, 4 x 1,024 x 1,600 27.9 against 25.1.
   const size_t pstride = (size_t)nblk * kBlock;
   const size_t n_pe = (size_t)T * (kVec ? C >> 2 : C);
   for (size_t j = (size_t)blk * kBlock + threadIdx.x; j < n_pe; j += pstride) {
@@ -516,9 +521,16 @@ __device__ __forceinline__ void add_small(EncTable tb, EncShared sh, float *__re
 // the adds end), then one wavefront per slot-list entry (covering K1's
 // regions exactly). A small bucket's wavefront frees its slot once it has
 // read it.
+// Registers: the float4 adds' twelve row slots in flight leave six wavefronts
+// per SIMD (three rows of three at seven: uniform tokens 22.1 against 22.4 us at
+// 8,192 x 768, but Zipf's 30.2 against 29.6; two at eight 22.2 and 31.8), so the
+// scan takes eight loads beside them; the dword adds need few, and six loads
+// leave eight wavefronts (8,184 x 771 uniform 26.8 against 31.6 us).
 template <bool kVec>
-__global__ __launch_bounds__(kBlock, kVec ? 6 : 8) void k_enc_bwd_add(EncTable tb, EncShared sh, float *__restrict__ dwte,
-                                                        const float *__restrict__ dout, int C, int n, int nscan) {
+__global__ __launch_bounds__(kBlock, kVec ? 6 : 8) void k_enc_bwd_add(EncTable tb, EncShared sh,
+                                                                      float *__restrict__ dwte,
+                                                                      const float *__restrict__ dout, int C, int n,
+                                                                      int nscan) {
   __shared__ unsigned lds[kWavesPerBlock * kCap];
   if ((int)blockIdx.x < nscan) {
     const int j = (int)blockIdx.x;
@@ -528,7 +540,7 @@ __global__ __launch_bounds__(kBlock, kVec ? 6 : 8) void k_enc_bwd_add(EncTable t
   const int wave = threadIdx.x >> 6;
   const int R = ((int)gridDim.x - nscan) * kWavesPerBlock / kBlock;
   add_small<kVec>(tb, sh, dwte, dout, C, ((int)blockIdx.x - nscan) * kWavesPerBlock + wave, R,
-                         lds + (size_t)wave * kCap);
+                  lds + (size_t)wave * kCap);
 }
 
 // K3: workgroups take (large bucket, 64-channel slice) work items from a
@@ -1110,7 +1122,7 @@ int launch_encoder_backward(float *dwte, float *dwpe, const float *dout, int *in
     const int shift = 32 - lg;
     const int ins_blocks = (int)grid_for((size_t)n, kBlock);
     // dwpe, in the first chunk's launch: two float4 entries per thread, or one
-    // entry of one channel where each has many rows
+    // entry of one channel where each has many rows (add_dwpe has the timings)
     const bool deep = B > 16;
     int pe_blocks = 0;
     if (c0 == 0)
